@@ -4,8 +4,10 @@
 // (cpp/nbody_operator.h:143-152, cpp/dense_operator.cpp:38-46) and nbody_eval
 // (cpp/nbody_operator.h:117-141): y_i = sum_j w_j K(x_i <- y_j) x_j without the
 // O(N^2) matrix. Points keep their input order and are cut into flat "cells":
-// 128-point target chunks, each streaming every source chunk through the same
-// leaf-stage kernel the FMM's P2P uses (LDS tiles, slice-split lanes).
+// 128-point target chunks, each streaming the sources through the same leaf-stage
+// kernel the FMM's P2P uses (LDS tiles, slice-split lanes). Where the target chunks
+// alone are too few for the chip, the sources are cut into parts, one workgroup per
+// (chunk, part), whose sums k_leaf_parts adds in part order (split_sources).
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -28,18 +30,30 @@ constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static double* g_scratch[kMaxDevices] = {};
 
-// The device address of `scratch` on the current device, looked up on the first
-// call per device (with that device current) and kept.
-static double* noalloc_scratch(int dev) {
+// Scratch of the parts' sums of one call (kPartRows doubles per target point and part),
+// for tbem_nbody_apply_noalloc; split_sources never asks for more.
+constexpr size_t kPartDoubles = size_t(2) << 20;
+static __device__ __align__(256) double part_scratch[kPartDoubles];
+static double* g_part_scratch[kMaxDevices] = {};
+
+struct NoallocScratch {
+    double *dens, *parts;
+};
+
+// The device addresses of the scratch arrays on the current device, looked up on the
+// first call per device (with that device current) and kept.
+static NoallocScratch noalloc_scratch(int dev) {
     TBEM_REQUIRE(dev >= 0 && dev < kMaxDevices, TBEM_E_UNSUPPORTED, "device index beyond the scratch table");
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch[dev]) {
-        void* ptr = nullptr;
-        TBEM_HIP(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
-        TBEM_REQUIRE(ptr != nullptr, TBEM_E_HIP, "no device address for the no-allocation scratch");
-        g_scratch[dev] = static_cast<double*>(ptr);
+    if (!g_scratch[dev] || !g_part_scratch[dev]) {
+        void *d = nullptr, *p = nullptr;
+        TBEM_HIP(hipGetSymbolAddress(&d, HIP_SYMBOL(scratch)));
+        TBEM_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(part_scratch)));
+        TBEM_REQUIRE(d != nullptr && p != nullptr, TBEM_E_HIP, "no device address for the no-allocation scratch");
+        g_scratch[dev] = static_cast<double*>(d);
+        g_part_scratch[dev] = static_cast<double*>(p);
     }
-    return g_scratch[dev];
+    return {g_scratch[dev], g_part_scratch[dev]};
 }
 
 // a flat tree of fixed-size chunks over n points in input order
@@ -95,6 +109,56 @@ static HostList all_pairs(const HostTree& tgt, int n_src) {
     return l;
 }
 
+// The work items of one direction: every target chunk against n_src sources, the sources
+// cut into equal parts so that the launch holds about kTargetItems workgroups: the kernel
+// keeps two to three per compute unit, and several rounds of them keep the last round's
+// idle units a small share. Bound: FP64 VALU issue once the chip is filled. Measured,
+// whole chunks -> parts: hypersingular, 20,011 points (157 workgroups of four waves on
+// 256 units): 1712 -> 950 us (15.9 -> 28.6 TFLOP/s); traction, 3,000 sources and 2,003
+// targets (16 workgroups): 169 -> 30 us. A part keeps at least
+// kMinPartSources sources: below that a workgroup's fixed costs (targets, first tile,
+// slice sums) outweigh its pairs. In mixed precision parts are whole FP32 tiles
+// (kLeafBlock sources, a multiple of every instance's), so that the tiles' partial sums
+// stay what they are without parts.
+constexpr int kTargetItems = 4096, kMinPartSources = 64;
+
+struct Split {
+    std::vector<WaveItem> h_items;  // kept: their upload may still be in flight
+    std::vector<WaveLeafParts> h_parts;
+    DevBuf<WaveItem> items;
+    DevBuf<WaveLeafParts> parts;
+    int n_items = 0, n_parts = 0;
+    size_t part_size = 0;
+};
+
+static void split_sources(const HostTree& tgt, int n_src, int precision, Split& out, hipStream_t s) {
+    std::vector<WaveItem>& items = out.h_items;
+    std::vector<WaveLeafParts>& parts = out.h_parts;
+    const int nc = (int)tgt.leaves.size(), unit = precision == TBEM_MIXED ? kLeafBlock : 1;
+    size_t np = std::min<size_t>(div_up(kTargetItems, nc), div_up(std::max(n_src, 1), kMinPartSources));
+    np = std::min(np, kPartDoubles / ((size_t)kPartRows * std::max(tgt.n_pts, 1)));
+    int per = np > 1 ? div_up((size_t)n_src, np) : std::max(n_src, 1);
+    per = div_up(per, unit) * unit;
+    const int n = div_up(std::max(n_src, 1), per);
+    size_t part = 0;
+    for (int k = 0; k < nc; k++) {
+        const size_t m = tgt.count[k];
+        if (m == 0) continue;
+        if (n == 1) {
+            items.push_back(WaveItem{k, 0, n_src > 0 ? 1 : 0, 0, n_src, 0, 0, 0, -1});
+            continue;
+        }
+        parts.push_back(WaveLeafParts{k, (int)part, n});
+        for (int p = 0; p < n; p++, part += kPartRows * m)
+            items.push_back(WaveItem{k, 0, 1, p * per, std::min(n_src, (p + 1) * per), 0, 0, 0, (int)part});
+    }
+    out.n_items = (int)items.size();
+    out.n_parts = (int)parts.size();
+    out.part_size = part;
+    out.items.upload(items, s);
+    out.parts.upload(parts, s);
+}
+
 struct NbodyPlan {
     int kid = 0, R = 1, precision = TBEM_FP64;
     KConst kc{};
@@ -103,8 +167,9 @@ struct NbodyPlan {
     DevTree d_obs_t, d_src_t;
     DevPoints op, sp;
     DevList fwd, adj;
+    Split fwd_split, adj_split;
     DevBuf<int> obs_leaves, src_leaves;
-    DevBuf<double> dens, gsort, xb, yb, outs;
+    DevBuf<double> dens, parts, gsort, xb, yb, outs;  // parts: both directions' part sums
     int device = 0;  // the device the handle's buffers live on
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;  // end of the last call's work (buffers are per handle)
@@ -137,12 +202,12 @@ static int nb_guard(F&& f) {
     }
 }
 
-static void nb_forward_impl(const NbodyPlan& P, const double* x, double* y, double* dens, hipStream_t s);
+static void nb_forward_impl(const NbodyPlan& P, const double* x, double* y, double* dens, double* parts, hipStream_t s);
 static void nb_adjoint_impl(NbodyPlan& P, const double* g, double* y, hipStream_t s);
 
 static void nb_forward(NbodyPlan& P, const double* x, double* y, hipStream_t s) {
     TBEM_HIP(hipStreamWaitEvent(s, P.done, 0));
-    nb_forward_impl(P, x, y, P.dens.p, s);
+    nb_forward_impl(P, x, y, P.dens.p, P.parts.p, s);
     TBEM_HIP(hipEventRecord(P.done, s));
 }
 
@@ -152,8 +217,15 @@ static void nb_adjoint(NbodyPlan& P, const double* g, double* y, hipStream_t s) 
     TBEM_HIP(hipEventRecord(P.done, s));
 }
 
-// dens: R * n_src doubles of scratch for the weighted densities
-static void nb_forward_impl(const NbodyPlan& P, const double* x, double* y, double* dens, hipStream_t s) {
+static void set_items(LeafStage& f, const Split& sp, double* parts) {
+    f.block_items = sp.items.p; f.n_block_items = sp.n_items;
+    f.block_parts = sp.parts.p; f.n_block_parts = sp.n_parts;
+    f.part_buf = parts;
+}
+
+// dens: R * n_src doubles of scratch for the weighted densities; parts: the part sums
+static void nb_forward_impl(const NbodyPlan& P, const double* x, double* y, double* dens, double* parts,
+                            hipStream_t s) {
     if (P.n_obs == 0) return;
     if (P.n_src == 0) {
         launch_fill(y, (size_t)P.R * P.n_obs, 0.0, s);
@@ -167,6 +239,7 @@ static void nb_forward_impl(const NbodyPlan& P, const double* x, double* y, doub
     f.rp_ptr = P.fwd.ptr.p; f.rp_beg = P.fwd.rbeg.p; f.rp_cnt = P.fwd.rcnt.p; f.rp_pre = P.fwd.rpre.p;
     f.ps = view(P.sp); f.pdens = dens; f.n_ps = P.n_src;
     f.out_sorted = y;  // identity permutation: write straight into y
+    set_items(f, P.fwd_split, parts);
     if (P.precision == TBEM_MIXED) launch_leaf_stage<float>(P.kid, false, f, P.kc, s, false);
     else launch_leaf_stage<double>(P.kid, false, f, P.kc, s, false);
 }
@@ -184,6 +257,7 @@ static void nb_adjoint_impl(NbodyPlan& P, const double* g, double* y, hipStream_
     f.rp_ptr = P.adj.ptr.p; f.rp_beg = P.adj.rbeg.p; f.rp_cnt = P.adj.rcnt.p; f.rp_pre = P.adj.rpre.p;
     f.ps = view(P.op); f.pdens = g; f.n_ps = P.n_obs;
     f.out_sorted = y;
+    set_items(f, P.adj_split, P.parts.p);
     if (P.precision == TBEM_MIXED) launch_leaf_stage<float>(P.kid, true, f, P.kc, s, false);
     else launch_leaf_stage<double>(P.kid, true, f, P.kc, s, false);
 }
@@ -227,7 +301,10 @@ int tbem_nbody_create(const tbem_nbody_desc* d, tbem_nbody_t* out) {
         P.adj.upload(all_pairs(P.src_t, P.n_obs), s);
         P.obs_leaves.upload(P.obs_t.leaves, s);
         P.src_leaves.upload(P.src_t.leaves, s);
+        split_sources(P.obs_t, P.n_src, P.precision, P.fwd_split, s);
+        split_sources(P.src_t, P.n_obs, P.precision, P.adj_split, s);
         P.dens.alloc((size_t)P.R * P.n_src);
+        P.parts.alloc(std::max(P.fwd_split.part_size, P.adj_split.part_size));
         TBEM_HIP(hipEventRecord(P.done, s));
         TBEM_HIP(hipStreamSynchronize(s));
         *out = h.release();
@@ -257,7 +334,8 @@ int tbem_nbody_apply_noalloc(tbem_nbody_t h, const double* d_x, double* d_y, voi
         TBEM_HIP(hipGetDevice(&dev));
         TBEM_REQUIRE(dev == P.device, TBEM_E_INVALID,
                      "tbem_nbody_apply_noalloc: the current device is not the handle's");
-        nb_forward_impl(P, d_x, d_y, noalloc_scratch(dev), (hipStream_t)stream);
+        const NoallocScratch sc = noalloc_scratch(dev);
+        nb_forward_impl(P, d_x, d_y, sc.dens, sc.parts, (hipStream_t)stream);
     });
 }
 

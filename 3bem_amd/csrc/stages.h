@@ -42,13 +42,15 @@ constexpr int kWaveBlock = 256;        // k_leaf_wave: four work items per workg
 constexpr int kWaveLeafMax = 128;      // leaves of up to this many points go to k_leaf_wave ...
 constexpr long kWavePairsMax = 65536;  // ... one wave per leaf, or per chunk of at most this
                                        // many pairs (points x sources) of a larger one
+constexpr int kPartsBlock = 128;       // k_leaf_parts
 constexpr int kSymBlock = 256;         // k_leaf_sym: four waves per leaf
 constexpr int kSymLeafMin = 16;        // k_leaf_sym takes leaves of kSymLeafMin .. kSymLeafMax
 constexpr int kSymLeafMax = 256;       // points (the plan chooses which, per kernel)
 constexpr int kSymSlots = kSymLeafMax + 64;  // k_leaf_sym's target slots per wave and component
 constexpr int kSymSrc = 3;             // k_leaf_sym: sources per lane
 
-// One work item of k_leaf_wave: the leaf at list position pos, whole or one chunk of
+// One work item of k_leaf_wave (and of k_leaf_stage, LeafStage.block_items): the leaf at
+// list position pos, whole or one chunk of
 // its sources. Point sources [v0, v1) of the leaf's packed ranges (offsets into their
 // concatenation; ranges f0 .. f1-1 hold them), surface cells [c0, c1) of its surface
 // list, and its own surface when self != 0. part < 0: the item is the whole leaf and
@@ -163,6 +165,11 @@ struct LeafStage {
     const WaveLeafParts* wave_parts;
     int n_parts;
     double* part_buf;
+    // The one-workgroup kernel's work items (null: whole leaves, above): a leaf, or a part
+    // of its sources, whose partial sums go to part_buf; block_parts: the leaves cut.
+    const WaveItem* block_items;
+    const WaveLeafParts* block_parts;
+    int n_block_items, n_block_parts;
     const double* grad_g;   // obs-gradient mode: upstream g (sorted, component-major)
     double* grad_out;       // obs-gradient mode: 3 per target (sorted, AoS)
     // Symmetric pairs (Kelvin U with one point set on both sides; null: none). Per leaf

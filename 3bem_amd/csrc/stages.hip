@@ -224,9 +224,10 @@ __device__ inline void stream_ranges(Tile<VT, R, NRM, NB>& tl, int e0, int e1,
     }
 }
 
-// Streams the points of ranges e0..e1 through the tile in full NB-point tiles cut
-// from the list's virtual concatenation (range e starts at offset rpre[e] of it),
-// so a tile may span range boundaries and only the last one is partial. Up to NB
+// Streams the points [v0, v1) of the list's virtual concatenation of ranges (range e
+// starts at offset rpre[e] of it; ranges e0..e1 hold them, v0 lying in e0) through the
+// tile in full NB-point tiles, so a tile may span range boundaries and only the last
+// one is partial. Up to NB
 // ranges are cached in LDS; each lane finds its range by a short forward scan
 // from the range holding the tile's first point. Ranges must be nonempty: then a
 // cache that starts at the range holding point `base` covers at least
@@ -243,14 +244,14 @@ constexpr int kCloseBit = 1 << 30;
 
 template <class VT, int R, bool NRM, int NB, class F>
 __device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB>& tl, int* s_pre, int* s_beg, int e0, int e1,
-                                            const int* __restrict__ rbeg, const int* __restrict__ rcnt,
+                                            int v0, int v1, const int* __restrict__ rbeg,
                                             const int* __restrict__ rpre, const PtsView& sp,
                                             const double* __restrict__ dens, int n_src, F&& compute,
                                             const int* __restrict__ rclose = nullptr, int* tile_close = nullptr,
                                             int* s_wflag = nullptr) {
     const int tid = threadIdx.x;
-    if (e0 >= e1) return;
-    const int total = uni(rpre[e1 - 1] + rcnt[e1 - 1]);
+    if (v0 >= v1) return;
+    const int total = v1;
     SrcReg<R, NRM> r;
     int mclose = 0;  // the lane's next point comes from a close range
     int lbase = e0;  // list index of cache entry 0
@@ -279,8 +280,8 @@ __device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB>& tl, int* s_pre
             load_point(r, (bf & ~kCloseBit) + (v - s_pre[f]), sp, dens, n_src);
         }
     };
-    int base = 0;
-    fetch(0);
+    int base = v0;
+    fetch(base);
     while (true) {
         const int cnt = min(NB, total - base);
         __syncthreads();
@@ -457,12 +458,26 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
     __shared__ StageSmem<T, R, NRM, NB, 2 * R> sm;
-    const int pos = a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
+    const WaveItem* it = a.block_items ? a.block_items + blockIdx.x : nullptr;
+    const int pos = it ? uni(it->pos) : a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
     if (pos < 0) return;  // padding of the layout (the whole workgroup)
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
-    const int pe0 = a.rp_ptr ? uni(a.rp_ptr[pos]) : 0, pe1 = a.rp_ptr ? uni(a.rp_ptr[pos + 1]) : 0;
-    const int se0 = a.sl_ptr ? uni(a.sl_ptr[pos]) : 0, se1 = a.sl_ptr ? uni(a.sl_ptr[pos + 1]) : 0;
+    // the whole leaf, or the item's part of its sources
+    int pe0 = 0, pe1 = 0, v0 = 0, v1 = 0;
+    if (a.rp_ptr) {
+        pe0 = uni(it ? it->f0 : a.rp_ptr[pos]);
+        pe1 = uni(it ? it->f1 : a.rp_ptr[pos + 1]);
+        v0 = it ? uni(it->v0) : 0;
+        v1 = it ? uni(it->v1) : pe0 < pe1 ? uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]) : 0;
+    }
+    int se0 = 0, se1 = 0;
+    if (a.sl_ptr) {
+        se0 = uni(it ? it->c0 : a.sl_ptr[pos]);
+        se1 = uni(it ? it->c1 : a.sl_ptr[pos + 1]);
+    }
+    const bool self = a.self_coeff && (!it || uni(it->self));
+    const int part = it ? uni(it->part) : -1;
     const int tid = threadIdx.x;
 
     for (int t0 = 0; t0 < m; t0 += 2 * NB) {
@@ -519,12 +534,12 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
                 }
             }
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, a.rp_beg, a.rp_cnt, a.rp_pre, a.ps, a.pdens,
+        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, v0, v1, a.rp_beg, a.rp_pre, a.ps, a.pdens,
                              a.n_ps, points, CLOSE ? a.rp_close : nullptr, CLOSE ? &tclose : nullptr,
                              sm.wflag);                                                              // (a)
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk,
                         surfaces);                                                                // (b)
-        if (a.self_coeff)
+        if (self)
             stream_surfaces(sm.st, 0, 1, &leaf, a.tt, a.self_surf, a.unit, a.self_coeff, a.n_e, a.blk,
                             surfaces);                                                            // (c)
         __syncthreads();
@@ -537,7 +552,11 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
         slice_sum<NB>(sm.red, sm.part, 2 * R, ntp, S, [&](int v, int g, double s) {
             const int h = v / R, q = v - h * R;
             if (h == 1 && nslot + g >= nt) return;
-            const int i = b + t0 + h * nslot + g;
+            const int t = t0 + h * nslot + g, i = b + t;
+            if (part >= 0) {
+                a.part_buf[(size_t)part + (size_t)q * m + t] = s;
+                return;
+            }
             const double w = a.t_weight ? a.t_weight[i] : 1.0;
             double* o = a.out_sorted + (size_t)q * a.n_tgt + i;
             *o = a.accumulate ? *o + w * (s * scale) : w * (s * scale);
@@ -728,20 +747,26 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     }
 }
 
-// The leaves k_leaf_wave ran in chunks: one workgroup per leaf, one target per thread
-// (m <= kWaveLeafMax), the chunks' partial sums added in chunk order.
-__global__ __launch_bounds__(kWaveLeafMax) void k_leaf_parts(LeafStage a, int R, double scale) {
-    const WaveLeafParts lp = a.wave_parts[blockIdx.x];
-    const int leaf = a.leaves[lp.pos];
+// The leaves that ran in chunks: one workgroup per leaf and output component (grid y),
+// the chunks' partial sums added in chunk order, eight loads in flight.
+__global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, const WaveLeafParts* __restrict__ parts,
+                                                           double scale) {
+    const WaveLeafParts lp = parts[blockIdx.x];
+    const int leaf = a.leaves[lp.pos], q = blockIdx.y;
     const int b = a.tt.begin[leaf], m = a.tt.count[leaf];
-    const int t = threadIdx.x;
-    if (t >= m) return;
-    const int i = b + t;
-    const double wgt = a.t_weight ? a.t_weight[i] : 1.0;
-    for (int q = 0; q < R; q++) {
-        const double* p = a.part_buf + (size_t)lp.part + q * m + t;
+    const size_t step = (size_t)kPartRows * m;
+    for (int t = threadIdx.x; t < m; t += kPartsBlock) {
+        const int i = b + t;
+        const double* p = a.part_buf + (size_t)lp.part + (size_t)q * m + t;
         double s = 0;
-        for (int c = 0; c < lp.n; c++) s += p[(size_t)c * kPartRows * m];
+        int c = 0;
+        for (; c + 8 <= lp.n; c += 8) {
+            double v[8];
+            for (int u = 0; u < 8; u++) v[u] = p[(c + u) * step];
+            for (int u = 0; u < 8; u++) s += v[u];
+        }
+        for (; c < lp.n; c++) s += p[c * step];
+        const double wgt = a.t_weight ? a.t_weight[i] : 1.0;
         double* o = a.out_sorted + (size_t)q * a.n_tgt + i;
         *o = a.accumulate ? *o + wgt * (s * scale) : wgt * (s * scale);
     }
@@ -1003,6 +1028,7 @@ __global__ __launch_bounds__(kGradBlock) void k_leaf_grad(LeafStage a, KC<D3> kc
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
     const int pe0 = a.rp_ptr ? uni(a.rp_ptr[pos]) : 0, pe1 = a.rp_ptr ? uni(a.rp_ptr[pos + 1]) : 0;
     const int se0 = a.sl_ptr ? uni(a.sl_ptr[pos]) : 0, se1 = a.sl_ptr ? uni(a.sl_ptr[pos + 1]) : 0;
+    const int np = pe0 < pe1 ? uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]) : 0;
     const int tid = threadIdx.x;
     for (int t0 = 0; t0 < m; t0 += NB) {
         const int nt = min(NB, m - t0);
@@ -1033,7 +1059,7 @@ __global__ __launch_bounds__(kGradBlock) void k_leaf_grad(LeafStage a, KC<D3> kc
             if (!active) return;
             for (int j = slice; j < cnt; j += S) pair_d(sm.st, j);
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, a.rp_beg, a.rp_cnt, a.rp_pre, a.ps, a.pdens,
+        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, np, a.rp_beg, a.rp_pre, a.ps, a.pdens,
                              a.n_ps, points);
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk, surfaces);
         if (a.self_coeff)
@@ -1093,6 +1119,7 @@ __global__ __launch_bounds__(kGradBlock, (grad_waves<KID, T>())) void k_leaf_gra
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
     const int pe0 = a.rp_ptr ? uni(a.rp_ptr[pos]) : 0, pe1 = a.rp_ptr ? uni(a.rp_ptr[pos + 1]) : 0;
+    const int np = pe0 < pe1 ? uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]) : 0;
     const int se0 = a.sl_ptr ? uni(a.sl_ptr[pos]) : 0, se1 = a.sl_ptr ? uni(a.sl_ptr[pos + 1]) : 0;
     const int tid = threadIdx.x;
     for (int t0 = 0; t0 < m; t0 += 2 * NB) {
@@ -1159,7 +1186,7 @@ __global__ __launch_bounds__(kGradBlock, (grad_waves<KID, T>())) void k_leaf_gra
                 grad_pair<KID, double>(dxb, dyb, dzb, dxb * dxb + dyb * dyb + dzb * dzb, sn, v, gB, GB, kc64);
             }
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, a.rp_beg, a.rp_cnt, a.rp_pre, a.ps, a.pdens,
+        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, np, a.rp_beg, a.rp_pre, a.ps, a.pdens,
                              a.n_ps, points, a.rp_close, a.rp_close ? &tclose : nullptr, sm.wflag);
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk, surfaces);
         if (a.self_coeff)
@@ -1625,8 +1652,8 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
             }
             TBEM_LAUNCH_CHECK();
             if (a.n_parts > 0) {
-                hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_parts), dim3(kWaveLeafMax), 0, s, a,
-                                   kernel_dim(KID), scale);
+                hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_parts, kernel_dim(KID)), dim3(kPartsBlock), 0, s, a,
+                                   a.wave_parts, scale);
                 TBEM_LAUNCH_CHECK();
             }
         }
@@ -1656,7 +1683,7 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
         }
         return;
     }
-    dim3 g(a.order ? a.n_order : a.n_leaves), b(leaf_block<KID, T>());
+    dim3 g(a.block_items ? a.n_block_items : a.order ? a.n_order : a.n_leaves), b(leaf_block<KID, T>());
     // the one-step rsqrt only differs from the full one in FP64
     if (fast && std::is_same<T, double>::value && a.rp_close && a.rp_ptr) {
         if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, true, true>), g, b, 0, s, a, kc, kc64, scale);
@@ -1672,6 +1699,11 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
         else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, false>), g, b, 0, s, a, kc, kc64, scale);
     }
     TBEM_LAUNCH_CHECK();
+    if (a.block_items && a.n_block_parts > 0) {
+        hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_block_parts, kernel_dim(KID)), dim3(kPartsBlock), 0, s, a,
+                           a.block_parts, scale);
+        TBEM_LAUNCH_CHECK();
+    }
 }
 
 template <int KID, class T>
