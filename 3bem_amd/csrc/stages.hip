@@ -1389,75 +1389,113 @@ __global__ __launch_bounds__(kWaveLeafMax) void k_leaf_grad_parts(LeafStage a, d
 }
 
 // ------------------------------------------------------------------------ helpers
-// out[c] (= or +=) op(M[level c]) in[c] (+ addin[c]) for the cells of each tile:
-// a 64 (rows) x 64 (cells) output tile per workgroup, 4 x 4 per thread (rows ty*4+i,
-// cells tx+16j), k in chunks of kGemmK staged in LDS; the next chunk is loaded into
-// registers while the current one is multiplied, so its latency overlaps the FMAs.
-constexpr int kGemmK = 32;
+// out[c] (= or +=) op(M[level c]) in[c] (+ addin[c]) for the cells of each tile, on the
+// FP64 MFMA units: the cells are the A operand's rows and op(M)'s rows the B operand's
+// columns, so that a lane's results lie along a cell's rows (128-byte stores). One
+// workgroup of WR x WC waves computes (16 WR RT) rows x (16 WC CT) cells, RT x CT MFMA
+// tiles per wave, k in chunks of KC staged in LDS; the next chunk is loaded into registers
+// while the current one is multiplied. v_mfma_f64_16x16x4f64 adds its four products to the
+// accumulator one by one, k ascending, each with one rounding, so a result is the same
+// chain of FMAs over k whatever the tile shape.
+// Bound: FP64 MFMA with many cells, the latency of the chunks' loads with few. Shapes
+// (launch_level_gemm): 64 x 64, four tiles per wave, where the launch then still has
+// kGemmWideMin workgroups; else 64 x 16, one tile per wave, four times the workgroups.
+// Measured against FP64 FMAs from 4 x 4 register tiles, per launch: blk 453 (traction,
+// order 150, at most 1,024 cells) 58 -> 22 us; blk 150 (mesh of 9,102 points) 22 -> 9.5;
+// 2M points, order 100 (blk 297): 16 launches 2311 -> 1500 us beside the point pairs.
+constexpr int kGemmWideMin = 512;
+typedef double gemm_f64x4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void k_level_gemm(int n, const int* __restrict__ cells,
-                                                    const int* __restrict__ tiles, const double* __restrict__ M,
-                                                    int trans, const double* __restrict__ in,
-                                                    const double* __restrict__ addin, double* __restrict__ out,
-                                                    float* __restrict__ out32, int add) {
-    constexpr int KC = kGemmK, PER = 64 * KC / 256;  // elements of each operand per thread and chunk
-    const int t = blockIdx.y;
-    const int first = uni(tiles[3 * t]), cnt = uni(tiles[3 * t + 1]), lvl = uni(tiles[3 * t + 2]);
+template <int WR, int WC, int RT, int CT, int KC>
+__global__ __launch_bounds__(WR* WC * 64) void k_level_gemm(int n, const int* __restrict__ cells,
+                                                          const int* __restrict__ tiles,
+                                                          const double* __restrict__ M, int trans,
+                                                          const double* __restrict__ in,
+                                                          const double* __restrict__ addin, double* __restrict__ out,
+                                                          float* __restrict__ out32, int add) {
+    constexpr int NT = WR * WC * 64, RB = 16 * WR * RT, CB = 16 * WC * CT;
+    constexpr int PR = RB * KC / NT, PC = CB * KC / NT;  // elements of each operand per thread and chunk
+    const int t = blockIdx.y, z = blockIdx.z * CB;
+    const int first = uni(tiles[3 * t]) + z, cnt = uni(tiles[3 * t + 1]) - z, lvl = uni(tiles[3 * t + 2]);
+    if (cnt <= 0) return;  // the tile has no such cells (uniform, before any barrier)
     const double* A = M + (size_t)lvl * n * n;
-    const int m0 = blockIdx.x * 64;
-    __shared__ double As[KC][65], Bs[KC][65];
-    __shared__ int cl[64];
-    const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-    if (tid < 64) cl[tid] = tid < cnt ? cells[first + tid] : -1;
+    const int m0 = blockIdx.x * RB;
+    __shared__ double Ms[KC][RB + 1], Cs[KC][CB + 1];
+    __shared__ int cl[CB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane % 16, lq = lane / 16;
+    if (tid < CB) cl[tid] = tid < cnt ? cells[first + tid] : -1;
     __syncthreads();
-    double pa[PER], pb[PER];
-    // A chunk: As[k][r] = op(A)[m0 + r][k0 + k]; B chunk: Bs[k][c] = in[cell c][k0 + k]
+    double pr[PR], pc[PC];
+    // Ms[k][r] = op(M)[m0 + r][k0 + k]; Cs[k][c] = in[cell c][k0 + k]
     auto fetch = [&](int k0) {
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + 256 * q;
-            const int r = trans ? e % 64 : e / KC, k = trans ? e / 64 : e % KC;
+#pragma unroll
+        for (int q = 0; q < PR; q++) {
+            const int e = tid + NT * q;
+            const int r = trans ? e % RB : e / KC, k = trans ? e / RB : e % KC;
             const int row = m0 + r, kk = k0 + k;
-            pa[q] = (row < n && kk < n) ? (trans ? A[(size_t)kk * n + row] : A[(size_t)row * n + kk]) : 0.0;
-            const int c = e / KC, kb = e % KC, cell = cl[c];
-            pb[q] = (cell >= 0 && k0 + kb < n) ? in[(size_t)cell * n + k0 + kb] : 0.0;
+            pr[q] = (row < n && kk < n) ? (trans ? A[(size_t)kk * n + row] : A[(size_t)row * n + kk]) : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < PC; q++) {
+            const int e = tid + NT * q, cell = cl[e / KC], kk = k0 + e % KC;
+            pc[q] = (cell >= 0 && kk < n) ? in[(size_t)cell * n + kk] : 0.0;
         }
     };
     auto store = [&]() {
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + 256 * q;
-            const int r = trans ? e % 64 : e / KC, k = trans ? e / 64 : e % KC;
-            As[k][r] = pa[q];
-            Bs[e % KC][e / KC] = pb[q];
+#pragma unroll
+        for (int q = 0; q < PR; q++) {
+            const int e = tid + NT * q;
+            Ms[trans ? e / RB : e % KC][trans ? e % RB : e / KC] = pr[q];
+        }
+#pragma unroll
+        for (int q = 0; q < PC; q++) {
+            const int e = tid + NT * q;
+            Cs[e % KC][e / KC] = pc[q];
         }
     };
-    double acc[4][4] = {};
+    const int r0 = (wave % WR) * RT * 16 + lr, c0 = (wave / WR) * CT * 16 + lr;
+    gemm_f64x4 acc[CT][RT] = {};
     fetch(0);
     for (int k0 = 0; k0 < n; k0 += KC) {
         store();
         __syncthreads();
         if (k0 + KC < n) fetch(k0 + KC);
-        for (int k = 0; k < KC; k++) {
-            double av[4], bv[4];
-            for (int i = 0; i < 4; i++) av[i] = As[k][ty * 4 + i];
-            for (int j = 0; j < 4; j++) bv[j] = Bs[k][tx + 16 * j];
-            for (int i = 0; i < 4; i++)
-                for (int j = 0; j < 4; j++) acc[i][j] += av[i] * bv[j];
+        const int steps = min(KC, n - k0 + 3) / 4;  // the last chunk's k past n are zeros
+#pragma unroll 4
+        for (int ks = 0; ks < steps; ks++) {
+            const double* pm = &Ms[4 * ks + lq][r0];
+            const double* px = &Cs[4 * ks + lq][c0];
+            double mv[RT], xv[CT];
+#pragma unroll
+            for (int i = 0; i < RT; i++) mv[i] = pm[16 * i];
+#pragma unroll
+            for (int j = 0; j < CT; j++) xv[j] = px[16 * j];
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int i = 0; i < RT; i++)
+                    acc[j][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(xv[j], mv[i], acc[j][i], 0, 0, 0);
         }
         __syncthreads();
     }
-    for (int j = 0; j < 4; j++) {
-        const int cell = cl[tx + 16 * j];
-        if (cell < 0) continue;
-        for (int i = 0; i < 4; i++) {
-            const int row = m0 + ty * 4 + i;
-            if (row >= n) continue;
-            const size_t o = (size_t)cell * n + row;
-            double v = acc[i][j];
-            if (addin) v += addin[o];
-            if (out32) out32[o] = (float)v;
-            else out[o] = add ? out[o] + v : v;
+    // D[4 r + lq][lr] in register r: cell 4 r + lq of the column tile, row lr of the row tile
+#pragma unroll
+    for (int j = 0; j < CT; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int cell = cl[c0 - lr + 16 * j + 4 * r + lq];
+            if (cell < 0) continue;
+#pragma unroll
+            for (int i = 0; i < RT; i++) {
+                const int row = m0 + r0 + 16 * i;
+                if (row >= n) continue;
+                const size_t o = (size_t)cell * n + row;
+                double v = acc[j][i][r];
+                if (addin) v += addin[o];
+                if (out32) out32[o] = (float)v;
+                else out[o] = add ? out[o] + v : v;
+            }
         }
-    }
 }
 
 __global__ void k_gather_dens(const double* __restrict__ x, const int* __restrict__ perm,
@@ -1512,8 +1550,13 @@ CellTiles make_level_tiles(const HostTree& t, int level, hipStream_t s) {
 void launch_level_gemm(const CellTiles& T, int blk, const double* M, bool trans, const double* in,
                        const double* addin, double* out, float* out32, bool add, hipStream_t s) {
     if (T.n == 0) return;
-    hipLaunchKernelGGL(k_level_gemm, dim3(div_up(blk, 64), T.n), dim3(256), 0, s, blk, T.cells.p, T.tiles.p, M,
-                       trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+    const int rb = div_up(blk, 64);
+    if (rb * T.n >= kGemmWideMin)
+        hipLaunchKernelGGL((k_level_gemm<2, 2, 2, 2, 32>), dim3(rb, T.n), dim3(256), 0, s, blk, T.cells.p, T.tiles.p,
+                           M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+    else
+        hipLaunchKernelGGL((k_level_gemm<4, 1, 1, 1, 64>), dim3(rb, T.n, 4), dim3(256), 0, s, blk, T.cells.p,
+                           T.tiles.p, M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
     TBEM_LAUNCH_CHECK();
 }
 
