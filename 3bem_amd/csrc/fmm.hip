@@ -38,13 +38,15 @@ constexpr size_t kM2lOutputBudget = size_t(6) << 30;
 
 // The point-target stage's leaf positions split between the one-wave kernel (leaves of
 // at most kWaveLeafMax points: one work item each, or chunks of a large one) and the
-// one-workgroup kernel (the rest), both ordered by decreasing work (split_leaves).
+// one-workgroup kernel (the rest, whole or in chunks), both ordered by decreasing work
+// (split_leaves).
 struct LeafSplit {
-    DevBuf<WaveItem> items;
-    DevBuf<WaveLeafParts> parts;
-    DevBuf<int> block;
-    int n_items = 0, n_parts = 0, n_block = 0;  // entries of items, parts, block (with padding)
-    int n_work = 0, n_block_leaves = 0;         // work items and workgroup leaves without it
+    DevBuf<WaveItem> items, block_items;
+    DevBuf<WaveLeafParts> parts;  // the wave items' cut leaves, then the block items'
+    DevBuf<int> block;            // the leaves of block_items, whole (the gradient)
+    int n_items = 0, n_block_items = 0, n_block = 0;  // entries of items, block_items, block (with padding)
+    int n_parts = 0, n_wave_parts = 0;
+    int n_work = 0, n_block_leaves = 0;               // work items and workgroup leaves without padding
     size_t part_size = 0;  // doubles of chunk sums between the kernels (Work::wpart)
 };
 
@@ -56,6 +58,8 @@ struct FmmPlan {
     size_t order = 0, leaf = 0;
     bool small_cells = false;
     LeafSplit leaf_split;  // of the observation leaves (forward)
+    LeafSplit surf_split;  // the same leaves without their point sources: the surface
+                           // sources alone, where the point pairs run beside the far field
     // Symmetric point pairs (Kelvin U or the Laplace single layer, one shared tree;
     // forward and transpose): the pairs of neighbouring leaves of kSymLeafMin ..
     // kSymLeafMax points, listed both ways, are evaluated once for both directions
@@ -67,8 +71,11 @@ struct FmmPlan {
         bool on = false;
         DevList ord, own;
         LeafSplit split;
-        DevBuf<int> base, order, g_pos, g_ptr, g_off;
-        int n_order = 0, n_g = 0, n_leaves = 0;
+        DevBuf<int> base, g_pos, g_ptr, g_off;
+        DevBuf<WaveItem> items;         // the owners, whole or in chunks (pos, v0, v1, part)
+        DevBuf<WaveLeafParts> g_parts;  // per receiving or cut position, its chunks
+        int n_items = 0, n_g = 0, n_leaves = 0;
+        size_t part_size = 0;           // doubles of the chunks' target sums (Work::wsym)
         size_t n_rev = 0;
         double pairs = 0;  // unordered point pairs
         std::vector<int> part_ptr, part;  // per position, its partner leaves (sorted): the
@@ -101,6 +108,7 @@ struct FmmPlan {
         std::vector<DevList> m2m;    // by src level L >= 1: cells at L, entry = parent
         DevList leaf_p2p, leaf_p2l;  // indexed by source leaf position
         LeafSplit leaf_split;        // of the source leaves
+        LeafSplit surf_split;        // their surface sources alone
         DevList sym_ord;             // leaf_p2p without the symmetric pairs (FmmPlan::sym)
         LeafSplit sym_split;
         std::vector<CellTiles> t_slev;  // every cell of each source level
@@ -179,7 +187,8 @@ struct Work {
     DevBuf<double> e2;      // transpose: modal M2L^T contribution to ebar per source cell
     DevBuf<double> fld;     // raw check potentials of one stage, blk per cell (input of the C2E GEMMs)
     DevBuf<double> ty;      // per-pair output of the M2M / L2L class operators
-    DevBuf<double> wpart;   // chunk sums of the one-wave leaf kernel (LeafSplit::part_size)
+    DevBuf<double> wpart;   // chunk sums of the leaf kernels (LeafSplit::part_size)
+    DevBuf<double> wsym;    // target sums of the symmetric pairs' chunks (FmmPlan::sym.part_size)
     DevBuf<double> wrev;    // reverse sums of the symmetric pairs (R rows of FmmPlan::sym.n_rev)
     hipEvent_t ev[12];  // 0..7 stage boundaries; 8, 9 around the M2L translation kernel; 10, 11
                         // around the point-pair (P2P) launch on the side stream
@@ -214,8 +223,11 @@ struct Work {
         out_sorted.alloc(P.R * P.n_obs);
         fld.alloc((size_t)std::max(P.dst.n_cells, P.dot.n_cells) * P.blk);
         ty.alloc(P.tr_y);
-        wpart.alloc(std::max(P.leaf_split.part_size, P.sym.split.part_size));
-        if (P.sym.on) wrev.alloc((size_t)P.R * P.sym.n_rev);
+        wpart.alloc(std::max({P.leaf_split.part_size, P.surf_split.part_size, P.sym.split.part_size}));
+        if (P.sym.on) {
+            wrev.alloc((size_t)P.R * P.sym.n_rev);
+            wsym.alloc(P.sym.part_size);
+        }
         if (P.m2l_mfma.enabled && !P.m2l_mfma.fp64) {
             chk_up.alloc((size_t)P.dst.n_cells * P.blk);
             chk_up.zero(stream);  // cells without a P2M/M2M stage keep a zero potential
@@ -704,17 +716,25 @@ static void close_flags(DevList& l, const int* leaves, const DevTree& tt, const 
 
 // Splits the positions of a point-target list (items = leaves of tree tt; point
 // ranges pts, surface cells surf, and each leaf's own surface): leaves of at most
-// kWaveLeafMax points go to the one-wave kernel, one item each when they have at most
-// kWavePairsMax pairs (points x sources); larger ones of at most kWaveChunkLeaf points
-// are cut into chunks of about equal sources (points cut anywhere, surface cells
-// whole, the own surface with the last chunk), whose sums k_leaf_parts adds in chunk
-// order; the rest go to the one-workgroup kernel. Both lists are laid out by
-// xcd_layout: per XCD a run of neighbouring leaves, the most work first.
+// kWaveLeafMax points go to the one-wave kernel when they have at most kWavePairsMax
+// pairs (points x sources), or when they have at most kWaveChunkLeaf points, then cut into
+// chunks of about equal sources (points cut anywhere, surface cells whole, the own surface
+// with the last chunk), whose sums k_leaf_parts adds in chunk order; the rest go to the
+// one-workgroup kernel. Both lists are laid out by xcd_layout: per XCD a run of
+// neighbouring leaves, the most work first.
 // (kWaveChunkLeaf: a wave holds ceil(m/2) targets per source slice, so above 64
 // points one slice is left and down to half of its lanes idle, where the 512-thread
 // kernel keeps 96% busy.)
-constexpr int kWaveChunkLeaf = 64;
-
+// A small problem has fewer such items than the chip has room for, and its longest one
+// sets the launch's length. The items of both kernels are therefore also cut where they
+// exceed the problem's total pairs divided by kWaveFill (kBlockFill) items, four per SIMD
+// (compute unit), but not below kWaveCapMin (kBlockCapMin) pairs, where an item's fixed
+// costs would take over. These cuts fall on whole LDS tiles (wave: kWaveTile sources;
+// block_tile), so that the FP32 partial sum of every tile is the same as uncut.
+// Measured (whole passes): mesh of 9,102 points, hypersingular, mixed 1316 -> 823 us (its
+// block leaves 489 -> 57 us); sphere of 15,360 points, Laplace 310 -> 213 us (leaf waves
+// 67 -> 22 us, symmetric pairs 95 -> 38); 300,007 points, order 50, mixed, forward and
+// backward 6.10 -> 4.30 ms; from about 1e9 pairs on nothing is cut that was not before.
 // Lays out work items (work, item), given in tree order, for a launch whose workgroup
 // b runs on XCD b % 8 (the hardware deals workgroups to the XCDs in turn), g items per
 // workgroup. The items are cut into 8 runs of about equal work, one per XCD, so that
@@ -747,39 +767,63 @@ static std::vector<I> xcd_layout(const std::vector<std::pair<long, I>>& items, i
     return out;
 }
 
+constexpr int kWaveChunkLeaf = 64;
+constexpr long kWaveFill = 4096, kWaveCapMin = 4096;
+constexpr long kBlockFill = 2048, kBlockCapMin = 16384;
+
 static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
-                         const HostList& surf, int n_e, LeafSplit& out, hipStream_t s) {
-    std::vector<std::pair<long, WaveItem>> w;
+                         const HostList& surf, int n_e, int block_tile, LeafSplit& out, hipStream_t s) {
+    std::vector<std::pair<long, WaveItem>> w, bi;
     std::vector<std::pair<long, int>> b;
-    std::vector<WaveLeafParts> parts;
+    std::vector<WaveLeafParts> wparts, bparts;
+    auto points_of = [&](size_t k) {
+        const int p0 = pts.ptr.empty() ? 0 : pts.ptr[k], p1 = pts.ptr.empty() ? 0 : pts.ptr[k + 1];
+        return p0 < p1 ? (long)pts.rpre[p1 - 1] + pts.rcnt[p1 - 1] : 0;
+    };
+    auto cells_of = [&](size_t k) { return surf.ptr.empty() ? 0 : surf.ptr[k + 1] - surf.ptr[k]; };
+    long total = 0;
+    for (size_t k = 0; k < leaves.size(); k++)
+        total += (long)tt.count[leaves[k]] * (points_of(k) + (long)n_e * (cells_of(k) + 1));
+    const long wave_cap = std::max(kWaveCapMin, total / kWaveFill), block_cap = std::max(kBlockCapMin, total / kBlockFill);
     long part = 0;
     for (size_t k = 0; k < leaves.size(); k++) {
         const int pos = (int)k;
         const long m = tt.count[leaves[k]];
         if (m == 0) continue;  // no targets, nothing to write
         const int p0 = pts.ptr.empty() ? 0 : pts.ptr[k], p1 = pts.ptr.empty() ? 0 : pts.ptr[k + 1];
-        const long np = p0 < p1 ? (long)pts.rpre[p1 - 1] + pts.rcnt[p1 - 1] : 0;
-        const int c0 = surf.ptr.empty() ? 0 : surf.ptr[k], c1 = surf.ptr.empty() ? 0 : surf.ptr[k + 1];
+        const long np = points_of(k);
+        const int c0 = surf.ptr.empty() ? 0 : surf.ptr[k], c1 = c0 + cells_of(k);
         const long src = np + (long)n_e * (c1 - c0 + 1);
         const long nc = (m * src + kWavePairsMax - 1) / kWavePairsMax;
-        if (m <= kWaveLeafMax && nc <= 1) {
-            w.push_back({m * src, WaveItem{pos, p0, p1, 0, (int)np, c0, c1, 1, -1}});
+        const bool wave = m <= (nc <= 1 ? kWaveLeafMax : kWaveChunkLeaf);
+        if (!wave) b.push_back({m * src, pos});
+        // runs of at most `per` sources, each cut further into chunks of at most `sub`
+        // points, whole tiles from the run's start
+        const long tile = wave ? kWaveTile : block_tile, cap = wave ? wave_cap : block_cap;
+        const long per = wave && nc > 1 ? (src + nc - 1) / nc : std::max(1L, src);
+        const long sub = m * src > cap ? std::max(1L, (cap / m + tile - 1) / tile) * tile : per;
+        long n_chunks = (np + per - 1) / per * ((per + sub - 1) / sub) + (c1 - c0) + 1;  // at most
+        if ((nc <= 1 || !wave) && np <= sub) n_chunks = 1;
+        auto& items = wave ? w : bi;
+        if (n_chunks == 1 || part + n_chunks * kPartRows * m > INT32_MAX) {
+            if (wave && nc > 1 && n_chunks > 1) {  // no room for its sums: a whole workgroup
+                b.push_back({m * src, pos});
+                bi.push_back({m * src, WaveItem{pos, p0, p1, 0, (int)np, c0, c1, 1, -1}});
+            } else {
+                items.push_back({m * src, WaveItem{pos, p0, p1, 0, (int)np, c0, c1, 1, -1}});
+            }
             continue;
         }
-        if (m > kWaveChunkLeaf || part + (nc + 1) * kPartRows * m > INT32_MAX) {
-            b.push_back({m * src, pos});
-            continue;
-        }
-        const long per = (src + nc - 1) / nc;
         std::vector<std::pair<long, WaveItem>> ch;
         const auto pre = pts.rpre.begin();
-        for (long v = 0; v < np; v += per) {
-            const int v0 = (int)v, v1 = (int)std::min(np, v + per);
-            const int f0 = (int)(std::upper_bound(pre + p0, pre + p1, v0) - pre) - 1;
-            const int f1 = (int)(std::lower_bound(pre + p0, pre + p1, v1) - pre);
-            ch.push_back({m * (v1 - v0), WaveItem{pos, f0, f1, v0, v1, 0, 0, 0, 0}});
-        }
-        const int cpc = (int)std::max(1L, per / std::max(1, n_e));
+        for (long run = 0; run < np; run += per)
+            for (long v = run, end = std::min(np, run + per); v < end; v += sub) {
+                const int v0 = (int)v, v1 = (int)std::min(end, v + sub);
+                const int f0 = (int)(std::upper_bound(pre + p0, pre + p1, v0) - pre) - 1;
+                const int f1 = (int)(std::lower_bound(pre + p0, pre + p1, v1) - pre);
+                ch.push_back({m * (v1 - v0), WaveItem{pos, f0, f1, v0, v1, 0, 0, 0, 0}});
+            }
+        const int cpc = (int)std::max(1L, std::min(per, sub) / std::max(1, n_e));
         for (int c = c0; c < c1; c += cpc) {
             const int ce = std::min(c1, c + cpc);
             ch.push_back({m * n_e * (ce - c), WaveItem{pos, 0, 0, 0, 0, c, ce, 0, 0}});
@@ -789,23 +833,27 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
         ch.back().first += m * n_e;
         for (size_t j = 0; j < ch.size(); j++) {
             ch[j].second.part = (int)(part + (long)j * kPartRows * m);
-            w.push_back(ch[j]);
+            items.push_back(ch[j]);
         }
-        parts.push_back(WaveLeafParts{pos, (int)part, (int)ch.size()});
+        (wave ? wparts : bparts).push_back(WaveLeafParts{pos, (int)part, (int)ch.size()});
         part += (long)ch.size() * kPartRows * m;
     }
-    const std::vector<WaveItem> wi =
-        xcd_layout(w, kWaveBlock / 64, WaveItem{-1, 0, 0, 0, 0, 0, 0, 0, -1});
-    const std::vector<int> bl = xcd_layout(b, 1, -1);
+    const WaveItem empty{-1, 0, 0, 0, 0, 0, 0, 0, -1};
+    const std::vector<WaveItem> wi = xcd_layout(w, kWaveBlock / 64, empty), bl = xcd_layout(bi, 1, empty);
+    const std::vector<int> whole = xcd_layout(b, 1, -1);
     out.n_work = (int)w.size();
     out.n_block_leaves = (int)b.size();
     out.n_items = (int)wi.size();
-    out.n_parts = (int)parts.size();
-    out.n_block = (int)bl.size();
+    out.n_block_items = (int)bl.size();
+    out.n_block = (int)whole.size();
+    out.n_wave_parts = (int)wparts.size();
+    wparts.insert(wparts.end(), bparts.begin(), bparts.end());
+    out.n_parts = (int)wparts.size();
     out.part_size = (size_t)part;
     out.items.upload(wi, s);
-    out.parts.upload(parts, s);
-    out.block.upload(bl, s);
+    out.block_items.upload(bl, s);
+    out.parts.upload(wparts, s);
+    out.block.upload(whole, s);
 }
 
 // FmmPlan::sym from the P2P pairs of the shared tree T (forward lists by leaf
@@ -897,14 +945,35 @@ static void build_sym(FmmPlan& P, const HostTree& T, const std::vector<std::arra
     cells_to_ranges(own, T);
     clk.mark("sym: ranges");
     std::vector<int> base(nl, 0);
-    std::vector<std::pair<long, int>> work;
-    size_t n_rev = 0;
+    std::vector<std::pair<long, WaveItem>> work;
+    size_t n_rev = 0, part = 0;
+    double all = 0;
+    for (int k = 0; k < nl; k++)
+        if (own.ptr[k] < own.ptr[k + 1])
+            all += (double)T.count[leaves[k]] * (own.rpre[own.ptr[k + 1] - 1] + own.rcnt[own.ptr[k + 1] - 1]);
+    // a small problem's owners are cut into chunks of whole wave blocks (64 x kSymSrc
+    // points, which keeps FP32 sums what they are uncut), at least one for each wave of
+    // the workgroup, so that the launch has about kSymFill workgroups
+    constexpr long kSymFill = 2048, kBlockPts = 64 * kSymSrc, kSymSubMin = kBlockPts * (kSymBlock / 64);
+    std::vector<WaveLeafParts> cut(nl, WaveLeafParts{0, 0, 0});
     for (int k = 0; k < nl; k++) {
         base[k] = (int)n_rev;
         const int e0 = own.ptr[k], e1 = own.ptr[k + 1];
         if (e0 == e1) continue;
         const long n = (long)own.rpre[e1 - 1] + own.rcnt[e1 - 1];
-        work.push_back({n * T.count[leaves[k]], k});
+        const long m = T.count[leaves[k]];
+        const long sub = std::max(kSymSubMin, (long)(all / kSymFill) / m);
+        const long nch = (n + sub - 1) / sub;
+        if (nch == 1 || part + (size_t)(nch * P.R * m) > (size_t)INT32_MAX) {
+            work.push_back({n * m, WaveItem{k, 0, 0, 0, (int)n, 0, 0, 0, -1}});
+        } else {
+            const long per = ((n + nch - 1) / nch + kBlockPts - 1) / kBlockPts * kBlockPts;
+            cut[k] = WaveLeafParts{k, (int)part, 0};
+            for (long v = 0; v < n; v += per, part += P.R * m, cut[k].n++)
+                work.push_back({std::min(per, n - v) * m,
+                                WaveItem{k, 0, 0, (int)v, (int)std::min(n, v + per), 0, 0, 0, (int)part}});
+        }
+        Y.n_leaves++;
         Y.pairs += (double)n * T.count[leaves[k]];
         n_rev += (size_t)n;
         TBEM_REQUIRE(n_rev <= (size_t)INT32_MAX, TBEM_E_UNSUPPORTED, "symmetric pairs: too many slots");
@@ -926,30 +995,33 @@ static void build_sym(FmmPlan& P, const HostTree& T, const std::vector<std::arra
     std::vector<int> g_cnt(nl, 0);
     for (size_t q = 0; q < own_cells.size(); q++) g_cnt[pos_of[own_cells[q]]]++;
     std::vector<int> g_pos, g_ptr(1, 0), g_at(nl, -1);
+    std::vector<WaveLeafParts> g_parts;
     for (int k = 0; k < nl; k++) {
-        if (g_cnt[k] == 0) continue;
+        if (g_cnt[k] == 0 && cut[k].n == 0) continue;
         g_at[k] = g_ptr.back();
         g_pos.push_back(k);
+        g_parts.push_back(cut[k]);
         g_ptr.push_back(g_ptr.back() + g_cnt[k]);
     }
     std::vector<int> g_off(g_ptr.back());
     for (int k = 0; k < nl; k++)
         for (int q = own_ptr[k]; q < own_ptr[k + 1]; q++) g_off[g_at[pos_of[own_cells[q]]]++] = slot[q];
-    const std::vector<int> order = xcd_layout(work, 1, -1);
+    const std::vector<WaveItem> items = xcd_layout(work, 1, WaveItem{-1, 0, 0, 0, 0, 0, 0, 0, -1});
     clk.mark("sym: slots");
     Y.ord.upload(ord, s);
     Y.own.upload(own, s);
     Y.base.upload(base, s);
-    Y.order.upload(order, s);
+    Y.items.upload(items, s);
     Y.g_pos.upload(g_pos, s);
     Y.g_ptr.upload(g_ptr, s);
     Y.g_off.upload(g_off, s);
-    Y.n_order = (int)order.size();
-    Y.n_leaves = (int)work.size();
+    Y.g_parts.upload(g_parts, s);
+    Y.n_items = (int)items.size();
+    Y.part_size = part;
     Y.n_g = (int)g_pos.size();
     Y.n_rev = n_rev;
     clk.mark("sym: upload");
-    split_leaves(T, leaves, ord, lm, P.n_e, Y.split, s);
+    split_leaves(T, leaves, ord, lm, P.n_e, leaf_stage_tile(P.kid, P.precision == TBEM_MIXED), Y.split, s);
     clk.mark("sym: split");
     close_flags(Y.ord, P.obs_leaves.p, P.dot, P.op, P.sp, s);
     Y.on = true;
@@ -1130,7 +1202,9 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
         const HostList lm = list_from_pairs(OT.leaves, OT.n_cells, tl.m2p, 0, nullptr);
         P->leaf_p2p.upload(lp, s);
         P->leaf_m2p.upload(lm, s);
-        split_leaves(OT, OT.leaves, lp, lm, P->n_e, P->leaf_split, s);
+        const int tile = leaf_stage_tile(P->kid, P->precision == TBEM_MIXED);
+        split_leaves(OT, OT.leaves, lp, lm, P->n_e, tile, P->leaf_split, s);
+        split_leaves(OT, OT.leaves, HostList(), lm, P->n_e, tile, P->surf_split, s);
         clk.mark("leaf lists");
         if (P->same_tree && (P->kid == TBEM_K_ELASTIC_DISPLACEMENT || P->kid == TBEM_K_LAPLACE_SINGLE) &&
             d->point_pairs == TBEM_POINT_PAIRS_AUTO)
@@ -1166,7 +1240,9 @@ const FmmPlan::AdjLists& FmmPlan::adjoint_lists(hipStream_t s) const {
         const HostList ll = list_from_pairs(ST.leaves, ST.n_cells, tl.p2l, 1, nullptr);
         A->leaf_p2p.upload(lp, s);
         A->leaf_p2l.upload(ll, s);
-        split_leaves(ST, ST.leaves, lp, ll, n_e, A->leaf_split, s);
+        const int tile = leaf_stage_tile(kid, precision == TBEM_MIXED);
+        split_leaves(ST, ST.leaves, lp, ll, n_e, tile, A->leaf_split, s);
+        split_leaves(ST, ST.leaves, HostList(), ll, n_e, tile, A->surf_split, s);
         if (sym.on) {  // one shared tree: source leaf positions are the forward's
             HostList ord = list_from_pairs(ST.leaves, ST.n_cells, tl.p2p, 1, nullptr);
             const size_t nl = ord.ptr.size() - 1;
@@ -1196,7 +1272,7 @@ const FmmPlan::AdjLists& FmmPlan::adjoint_lists(hipStream_t s) const {
             ord.cell = std::move(cell);
             cells_to_ranges(ord, ST);
             A->sym_ord.upload(ord, s);
-            split_leaves(ST, ST.leaves, ord, ll, n_e, A->sym_split, s);
+            split_leaves(ST, ST.leaves, ord, ll, n_e, tile, A->sym_split, s);
             close_flags(A->sym_ord, src_leaves.p, dst, sp, op, s);
         }
     }
@@ -1337,8 +1413,10 @@ static void set_split(LeafStage& f, const LeafSplit& sp, Work& W) {
         TBEM_HIP(hipEventSynchronize(W.done));
         W.wpart.alloc(sp.part_size);
     }
+    f.split = 1;
     f.wave_items = sp.items.p; f.n_wave = sp.n_items;
-    f.wave_parts = sp.parts.p; f.n_parts = sp.n_parts; f.part_buf = W.wpart.p;
+    f.block_items = sp.block_items.p; f.n_block_items = sp.n_block_items;
+    f.parts = sp.parts.p; f.n_parts = sp.n_parts; f.n_wave_parts = sp.n_wave_parts; f.part_buf = W.wpart.p;
     f.block_pos = sp.block.p; f.n_block = sp.n_block;
 }
 
@@ -1354,8 +1432,8 @@ static void use_sym(LeafStage& f, const FmmPlan& P, Work& W, const FmmPlan::AdjL
     f.rp_pre = o.rpre.p; f.rp_close = o.rclose.p;
     set_split(f, A ? A->sym_split : Y.split, W);
     f.sy_ptr = Y.own.ptr.p; f.sy_beg = Y.own.rbeg.p; f.sy_cnt = Y.own.rcnt.p; f.sy_pre = Y.own.rpre.p;
-    f.sy_base = Y.base.p; f.sy_order = Y.order.p; f.n_sy_order = Y.n_order;
-    f.sg_pos = Y.g_pos.p; f.sg_ptr = Y.g_ptr.p; f.sg_off = Y.g_off.p; f.n_sg = Y.n_g;
+    f.sy_base = Y.base.p; f.sy_items = Y.items.p; f.n_sy_items = Y.n_items; f.sy_part_buf = W.wsym.p;
+    f.sg_pos = Y.g_pos.p; f.sg_ptr = Y.g_ptr.p; f.sg_off = Y.g_off.p; f.sg_parts = Y.g_parts.p; f.n_sg = Y.n_g;
     f.rev = W.wrev.p; f.n_rev = Y.n_rev;
 }
 
@@ -1408,6 +1486,7 @@ static void forward_T(const FmmPlan& P, Work& W, const double* x, double* y, hip
         // then M2P + L2P (FP64) added to the P2P output
         TBEM_HIP(hipStreamWaitEvent(s, W.join, 0));
         LeafStage f = leaf_stage_args(P, W);
+        set_split(f, P.surf_split, W);
         f.rp_ptr = nullptr;
         f.accumulate = 1;
         launch_leaf_stage<double>(P.kid, false, f, P.kc, s, true);
@@ -1589,6 +1668,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
     if (split) {  // P2L^T + P2M^T (FP64) added to the side stream's P2P^T
         TBEM_HIP(hipStreamWaitEvent(s, W.join, 0));
         LeafStage f = leaf_args();
+        set_split(f, A.surf_split, W);
         f.rp_ptr = nullptr;
         f.accumulate = 1;
         launch_leaf_stage<double>(P.kid, true, f, P.kc, s, true);
@@ -1952,7 +2032,7 @@ int tbem_fmm_info(tbem_fmm_t h, tbem_fmm_info_t* o) {
         double wb = 0;
         for (const DevBuf<double>* b : {&W.dens, &W.mult, &W.locals, &W.out_sorted, &W.xbuf, &W.ybuf, &W.gsort,
                                         &W.lbar, &W.cbar, &W.mbar, &W.ebar, &W.grad_sorted, &W.e2, &W.fld, &W.ty,
-                                        &W.wpart, &W.wrev})
+                                        &W.wpart, &W.wsym, &W.wrev})
             wb += (double)b->n * sizeof(double);
         for (const DevBuf<float>* b : {&W.chk_up, &W.m2l_w}) wb += (double)b->n * sizeof(float);
         o->work_bytes = wb;

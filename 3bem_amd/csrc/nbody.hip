@@ -218,8 +218,9 @@ static void nb_adjoint(NbodyPlan& P, const double* g, double* y, hipStream_t s) 
 }
 
 static void set_items(LeafStage& f, const Split& sp, double* parts) {
+    f.split = 1;
     f.block_items = sp.items.p; f.n_block_items = sp.n_items;
-    f.block_parts = sp.parts.p; f.n_block_parts = sp.n_parts;
+    f.parts = sp.parts.p; f.n_parts = sp.n_parts;
     f.part_buf = parts;
 }
 

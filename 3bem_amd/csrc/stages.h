@@ -42,6 +42,7 @@ constexpr int kWaveBlock = 256;        // k_leaf_wave: four work items per workg
 constexpr int kWaveLeafMax = 128;      // leaves of up to this many points go to k_leaf_wave ...
 constexpr long kWavePairsMax = 65536;  // ... one wave per leaf, or per chunk of at most this
                                        // many pairs (points x sources) of a larger one
+constexpr int kWaveTile = 64;          // k_leaf_wave's sources per LDS tile
 constexpr int kPartsBlock = 128;       // k_leaf_parts
 constexpr int kSymBlock = 256;         // k_leaf_sym: four waves per leaf
 constexpr int kSymLeafMin = 16;        // k_leaf_sym takes leaves of kSymLeafMin .. kSymLeafMax
@@ -152,40 +153,45 @@ struct LeafStage {
     int n_e, blk;
     double* out_sorted;
     int accumulate;         // out_sorted += (instead of =) the stage's sums
-    // The leaf positions a launch serves (null: 0 .. n_leaves-1, one workgroup each).
+    // The leaf positions a gradient launch serves (null: 0 .. n_leaves-1, one workgroup each).
     const int* order;
     int n_order;
-    // Optional split of the positions (launch_leaf_stage): wave_items, leaves of at most
+    // Optional split of the positions (launch_leaf_stage; split = 0: none): wave_items, leaves of at most
     // kWaveLeafMax points, whole or in chunks, one wave each, the most work first;
-    // block_pos, the rest, one workgroup each. wave_parts: the leaves cut into chunks,
-    // whose partial sums part_buf holds between the two kernels.
-    const WaveItem* wave_items;
+    // block_items, the rest, whole or in chunks, one workgroup each (block_pos: the same
+    // leaves whole, for the gradient). parts: the leaves cut into chunks, the n_wave_parts
+    // of wave_items first, whose partial sums part_buf holds between the kernels.
+    int split, split_rest;  // split_rest: the launch after wave_items'
+    const WaveItem *wave_items, *block_items;
     const int* block_pos;
-    int n_wave, n_block;
-    const WaveLeafParts* wave_parts;
-    int n_parts;
+    int n_wave, n_block_items, n_block;
+    const WaveLeafParts* parts;
+    int n_wave_parts, n_parts;
     double* part_buf;
-    // The one-workgroup kernel's work items (null: whole leaves, above): a leaf, or a part
-    // of its sources, whose partial sums go to part_buf; block_parts: the leaves cut.
-    const WaveItem* block_items;
-    const WaveLeafParts* block_parts;
-    int n_block_items, n_block_parts;
     const double* grad_g;   // obs-gradient mode: upstream g (sorted, component-major)
     double* grad_out;       // obs-gradient mode: 3 per target (sorted, AoS)
     // Symmetric pairs (Kelvin U with one point set on both sides; null: none). Per leaf
     // position, the point ranges of the leaves whose pairs with it k_leaf_sym
     // evaluates once for both directions (the rp_* lists then leave those pairs
     // out): sy_base[pos] is the first slot of the leaf's reverse sums in rev (R
-    // component rows of n_rev); sy_order: the positions that own pairs, one
-    // workgroup each; sg_pos / sg_ptr / sg_off: per receiving position, the slot
-    // offsets (in rev) of the sums addressed to its first point, added in list order.
-    const int *sy_ptr, *sy_beg, *sy_cnt, *sy_pre, *sy_base, *sy_order;
-    int n_sy_order;
+    // component rows of n_rev); sy_items: the positions that own pairs, one
+    // workgroup each, or one per chunk [v0, v1) of the owned points, whose target sums
+    // go to sy_part_buf; sg_pos / sg_ptr / sg_off: per receiving or cut position, the slot
+    // offsets (in rev) of the sums addressed to its first point, added in list order after
+    // its own chunks' (sg_parts, n = 0: not cut).
+    const int *sy_ptr, *sy_beg, *sy_cnt, *sy_pre, *sy_base;
+    const WaveItem* sy_items;
+    int n_sy_items;
+    double* sy_part_buf;
     const int *sg_pos, *sg_ptr, *sg_off;
+    const WaveLeafParts* sg_parts;
     int n_sg;
     double* rev;
     size_t n_rev;
 };
+
+// Sources per LDS tile of k_leaf_stage for a kernel and precision of the point pairs.
+int leaf_stage_tile(int kid, bool fp32);
 
 // FP64 only: every check potential here feeds a check-to-equivalent pseudo-inverse
 // (or is the transpose of such a step), whose conditioning FP32 input cannot survive.

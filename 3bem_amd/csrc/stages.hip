@@ -458,8 +458,8 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
     __shared__ StageSmem<T, R, NRM, NB, 2 * R> sm;
-    const WaveItem* it = a.block_items ? a.block_items + blockIdx.x : nullptr;
-    const int pos = it ? uni(it->pos) : a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
+    const WaveItem* it = a.split ? a.block_items + blockIdx.x : nullptr;
+    const int pos = it ? uni(it->pos) : (int)blockIdx.x;
     if (pos < 0) return;  // padding of the layout (the whole workgroup)
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
@@ -749,9 +749,8 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
 
 // The leaves that ran in chunks: one workgroup per leaf and output component (grid y),
 // the chunks' partial sums added in chunk order, eight loads in flight.
-__global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, const WaveLeafParts* __restrict__ parts,
-                                                           double scale) {
-    const WaveLeafParts lp = parts[blockIdx.x];
+__global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, double scale) {
+    const WaveLeafParts lp = a.parts[blockIdx.x];
     const int leaf = a.leaves[lp.pos], q = blockIdx.y;
     const int b = a.tt.begin[leaf], m = a.tt.count[leaf];
     const size_t step = (size_t)kPartRows * m;
@@ -902,12 +901,13 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
     constexpr int R = kernel_dim(KID);
     __shared__ SymTarget tg[kSymSlots];
     __shared__ double facc[NW][3 * kSymSlots];
-    const int pos = uni(a.sy_order[blockIdx.x]);
+    const WaveItem* it = a.sy_items + blockIdx.x;
+    const int pos = uni(it->pos);
     if (pos < 0) return;  // padding of the layout (the whole workgroup)
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
     const int e0 = uni(a.sy_ptr[pos]), e1 = uni(a.sy_ptr[pos + 1]);
-    const int n = uni(a.sy_pre[e1 - 1] + a.sy_cnt[e1 - 1]);  // listed positions own at least one range
+    const int n0 = uni(it->v0), n = uni(it->v1), part = uni(it->part);  // the owned points it takes
     const size_t base = (size_t)uni(a.sy_base[pos]);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     // slots per group copy (r + k < S), the copies, and this lane's group and offset:
@@ -953,7 +953,7 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
     }
     double* fa = facc[w] + gc * S;
     constexpr int PB = 64 * kSymSrc;  // stream positions per wave block
-    for (int p0 = w * PB; p0 < n; p0 += NW * PB) {
+    for (int p0 = n0 + w * PB; p0 < n; p0 += NW * PB) {
         SymSource<T> sv[kSymSrc];
         int close = 0;
         for (int u = 0; u < kSymSrc; u++) sym_load<R>(sv[u], p0 + 64 * u + lane, n, e0, e1, a, bx, close);
@@ -980,23 +980,30 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
                 s += f[i];
                 if (i + m < S) s += f[i + m];
             }
+        if (part >= 0) {  // k_sym_gather adds the leaf's chunks
+            a.sy_part_buf[(size_t)part + o] = s;
+            continue;
+        }
         const double wgt = a.t_weight ? a.t_weight[b + i] : 1.0;
         double* out = a.out_sorted + (size_t)q * a.n_tgt + b + i;
         *out += wgt * (s * scale);
     }
 }
 
-// u of the leaves at sg_pos += the reverse sums addressed to them, slot by slot in
-// list order
+// u of the leaves at sg_pos += the target sums of their own chunks, where k_leaf_sym ran
+// them in chunks, then += the reverse sums addressed to them, slot by slot in list order
 __global__ __launch_bounds__(256) void k_sym_gather(LeafStage a, int R, double scale) {
     const int pos = a.sg_pos[blockIdx.x];
     const int leaf = a.leaves[pos];
     const int b = a.tt.begin[leaf], m = a.tt.count[leaf];
     const int e0 = a.sg_ptr[blockIdx.x], e1 = a.sg_ptr[blockIdx.x + 1];
+    const WaveLeafParts lp = a.sg_parts[blockIdx.x];
     for (int o = threadIdx.x; o < R * m; o += 256) {
         const int q = o / m, i = o - q * m;
         const double* r = a.rev + (size_t)q * a.n_rev + i;
-        double s = 0;
+        const double* p = a.sy_part_buf + (size_t)lp.part + o;
+        double f = 0, s = 0;
+        for (int c = 0; c < lp.n; c++) f += p[(size_t)c * R * m];
         int e = e0;
         for (; e + 8 <= e1; e += 8) {  // eight loads in flight, added in list order
             double v[8];
@@ -1006,7 +1013,10 @@ __global__ __launch_bounds__(256) void k_sym_gather(LeafStage a, int R, double s
         for (; e < e1; e++) s += r[a.sg_off[e]];
         const double wgt = a.t_weight ? a.t_weight[b + i] : 1.0;
         double* out = a.out_sorted + (size_t)q * a.n_tgt + b + i;
-        *out += wgt * (s * scale);
+        double u = *out;
+        if (lp.n > 0) u += wgt * (f * scale);
+        if (e0 < e1) u += wgt * (s * scale);
+        *out = u;
     }
 }
 
@@ -1375,7 +1385,7 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_grad2_wave(LeafStage a, KC<
 
 // The gradient's chunked leaves: grad_out[3 i + mm] = the chunks' sums, in chunk order.
 __global__ __launch_bounds__(kWaveLeafMax) void k_leaf_grad_parts(LeafStage a, double scale) {
-    const WaveLeafParts lp = a.wave_parts[blockIdx.x];
+    const WaveLeafParts lp = a.parts[blockIdx.x];
     const int leaf = a.leaves[lp.pos];
     const int b = a.tt.begin[leaf], m = a.tt.count[leaf];
     const int t = threadIdx.x;
@@ -1682,7 +1692,7 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
     const KC<T> kc = kc_of<T>(c);
     const KC<double> kc64 = make_kc64(c);
     const double scale = (double)kop_scale<KID, double>(kc64);
-    if (a.wave_items || a.block_pos) {  // small leaves one wave per item, the rest one workgroup each
+    if (a.split && !a.split_rest) {  // small leaves one wave per item, the rest one workgroup per item
         if (a.n_wave > 0) {
             const dim3 g((a.n_wave + kWaveBlock / 64 - 1) / (kWaveBlock / 64)), b(kWaveBlock);
             const bool f64 = fast && std::is_same<T, double>::value;
@@ -1694,28 +1704,16 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
                 else hipLaunchKernelGGL((k_leaf_wave<KID, T, false, false>), g, b, 0, s, a, kc, kc64, scale);
             }
             TBEM_LAUNCH_CHECK();
-            if (a.n_parts > 0) {
-                hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_parts, kernel_dim(KID)), dim3(kPartsBlock), 0, s, a,
-                                   a.wave_parts, scale);
-                TBEM_LAUNCH_CHECK();
-            }
         }
-        if (a.n_block > 0) {
-            LeafStage bl = a;
-            bl.order = a.block_pos;
-            bl.n_order = a.n_block;
-            bl.wave_items = nullptr;
-            bl.block_pos = nullptr;
-            bl.n_wave = bl.n_parts = 0;
-            bl.sy_order = nullptr;
-            leaf_launch<KID, T>(adj, fast, bl, c, s);
-        }
-        if (a.sy_order && a.rp_ptr) {  // the pairs left out of the rp_* lists, then their reverse sums
+        LeafStage bl = a;
+        bl.split_rest = 1;
+        leaf_launch<KID, T>(adj, fast, bl, c, s);  // block_items, then the parts of both
+        if (a.sy_items && a.rp_ptr) {  // the pairs left out of the rp_* lists, then their reverse sums
             TBEM_REQUIRE((KID == K_EU || KID == K_LS) && fast, TBEM_E_INVALID,
                          "symmetric pairs: Kelvin U and the Laplace single layer only");
-            if (a.n_sy_order > 0) {
+            if (a.n_sy_items > 0) {
                 if constexpr (KID == K_EU || KID == K_LS)
-                    hipLaunchKernelGGL((k_leaf_sym<KID, T>), dim3(a.n_sy_order), dim3(kSymBlock), 0, s, a, kc,
+                    hipLaunchKernelGGL((k_leaf_sym<KID, T>), dim3(a.n_sy_items), dim3(kSymBlock), 0, s, a, kc,
                                        scale);
                 TBEM_LAUNCH_CHECK();
             }
@@ -1726,25 +1724,27 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
         }
         return;
     }
-    dim3 g(a.block_items ? a.n_block_items : a.order ? a.n_order : a.n_leaves), b(leaf_block<KID, T>());
-    // the one-step rsqrt only differs from the full one in FP64
-    if (fast && std::is_same<T, double>::value && a.rp_close && a.rp_ptr) {
-        if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, true, true>), g, b, 0, s, a, kc, kc64, scale);
-        else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, true, true>), g, b, 0, s, a, kc, kc64, scale);
-    } else if (std::is_same<T, float>::value && a.rp_close && a.rp_ptr) {
-        if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, false, true>), g, b, 0, s, a, kc, kc64, scale);
-        else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, false, true>), g, b, 0, s, a, kc, kc64, scale);
-    } else if (fast && std::is_same<T, double>::value) {
-        if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, true>), g, b, 0, s, a, kc, kc64, scale);
-        else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, true>), g, b, 0, s, a, kc, kc64, scale);
-    } else {
-        if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, false>), g, b, 0, s, a, kc, kc64, scale);
-        else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, false>), g, b, 0, s, a, kc, kc64, scale);
+    const int n_blocks = a.split ? a.n_block_items : a.n_leaves;
+    if (n_blocks > 0) {
+        const dim3 g(n_blocks), b(leaf_block<KID, T>());
+        // the one-step rsqrt only differs from the full one in FP64
+        if (fast && std::is_same<T, double>::value && a.rp_close && a.rp_ptr) {
+            if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, true, true>), g, b, 0, s, a, kc, kc64, scale);
+            else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, true, true>), g, b, 0, s, a, kc, kc64, scale);
+        } else if (std::is_same<T, float>::value && a.rp_close && a.rp_ptr) {
+            if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, false, true>), g, b, 0, s, a, kc, kc64, scale);
+            else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, false, true>), g, b, 0, s, a, kc, kc64, scale);
+        } else if (fast && std::is_same<T, double>::value) {
+            if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, true>), g, b, 0, s, a, kc, kc64, scale);
+            else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, true>), g, b, 0, s, a, kc, kc64, scale);
+        } else {
+            if (adj) hipLaunchKernelGGL((k_leaf_stage<KID, T, true, false>), g, b, 0, s, a, kc, kc64, scale);
+            else hipLaunchKernelGGL((k_leaf_stage<KID, T, false, false>), g, b, 0, s, a, kc, kc64, scale);
+        }
+        TBEM_LAUNCH_CHECK();
     }
-    TBEM_LAUNCH_CHECK();
-    if (a.block_items && a.n_block_parts > 0) {
-        hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_block_parts, kernel_dim(KID)), dim3(kPartsBlock), 0, s, a,
-                           a.block_parts, scale);
+    if (a.n_parts > 0) {
+        hipLaunchKernelGGL(k_leaf_parts, dim3(a.n_parts, kernel_dim(KID)), dim3(kPartsBlock), 0, s, a, scale);
         TBEM_LAUNCH_CHECK();
     }
 }
@@ -1754,7 +1754,7 @@ static void grad_launch(bool fp32_points, const LeafStage& a, const KConst& c, h
     if (a.n_leaves == 0) return;
     const double scale = (double)kop_scale<KID, double>(make_kc64(c));
     if constexpr (has_analytic_grad(KID)) {
-        if (a.wave_items || a.block_pos) {  // the forward's split: small leaves and chunks on waves
+        if (a.split) {  // the forward's split: small leaves and chunks on waves
             if (a.n_wave > 0) {
                 const dim3 g((a.n_wave + kWaveBlock / 64 - 1) / (kWaveBlock / 64)), b(kWaveBlock);
                 if (fp32_points)
@@ -1764,8 +1764,8 @@ static void grad_launch(bool fp32_points, const LeafStage& a, const KConst& c, h
                     hipLaunchKernelGGL((k_leaf_grad2_wave<KID, double>), g, b, 0, s, a, make_kc64(c), make_kc64(c),
                                        scale);
                 TBEM_LAUNCH_CHECK();
-                if (a.n_parts > 0) {
-                    hipLaunchKernelGGL(k_leaf_grad_parts, dim3(a.n_parts), dim3(kWaveLeafMax), 0, s, a, scale);
+                if (a.n_wave_parts > 0) {
+                    hipLaunchKernelGGL(k_leaf_grad_parts, dim3(a.n_wave_parts), dim3(kWaveLeafMax), 0, s, a, scale);
                     TBEM_LAUNCH_CHECK();
                 }
             }
@@ -1773,9 +1773,7 @@ static void grad_launch(bool fp32_points, const LeafStage& a, const KConst& c, h
             LeafStage bl = a;
             bl.order = a.block_pos;
             bl.n_order = a.n_block;
-            bl.wave_items = nullptr;
-            bl.block_pos = nullptr;
-            bl.n_wave = bl.n_parts = 0;
+            bl.split = 0;
             grad_launch<KID, T>(fp32_points, bl, c, s);
             return;
         }
@@ -1810,6 +1808,16 @@ void launch_surf_stage(int kid, bool src_surf, bool add, bool adj, const SurfSta
                        hipStream_t s) {
     using T = double;
     TBEM_KID_SWITCH(kid, surf_launch, src_surf, add, adj, a, kc, s);
+}
+
+int leaf_stage_tile(int kid, bool fp32) {
+    switch (kid) {
+#define TBEM_TILE(K) case K: return fp32 ? leaf_block<K, float>() : leaf_block<K, double>();
+        TBEM_TILE(K_LS) TBEM_TILE(K_LD) TBEM_TILE(K_LH) TBEM_TILE(K_EU) TBEM_TILE(K_ET) TBEM_TILE(K_EA)
+        TBEM_TILE(K_EH) TBEM_TILE(K_ID1) TBEM_TILE(K_ID3)
+#undef TBEM_TILE
+    }
+    throw Error(TBEM_E_INVALID, "unknown kernel id");
 }
 
 template <class T>
