@@ -143,6 +143,36 @@ __global__ void k_m2l_swizzle(int n, int mt, int kt, int trans, const double* __
     }
 }
 
+// Hands the entries 4q + i (i < 4) of a column of n values to put(q, i, v), for the
+// k-steps q = q0, q0 + dq, ... below kt; zeros past n, and everywhere for a null column.
+// Four consecutive entries per load (16 or 2 x 16 bytes; the columns are aligned to one
+// entry only, which these loads allow) and four loads in flight: reading an entry at a
+// time, each wave waited for the cache once per pass over its few rows. M2L stage before
+// and after: 4M points, Laplace, order 75, FP32 25.3 -> 20.9 ms; 1M points, clusters, order
+// 75, FP64 19.6 -> 17.9; 1M points, hypersingular, order 50, FP64 21.8 -> 20.9 (24.1 -> 21.8
+// by the 128-byte stores of k_m2l_mfma64).
+template <class T, class F>
+__device__ __forceinline__ void stage_quads(const T* col, int n, int kt, int q0, int dq, F&& put) {
+    typedef T quad __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    const int full = n / 4;  // the k-steps wholly below n
+    for (int q = q0; q < kt; q += 4 * dq) {
+        quad v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int k = q + u * dq;
+            v[u] = quad{0, 0, 0, 0};
+            if (col && k < full) v[u] = *(const quad*)(col + 4 * k);
+            else if (col && k < kt)
+                for (int i = 0; i < 3; i++)  // the last, partial k-step
+                    if (4 * k + i < n) v[u][i] = col[4 * k + i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (q + u * dq < kt)
+                for (int i = 0; i < 4; i++) put(q + u * dq, i, v[u][i]);
+    }
+}
+
 // One row tile (16 rows of M_c) times the NCT staged column tiles. A comes from
 // global memory (L2-resident), loaded kPre k-steps ahead of its use so that the
 // loads' latency overlaps kPre * NCT MFMAs. The last block of a row tile already
@@ -190,11 +220,11 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma(int n, int mt, int kt, int
     const int cls = uni(ucls[u]), off = uni(uoff[u]), cnt = uni(ucnt[u]);
     if (cnt == 0) return;  // padding unit: uniform exit before any barrier
     const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
-    const int kpad = kt * 4;
-    // stage: lane = column (pair), waves stride over k
+    // stage: lane = column (pair), waves stride over the k-steps
     const float* col = lane < cnt ? chk + (size_t)pair_src[colpair[off + lane]] * n : nullptr;
-    for (int kk = wave; kk < kpad; kk += NW)
-        Bs[kk * 64 + (lane ^ ((kk & 3) << 4))] = (col && kk < n) ? col[kk] : 0.f;
+    stage_quads<float>(col, n, kt, wave, NW, [&](int q, int i, float v) {
+        Bs[(4 * q + i) * 64 + (lane ^ (i << 4))] = v;
+    });
     __syncthreads();
     // B operand of column tile ct at k-step ks: row ks*4 + lq, column ct*16 + lr,
     // stored at ((ct ^ lq) * 16 + lr)
@@ -313,7 +343,7 @@ __device__ __forceinline__ void m2l_row_tile64(const double* __restrict__ A, con
             const double* bk = b + (k0 + i) * 4 * kUnitCols64;
 #pragma unroll
             for (int ct = 0; ct < NCT; ct++)
-                acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(cur[i], bk[16 * ct], acc[ct], 0, 0, 0);
+                acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(bk[16 * ct], cur[i], acc[ct], 0, 0, 0);
         }
         for (int i = 0; i < kPre; i++) cur[i] = nxt[i];
     }
@@ -322,8 +352,9 @@ __device__ __forceinline__ void m2l_row_tile64(const double* __restrict__ A, con
 // One workgroup of NW waves per unit: the unit's source coefficients staged in LDS
 // (row k, column = pair, kpad x 32 doubles), then wave w takes row tiles w, w + NW, ...
 // The FP64 MFMA leaves D[4*r + lq][lr] in register r of lane (lq, lr) (not the f32
-// 16x16x4 order), so Y[pair][rt*16 + 4*r + lq] = D[4*r + lq][lr] of column tile ct
-// (pair ct*16 + lr): the four lanes lq of a pair write 32 contiguous bytes per r.
+// 16x16x4 order). The staged columns are its A operand and the operator's rows its B
+// operand (the same lane layout), so Y[pair ct*16 + 4*r + lq][rt*16 + lr] = D[4*r + lq][lr]
+// and the 16 lanes lr write 128 contiguous bytes of a pair.
 template <int NW, int kPre>
 __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, int ystride,
                                                      const double* __restrict__ S, const int* __restrict__ ucls,
@@ -335,13 +366,14 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
     const int cls = uni(ucls[u]), off = uni(uoff[u]), cnt = uni(ucnt[u]);
     if (cnt == 0) return;  // padding unit: uniform exit before any barrier
     const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
-    const int kpad = kt * 4;
     // stage: lane % kUnitCols64 = column (pair); the rest of the lane index and the
-    // waves stride over k
-    constexpr int RPW = 64 / kUnitCols64;  // k rows per wave and pass
+    // waves stride over the k-steps
+    constexpr int RPW = 64 / kUnitCols64;  // k-steps per wave and pass
     const int c = lane % kUnitCols64, h = lane / kUnitCols64;
     const double* col = c < cnt ? x + (size_t)pair_src[colpair[off + c]] * n : nullptr;
-    for (int kk = RPW * wave + h; kk < kpad; kk += RPW * NW) Bd[kk * kUnitCols64 + c] = (col && kk < n) ? col[kk] : 0.0;
+    stage_quads<double>(col, n, kt, RPW * wave + h, RPW * NW, [&](int q, int i, double v) {
+        Bd[(4 * q + i) * kUnitCols64 + c] = v;
+    });
     __syncthreads();
     // B operand of column tile ct at k-step ks: row ks*4 + lq, column ct*16 + lr
     const int lr = lane % 16, lq = lane / 16;
@@ -349,6 +381,14 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
     constexpr int MAXCT = kUnitCols64 / 16;
     const int nct = (cnt + 15) / 16;  // 1 .. MAXCT (uniform)
     const double* Acls = S + (size_t)cls * mt * kt * 64 + lane;
+    int yp[MAXCT][4];  // the lane's pairs' rows of Y (-1: none)
+#pragma unroll
+    for (int ct = 0; ct < MAXCT; ct++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int nn = ct * 16 + 4 * r + lq;
+            yp[ct][r] = nn < cnt ? colpair[off + nn] - ybase : -1;
+        }
     double cur[kPre];
     for (int i = 0; i < kPre; i++) cur[i] = (wave < mt && i < kt) ? Acls[((size_t)wave * kt + i) * 64] : 0.0;
     for (int rt = wave; rt < mt; rt += NW) {
@@ -359,13 +399,11 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
         else if (MAXCT == 2 || nct == 2) m2l_row_tile64<(MAXCT < 2 ? MAXCT : 2), kPre>(A, An, b, kt, acc, cur);
         else if (nct == 3) m2l_row_tile64<(MAXCT < 3 ? MAXCT : 3), kPre>(A, An, b, kt, acc, cur);
         else m2l_row_tile64<MAXCT, kPre>(A, An, b, kt, acc, cur);
-        for (int ct = 0; ct < nct; ct++) {
-            const int nn = ct * 16 + lr;
-            if (nn < cnt) {
-                double* y = Y + (size_t)(colpair[off + nn] - ybase) * ystride + rt * 16 + lq;
-                for (int r = 0; r < 4; r++) y[4 * r] = acc[ct][r];
-            }
-        }
+#pragma unroll
+        for (int ct = 0; ct < MAXCT; ct++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (yp[ct][r] >= 0) Y[(size_t)yp[ct][r] * ystride + rt * 16 + lr] = acc[ct][r];
     }
 }
 
