@@ -1140,7 +1140,7 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     P->p2m.upload(self_list(ST, ST.leaves), s);
     P->t_p2m = make_cell_tiles(ST.leaves, ST, s);
     // M2M and L2L on class operators: the cells of one tree always lie on one grid
-    const bool tr_classes = d->translations == TBEM_TRANSLATIONS_AUTO && m2l_fp64_size_ok(P->blk);
+    const bool tr_classes = d->translations == TBEM_TRANSLATIONS_AUTO && m2l_mfma_size_ok(P->blk) && m2l_fp64_size_ok(P->blk);
     auto note_y = [&](const M2lMfma& M) {
         if (M.enabled) P->tr_y = std::max(P->tr_y, (size_t)M.y_pairs * M.ystride);
     };
@@ -1162,10 +1162,12 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     P->t_m2l = make_cell_tiles(m2l_h.items, OT, s);
     P->m2l_no_cutoff = m2l_clear_of_cutoff(m2l_h, OT, ST, P->surf);
     clk.mark("lists");
-    // FP64: class operators where the classes exist (the builder also requires the
-    // operators to fit an eighth of the device memory)
-    const bool fp64_classes = P->precision == TBEM_FP64 && d->translations == TBEM_TRANSLATIONS_AUTO &&
-                              P->tree_layout != kTreesOwnBoxes && m2l_fp64_size_ok(P->blk);
+    // FP64, and mixed precision below the FP32 operators' sizes: class operators where the
+    // classes exist and pay (the builder also requires the operators to fit an eighth of
+    // the device memory)
+    const bool fp64_classes = (P->precision == TBEM_FP64 || !m2l_mfma_size_ok(P->blk)) &&
+                              d->translations == TBEM_TRANSLATIONS_AUTO && P->tree_layout != kTreesOwnBoxes &&
+                              m2l_fp64_classes_pay(P->kid, P->n_e, m2l_h.cell.size());
     if (P->precision == TBEM_MIXED || fp64_classes)
         build_m2l_mfma(P->m2l_mfma, P->kid, P->kc, OT, ST, P->dot, P->dst, P->tree_layout != kTreesOwnBoxes,
                        fp64_classes, d->m2l_output_budget ? d->m2l_output_budget : kM2lOutputBudget, m2l_h, P->m2l,
@@ -1465,7 +1467,7 @@ static void forward_T(const FmmPlan& P, Work& W, const double* x, double* y, hip
         launch_fill(y, (size_t)R * No, 0.0, s);
         return;
     }
-    const bool mfma = std::is_same<T, float>::value && P.m2l_mfma.enabled;
+    const bool mfma = std::is_same<T, float>::value && P.m2l_mfma.enabled && !P.m2l_mfma.fp64;
     W.split_last = W.overlap;
     if (W.overlap) {
         // P2P on the side stream once the densities are gathered, beside the far field
@@ -1530,7 +1532,7 @@ static void obs_grad(const FmmPlan& P, Work& W, const double* x, const double* g
     if (reuse_token != 0 && reuse_token == W.far_token) {
         launch_gather_dens(x, P.sp.perm.p, P.sp.w.p, Ns, R, W.dens.p, s);
     } else {
-        farfield(P, W, x, s, P.precision == TBEM_MIXED && P.m2l_mfma.enabled);
+        farfield(P, W, x, s, P.precision == TBEM_MIXED && P.m2l_mfma.enabled && !P.m2l_mfma.fp64);
         W.far_token = ++W.next_token;
     }
     if (W.gsort.n < (size_t)R * No) W.gsort.alloc((size_t)R * No);
@@ -1560,7 +1562,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
     if (W.lbar.n < nco) { W.lbar.alloc(nco); W.cbar.alloc(nco); }
     if (W.mbar.n < ncs) { W.mbar.alloc(ncs); W.ebar.alloc(ncs); }
     if (W.dens.n < (size_t)R * Ns) W.dens.alloc((size_t)R * Ns);
-    const bool mfma = std::is_same<T, float>::value && P.m2l_mfma.enabled;
+    const bool mfma = std::is_same<T, float>::value && P.m2l_mfma.enabled && !P.m2l_mfma.fp64;
     const FmmPlan::AdjLists& A = P.adjoint_lists(s);
     if (mfma && W.e2.n < ncs) { W.e2.alloc(ncs); W.m2l_w.alloc(nco); }
     launch_gather_dens(g, P.op.perm.p, nullptr, No, R, W.gsort.p, s);

@@ -49,6 +49,8 @@ struct M2lMfma {
 bool m2l_mfma_size_ok(int blk);
 // The same for the FP64 operators (32 staged FP64 columns per unit).
 bool m2l_fp64_size_ok(int blk);
+// Whether the FP64 class operators serve this M2L better than the surfaces' kernel.
+bool m2l_fp64_classes_pay(int kid, int n_e, size_t n_pairs);
 // fp64: build the FP64 path's operators (see above) instead of the mixed path's.
 // y_budget: bytes the per-pair output may take; the pairs are sliced to fit.
 // t_surf, s_surf: the target's check and the source's equivalent surface (unit

@@ -601,7 +601,7 @@ static size_t staged_bytes(int n, bool fp64) {
 }
 
 static bool size_ok(int n, bool fp64) {
-    if (n > kMaxBlk || n < kMinBlk) return false;
+    if (n > kMaxBlk || n < (fp64 ? 1 : kMinBlk)) return false;
     // the staged columns must fit one workgroup's LDS on this device
     int dev = 0, max_shm = 0;
     TBEM_HIP(hipGetDevice(&dev));
@@ -611,6 +611,26 @@ static bool size_ok(int n, bool fp64) {
 
 bool m2l_mfma_size_ok(int n) { return size_ok(n, false); }
 bool m2l_fp64_size_ok(int n) { return size_ok(n, true); }
+
+// Which of the FP64 M2L's two forms is the faster, from the time per pair that each took
+// (MI355X, 1.1M to 5.6M pairs): the surfaces' n_e^2 kernel evaluations about n_e^2 (0.5 +
+// 0.043 F) ps, F flops per evaluation (Laplace single layer, order 35: 1450 ps; elastic
+// displacement, order 6: 85; hypersingular, order 10: 460), the class operators, bound by
+// their per-pair output's traffic, about 6.5 ps per output row (order 35, 48 rows: 295 ps;
+// 32 rows: 205). A quarter is left for the second launch and the classes' plan, and fewer
+// than kMinClassPairs pairs gain too little to build them for. From kMinBlk rows on the
+// classes serve every size. M2L stage, surfaces -> classes: 60k points in a cube, order 20
+// 1032 -> 452 us, order 35 3214 -> 654, order 47 6141 -> 688; 500k in clusters, order 35
+// 5964 -> 1671; hypersingular, 100k points, order 10 506 -> 377 (order 6 182 -> 245, left).
+constexpr size_t kMinClassPairs = 50000;
+bool m2l_fp64_classes_pay(int kid, int n_e, size_t n_pairs) {
+    const int n = kernel_dim(kid) * n_e;
+    if (!m2l_fp64_size_ok(n)) return false;
+    if (n >= kMinBlk) return true;
+    static const double flops[9] = {11, 18, 1, 28, 45, 45, 68, 1, 3};
+    const double surf = (double)n_e * n_e * (0.5 + 0.043 * flops[kid]), cls = 6.5 * 16 * div_up((size_t)n, 16);
+    return n_pairs >= kMinClassPairs && surf >= 1.25 * cls;
+}
 
 void build_m2l_mfma(M2lMfma& M, int kid, const KConst& kc, const HostTree& ot, const HostTree& st,
                     const DevTree& dot, const DevTree& dst, bool same_grid, bool fp64, size_t y_budget,
@@ -911,6 +931,15 @@ static SliceUnits slice_units(const M2lMfma& M, int q) {
     return {M.slice_units[q + 1] - u0, M.unit_class.p + u0, M.unit_off.p + u0, M.unit_cnt.p + u0};
 }
 
+// Waves per workgroup of the narrow kernels: of 3, 4 and 5, the one that leaves the fewest
+// waves without a row tile in the last round (the larger of two equals).
+static int narrow_waves(int mt) {
+    int best = 4;
+    for (int w : {5, 3})
+        if (div_up(mt, w) * w < div_up(mt, best) * best) best = w;
+    return best;
+}
+
 // Y (slice q) = M_c * chk_up[src(p)] (transpose: M_c^T * chk_up[tgt(p)]), FP32 MFMA
 static void mfma32_slice(const M2lMfma& M, int q, const int* pair_src, const float* chk_up, float* Y,
                          bool transpose, hipStream_t s) {
@@ -925,6 +954,9 @@ static void mfma32_slice(const M2lMfma& M, int q, const int* pair_src, const flo
     if (wide)
         hipLaunchKernelGGL((k_m2l_mfma<8, kPreWide>), dim3(U.n), dim3(512), shm, s, M.blk, M.mt, M.kt, M.ystride, S,
                            U.ucls, U.uoff, U.ucnt, M.colpair.p, src, yb, chk_up, Y);
+    else if (narrow_waves(M.mt) == 5)
+        hipLaunchKernelGGL((k_m2l_mfma<5, kPreNarrow>), dim3(U.n), dim3(320), shm, s, M.blk, M.mt, M.kt, M.ystride,
+                           S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, yb, chk_up, Y);
     else
         hipLaunchKernelGGL((k_m2l_mfma<4, kPreNarrow>), dim3(U.n), dim3(256), shm, s, M.blk, M.mt, M.kt, M.ystride,
                            S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, yb, chk_up, Y);
@@ -942,6 +974,12 @@ static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const dou
     if (3 * shm > kLdsPerCu)
         hipLaunchKernelGGL((k_m2l_mfma64<kWaves64, kPre64>), dim3(U.n), dim3(kWaves64 * 64), shm, s, M.blk, M.mt,
                            M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
+    else if (narrow_waves(M.mt) == 5)
+        hipLaunchKernelGGL((k_m2l_mfma64<5, kPre64Narrow>), dim3(U.n), dim3(320), shm, s, M.blk, M.mt, M.kt,
+                           M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
+    else if (narrow_waves(M.mt) == 3)
+        hipLaunchKernelGGL((k_m2l_mfma64<3, kPre64Narrow>), dim3(U.n), dim3(192), shm, s, M.blk, M.mt, M.kt,
+                           M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
     else
         hipLaunchKernelGGL((k_m2l_mfma64<kWaves64Narrow, kPre64Narrow>), dim3(U.n), dim3(kWaves64Narrow * 64), shm,
                            s, M.blk, M.mt, M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src,
