@@ -178,6 +178,8 @@ class YLease {
     std::unique_lock<std::mutex> lk_;
 };
 
+constexpr double kOverlapPairs = 1.2e9;  // Work::overlap
+
 struct Work {
     hipStream_t stream = nullptr;
     DevBuf<double> dens, mult, locals, out_sorted, xbuf, ybuf;
@@ -198,8 +200,11 @@ struct Work {
     // stream beside the far field (P2M ... L2L: MFMA and small launches beside the
     // P2P's VALU work), joined before the surface sources (M2P, L2P) are added. On by
     // default where the far field is large (R * n_e >= 48: 2M points, order 100, FP64
-    // 30.0 -> 27.9 ms); at low order the extra surface launch costs more than the
-    // overlap gains (1M points, order 6: 4.8 -> 5.1 ms).
+    // 30.0 -> 27.9 ms), and at low order where the point pairs are few, so that the far
+    // field's chain of short launches takes a fair part of the pass (order 6, off -> on:
+    // 20k points 252 -> 237 us, 100k 652 -> 530, 250k (4e8 pairs) 1049 -> 863, 500k (1.1e9)
+    // 1672 -> 1620; 1M (1.8e9) 2735 -> 2775: the second surface launch then costs what
+    // the overlap gains).
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     bool overlap = true;
@@ -214,7 +219,7 @@ struct Work {
         TBEM_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         TBEM_HIP(hipEventRecord(done, stream));
         TBEM_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-        overlap = P.blk >= 48;
+        overlap = P.blk >= 48 || P.p2p_pairs <= kOverlapPairs;
         TBEM_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
         TBEM_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
         dens.alloc(P.R * P.n_src);
