@@ -1180,6 +1180,7 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     clk.mark("m2l_mfma");
     TBEM_HIP(hipEventCreateWithFlags(&P->y_done, hipEventDisableTiming));
     TBEM_HIP(hipEventRecord(P->y_done, s));
+    if (!P->m2l_mfma.enabled) P->m2l.order_by_work(m2l_h.ptr, s);
     if (P->m2l_mfma.enabled) {
         const size_t ny = (size_t)P->m2l_mfma.y_pairs * P->m2l_mfma.ystride;
         if (P->m2l_mfma.fp64) P->m2l_y64.alloc(ny);
@@ -1238,7 +1239,11 @@ const FmmPlan::AdjLists& FmmPlan::adjoint_lists(hipStream_t s) const {
     A->l2p.upload(self_list(OT, OT.leaves), s);
     A->l2l.resize(OT.n_levels);
     for (int L = 0; L + 1 < OT.n_levels; L++) A->l2l[L].upload(children_list(OT, L), s);
-    A->m2l.upload(list_from_pairs(cells_with(tl.m2l, 1, ST.n_cells), ST.n_cells, tl.m2l, 1, nullptr), s);
+    {
+        const HostList l = list_from_pairs(cells_with(tl.m2l, 1, ST.n_cells), ST.n_cells, tl.m2l, 1, nullptr);
+        A->m2l.upload(l, s);
+        if (!m2l_mfma.enabled) A->m2l.order_by_work(l.ptr, s);
+    }
     A->m2p.upload(list_from_pairs(cells_with(tl.m2p, 1, ST.n_cells), ST.n_cells, tl.m2p, 1, &OT), s);
     A->m2m.resize(ST.n_levels);
     for (int L = 1; L < ST.n_levels; L++) A->m2m[L].upload(parent_list(ST, L), s);
@@ -1308,6 +1313,7 @@ static void set_list(SurfStage& a, const DevList& l) {
     a.rbeg = l.rbeg.p;
     a.rcnt = l.rcnt.p;
     a.rpre = l.rpre.p;
+    a.order = l.by_work.p;
 }
 
 // gather, upward pass, M2L/P2L and L2L: everything the leaf stage consumes. FP64,

@@ -249,7 +249,16 @@ inline KC<D3> make_kcd(const KConst& c) {
 // d = src - obs, r2 = |d|^2; no / ns are the obs and src normals.
 // CUT = false leaves out the r2 < 1e-12 test, for callers that have shown that no
 // pair they pass is that close (the result is then the same bit for bit).
-template <int KID, bool ADJ, class T, bool FAST = false, bool CUT = true>
+// TWO: a lone target, rounded as the two-target loops round theirs (there the products of
+// source values alone, u2 v and the transpose's t2 n.v, are shared by both targets and so
+// rounded by themselves, where here they would be fused into their sums).
+template <class T>
+__device__ __forceinline__ T mul_rounded(T a, T b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
+template <int KID, bool ADJ, class T, bool FAST = false, bool CUT = true, bool TWO = false>
 __device__ __forceinline__ void kop(T dx, T dy, T dz, T r2, const T* no, const T* ns, const T* v,
                                     T* acc, const KC<T>& k) {
     if (KID == K_LH) return;
@@ -280,6 +289,12 @@ __device__ __forceinline__ void kop(T dx, T dy, T dz, T r2, const T* no, const T
     const T dv = dx * v[0] + dy * v[1] + dz * v[2];
     if (KID == K_EU) {  // symmetric: fwd == adj
         const T t = dv * ri2;
+        if constexpr (TWO) {
+            acc[0] += ri * (mul_rounded(k.u2, v[0]) + dx * t);
+            acc[1] += ri * (mul_rounded(k.u2, v[1]) + dy * t);
+            acc[2] += ri * (mul_rounded(k.u2, v[2]) + dz * t);
+            return;
+        }
         acc[0] += ri * (k.u2 * v[0] + dx * t);
         acc[1] += ri * (k.u2 * v[1] + dy * t);
         acc[2] += ri * (k.u2 * v[2] + dz * t);
@@ -329,7 +344,8 @@ __device__ __forceinline__ void kop(T dx, T dy, T dz, T r2, const T* no, const T
         } else {
             // d3 (t2 nov r + nu (m drv + v drdm) - 5 drv r drdm)
             //   + t2 (3 n drv drdm + v nn + nsv m) + h3 (nsv r drdm + nn drv r) + h2 n nov
-            ca = d3 * (k.t2 * nov - T(5) * pd) + k.h3 * (nsv * drdm + nn * drv);
+            const T tv = TWO ? mul_rounded(k.t2, nov) : k.t2 * nov;
+            ca = d3 * (tv - T(5) * pd) + k.h3 * (nsv * drdm + nn * drv);
             cm = d3 * k.nu * drv + k.t2 * nsv;
             cv = d3 * k.nu * drdm + k.t2 * nn;
             cn = T(3) * k.t2 * pd + k.h2 * nov;

@@ -129,8 +129,10 @@ struct HostList {
 struct DevList {
     int n_items = 0;
     DevBuf<int> items, ptr, cell, rbeg, rcnt, rpre;
+    DevBuf<int> by_work; // item indices, the most cells first (order_by_work; empty: as listed)
     DevBuf<int> rclose;  // point-range lists of the point-target stage: launch_range_close
     void upload(const HostList& l, hipStream_t s);
+    void order_by_work(const std::vector<int>& host_ptr, hipStream_t s);
 };
 
 // Cells grouped into tiles of at most 64 cells of one level (make_cell_tiles).

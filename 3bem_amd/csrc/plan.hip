@@ -82,6 +82,17 @@ void DevPoints::upload(const HostTree& t, const double* locs, const double* norm
     TBEM_HIP(hipStreamSynchronize(s));
 }
 
+// The launch order of a stage that runs one workgroup per item: longest first, so that
+// none of them is left running alone at the end.
+void DevList::order_by_work(const std::vector<int>& p, hipStream_t s) {
+    if (p.size() < 2) return;
+    std::vector<int> o(p.size() - 1);
+    for (size_t k = 0; k < o.size(); k++) o[k] = (int)k;
+    std::stable_sort(o.begin(), o.end(), [&](int a, int b) { return p[a + 1] - p[a] > p[b + 1] - p[b]; });
+    by_work.upload(o, s);
+    TBEM_HIP(hipStreamSynchronize(s));  // o goes out of scope
+}
+
 void DevList::upload(const HostList& l, hipStream_t s) {
     n_items = (int)l.items.size();
     items.upload(l.items, s);

@@ -105,6 +105,7 @@ struct SurfStage {
     const double* unit;     // unit sphere = surface normals
     int n_e, blk;
     double* out;            // blk per cell of tt: the raw check potentials (= or += with add)
+    const int* order;       // the items' launch order (null: as listed), the most work first
     int no_cutoff;          // surface sources: every pair is known to lie beyond the r2 < 1e-12
                             // cutoff, so the kernels leave the test out (same result)
 };

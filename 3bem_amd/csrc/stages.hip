@@ -328,7 +328,7 @@ __device__ inline void stream_surfaces(Tile<double, R, NRM, NB>& tl, int e0, int
     int base = 0;
     auto fetch = [&](int b) {
         const int v = b + tid;
-        if (v < total) {
+        if (tid < NB && v < total) {
             const int k = v / n_e;
             load_surf(r, cell[e0 + k], v - k * n_e, st, surf, unit, coeff, n_e, blk);
         }
@@ -350,7 +350,8 @@ __device__ inline void stream_surfaces(Tile<double, R, NRM, NB>& tl, int e0, int
 // ---------------------------------------------------------------------- pair loop
 // One source j of the tile on one target (FP64 coordinates tx, ty, tz): the
 // displacement is formed in FP64, then the kernel runs in T.
-template <int KID, bool ADJ, bool FAST = false, bool CUT = true, class T, class VT, int R, bool NRM, int NB>
+template <int KID, bool ADJ, bool FAST = false, bool CUT = true, bool TWO = false, class T, class VT, int R, bool NRM,
+          int NB>
 __device__ __forceinline__ void pair(const Tile<VT, R, NRM, NB>& tl, int j, double tx, double ty, double tz,
                                      const T* tn, T* acc, const KC<T>& kc) {
     const T sn[3] = {NRM ? T(tl.nx[j]) : T(0), NRM ? T(tl.ny[j]) : T(0), NRM ? T(tl.nz[j]) : T(0)};
@@ -359,11 +360,11 @@ __device__ __forceinline__ void pair(const Tile<VT, R, NRM, NB>& tl, int j, doub
     if (!ADJ) {
         const T dx = T(tl.x[j] - tx), dy = T(tl.y[j] - ty), dz = T(tl.z[j] - tz);
         const T r2 = dx * dx + dy * dy + dz * dz;
-        kop<KID, false, T, FAST, CUT>(dx, dy, dz, r2, tn, sn, v, acc, kc);
+        kop<KID, false, T, FAST, CUT, TWO>(dx, dy, dz, r2, tn, sn, v, acc, kc);
     } else {
         const T dx = T(tx - tl.x[j]), dy = T(ty - tl.y[j]), dz = T(tz - tl.z[j]);
         const T r2 = dx * dx + dy * dy + dz * dz;
-        kop<KID, true, T, FAST, CUT>(dx, dy, dz, r2, sn, tn, v, acc, kc);
+        kop<KID, true, T, FAST, CUT, TWO>(dx, dy, dz, r2, sn, tn, v, acc, kc);
     }
 }
 
@@ -377,7 +378,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     __shared__ StageSmem<double, R, NRM, NB, (DUAL ? 2 : 1) * R> sm;
     extern __shared__ double field[];  // R * n_e
-    const int item = blockIdx.x;
+    const int item = a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
     const int cell = uni(a.items[item]);
     const int lvl = uni(a.tt.level[cell]);
     const double rc = a.tt.level_r[lvl];
@@ -438,6 +439,62 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
     }
     double* o = a.out + (size_t)cell * a.blk;
     for (int row = tid; row < a.blk; row += NB) o[row] = add ? o[row] + field[row] : field[row];
+}
+
+// The same stage for kSurfBlock / 2 < n_e <= kSurfOneMax with one target per lane and a
+// workgroup as wide as its targets times the S slices k_surf_stage would use
+// (S = kSurfBlock / ceil(n_e / 2)), on the same kSurfBlock-source tiles, so that every
+// target's sums run in the same order and keep their bits. Bound: the serial chain of a
+// target's sources where cells are few, each source a dependent rsqrt and its FMAs; two
+// sources per step overlap theirs. Half the chain of the two-target form, and no wave left
+// with a few lanes (n_e = 151: 76 slots in two waves there, 151 in three here). Measured,
+// traction, order 150, 13,546 M2L pairs (one workgroup per cell, most pairs first): 4070 ->
+// 1943 us, transposed 2453 -> 1534; 2M points, order 100: P2M 366 -> 300 us.
+constexpr int kSurfOneMax = 256;
+
+template <int KID, bool SRC_SURF, bool ADJ, bool CUT = true>
+__global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double> kc, double scale, int S, int add) {
+    constexpr int NB = kSurfBlock;
+    constexpr int R = kernel_dim(KID);
+    constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
+    __shared__ union {
+        Tile<double, R, NRM, NB> st;
+        double red[R * kSurfOneMax];
+    } sm;
+    const int item = a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
+    const int cell = uni(a.items[item]);
+    const double rc = a.tt.level_r[uni(a.tt.level[cell])];
+    const int e0 = uni(a.ptr[item]), e1 = uni(a.ptr[item + 1]);
+    const int tid = threadIdx.x, n_e = a.n_e;
+    const int tg = tid % n_e, slice = tid / n_e;
+    const bool active = slice < S;
+    double p[3];
+    moved(rc, a.t_surf + 3 * tg, a.tt.cx[cell], a.tt.cy[cell], a.tt.cz[cell], p);
+    const double tn[3] = {a.unit[3 * tg], a.unit[3 * tg + 1], a.unit[3 * tg + 2]};
+    drain_loads();
+    double acc[R];
+    for (int q = 0; q < R; q++) acc[q] = 0.0;
+    auto compute = [&](int cnt) {
+        if (!active) return;
+#pragma unroll 2
+        for (int j = slice; j < cnt; j += S) pair<KID, ADJ, false, CUT, true>(sm.st, j, p[0], p[1], p[2], tn, acc, kc);
+    };
+    if (SRC_SURF)
+        stream_surfaces(sm.st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
+    else
+        stream_ranges(sm.st, e0, e1, a.rbeg, a.rcnt, a.sp, a.dens, a.n_src_pts, compute);
+    __syncthreads();
+    if (active)
+        for (int q = 0; q < R; q++) sm.red[(q * S + slice) * n_e + tg] = acc[q];
+    __syncthreads();
+    double* o = a.out + (size_t)cell * a.blk;
+    for (int row = tid; row < a.blk; row += blockDim.x) {
+        const int q = row / n_e, t = row - q * n_e;
+        double s = 0;
+        for (int k = 0; k < S; k++) s += sm.red[(q * S + k) * n_e + t];
+        s *= scale;
+        o[row] = add ? o[row] + s : s;
+    }
 }
 
 // -------------------------------------------------------------------- point targets
@@ -1667,6 +1724,25 @@ static void surf_launch(bool src_surf, bool add, bool adj, const SurfStage& a, c
     const double scale = (double)kop_scale<KID, double>(kc);
     const size_t shm = (size_t)kernel_dim(KID) * a.n_e * sizeof(double);
     dim3 g(a.n_items), b(kSurfBlock);
+    if (a.n_e > kSurfBlock / 2 && a.n_e <= kSurfOneMax) {
+        const int S = kSurfBlock / ((a.n_e + 1) / 2);
+        const dim3 w(div_up((size_t)a.n_e * S, 64) * 64);
+        const int ad = add ? 1 : 0;
+        if (src_surf && a.no_cutoff && !adj)
+            hipLaunchKernelGGL((k_surf_one<KID, true, false, false>), g, w, 0, s, a, kc, scale, S, ad);
+        else if (src_surf && a.no_cutoff)
+            hipLaunchKernelGGL((k_surf_one<KID, true, true, false>), g, w, 0, s, a, kc, scale, S, ad);
+        else if (src_surf && !adj)
+            hipLaunchKernelGGL((k_surf_one<KID, true, false>), g, w, 0, s, a, kc, scale, S, ad);
+        else if (src_surf)
+            hipLaunchKernelGGL((k_surf_one<KID, true, true>), g, w, 0, s, a, kc, scale, S, ad);
+        else if (!adj)
+            hipLaunchKernelGGL((k_surf_one<KID, false, false>), g, w, 0, s, a, kc, scale, S, ad);
+        else
+            hipLaunchKernelGGL((k_surf_one<KID, false, true>), g, w, 0, s, a, kc, scale, S, ad);
+        TBEM_LAUNCH_CHECK();
+        return;
+    }
     const int v = (src_surf && a.no_cutoff ? 8 : src_surf ? 4 : 0) + (adj ? 2 : 0) + (a.n_e > kSurfBlock / 2 ? 1 : 0);
     const int ad = add ? 1 : 0;
     switch (v) {
