@@ -389,12 +389,13 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
             const int nn = ct * 16 + 4 * r + lq;
             yp[ct][r] = nn < cnt ? colpair[off + nn] - ybase : -1;
         }
+    const int rt0 = blockIdx.y * NW + wave, step = gridDim.y * NW;
     double cur[kPre];
-    for (int i = 0; i < kPre; i++) cur[i] = (wave < mt && i < kt) ? Acls[((size_t)wave * kt + i) * 64] : 0.0;
-    for (int rt = wave; rt < mt; rt += NW) {
+    for (int i = 0; i < kPre; i++) cur[i] = (rt0 < mt && i < kt) ? Acls[((size_t)rt0 * kt + i) * 64] : 0.0;
+    for (int rt = rt0; rt < mt; rt += step) {
         f64x4 acc[MAXCT] = {};
         const double* A = Acls + (size_t)rt * kt * 64;
-        const double* An = rt + NW < mt ? A + (size_t)NW * kt * 64 : nullptr;
+        const double* An = rt + step < mt ? A + (size_t)step * kt * 64 : nullptr;
         if (nct == 1) m2l_row_tile64<1, kPre>(A, An, b, kt, acc, cur);
         else if (MAXCT == 2 || nct == 2) m2l_row_tile64<(MAXCT < 2 ? MAXCT : 2), kPre>(A, An, b, kt, acc, cur);
         else if (nct == 3) m2l_row_tile64<(MAXCT < 3 ? MAXCT : 3), kPre>(A, An, b, kt, acc, cur);
@@ -963,6 +964,13 @@ static void mfma32_slice(const M2lMfma& M, int q, const int* pair_src, const flo
     TBEM_LAUNCH_CHECK();
 }
 
+// A launch of few units (the M2M and L2L of the upper levels, the M2L of a small problem)
+// spreads each unit's row tiles over up to kUnitsFill / units workgroups, each staging the
+// unit's columns again: the rows' products are what a lone workgroup spends its time on.
+// M2M and L2L per launch, blk 453: 70 -> 23 us; blk 150: 38 -> 15 us (300,007 points), 25 ->
+// 12 us (9,102 points).
+constexpr int kUnitsFill = 1024;
+
 // Y (slice q) = K_c * x[src(p)] (transpose: K_c^T * x[tgt(p)]), FP64 MFMA
 static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const double* x, double* Y, bool transpose,
                          hipStream_t s) {
@@ -971,17 +979,19 @@ static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const dou
     const size_t shm = staged_bytes(M.blk, true);
     const double* S = transpose ? M.ST64.p : M.S64.p;
     const int* src = transpose ? M.pair_tgt.p : pair_src;
-    if (3 * shm > kLdsPerCu)
-        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64, kPre64>), dim3(U.n), dim3(kWaves64 * 64), shm, s, M.blk, M.mt,
+    const int nw = 3 * shm > kLdsPerCu ? kWaves64 : narrow_waves(M.mt);
+    const dim3 g(U.n, std::max(1, std::min(div_up(M.mt, nw), kUnitsFill / U.n)));
+    if (nw == kWaves64)
+        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64, kPre64>), g, dim3(kWaves64 * 64), shm, s, M.blk, M.mt,
                            M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
-    else if (narrow_waves(M.mt) == 5)
-        hipLaunchKernelGGL((k_m2l_mfma64<5, kPre64Narrow>), dim3(U.n), dim3(320), shm, s, M.blk, M.mt, M.kt,
+    else if (nw == 5)
+        hipLaunchKernelGGL((k_m2l_mfma64<5, kPre64Narrow>), g, dim3(320), shm, s, M.blk, M.mt, M.kt,
                            M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
-    else if (narrow_waves(M.mt) == 3)
-        hipLaunchKernelGGL((k_m2l_mfma64<3, kPre64Narrow>), dim3(U.n), dim3(192), shm, s, M.blk, M.mt, M.kt,
+    else if (nw == 3)
+        hipLaunchKernelGGL((k_m2l_mfma64<3, kPre64Narrow>), g, dim3(192), shm, s, M.blk, M.mt, M.kt,
                            M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
     else
-        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64Narrow, kPre64Narrow>), dim3(U.n), dim3(kWaves64Narrow * 64), shm,
+        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64Narrow, kPre64Narrow>), g, dim3(kWaves64Narrow * 64), shm,
                            s, M.blk, M.mt, M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src,
                            M.slice_pairs[q], x, Y);
     TBEM_LAUNCH_CHECK();
