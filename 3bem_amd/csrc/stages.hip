@@ -445,11 +445,11 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
 // workgroup as wide as its targets times the S slices k_surf_stage would use
 // (S = kSurfBlock / ceil(n_e / 2)), on the same kSurfBlock-source tiles, so that every
 // target's sums run in the same order and keep their bits. Bound: the serial chain of a
-// target's sources where cells are few, each source a dependent rsqrt and its FMAs; two
+// target's sources where cells are few, each source a dependent rsqrt and its FMAs; four
 // sources per step overlap theirs. Half the chain of the two-target form, and no wave left
 // with a few lanes (n_e = 151: 76 slots in two waves there, 151 in three here). Measured,
 // traction, order 150, 13,546 M2L pairs (one workgroup per cell, most pairs first): 4070 ->
-// 1943 us, transposed 2453 -> 1534; 2M points, order 100: P2M 366 -> 300 us.
+// 1457 us (1943 one source per step), transposed 2453 -> 1297 (1534).
 constexpr int kSurfOneMax = 256;
 
 template <int KID, bool SRC_SURF, bool ADJ, bool CUT = true>
@@ -476,8 +476,14 @@ __global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double
     for (int q = 0; q < R; q++) acc[q] = 0.0;
     auto compute = [&](int cnt) {
         if (!active) return;
-#pragma unroll 2
-        for (int j = slice; j < cnt; j += S) pair<KID, ADJ, false, CUT, true>(sm.st, j, p[0], p[1], p[2], tn, acc, kc);
+        int j = slice;
+        for (; j + 3 * S < cnt; j += 4 * S) {
+            pair<KID, ADJ, false, CUT, true>(sm.st, j, p[0], p[1], p[2], tn, acc, kc);
+            pair<KID, ADJ, false, CUT, true>(sm.st, j + S, p[0], p[1], p[2], tn, acc, kc);
+            pair<KID, ADJ, false, CUT, true>(sm.st, j + 2 * S, p[0], p[1], p[2], tn, acc, kc);
+            pair<KID, ADJ, false, CUT, true>(sm.st, j + 3 * S, p[0], p[1], p[2], tn, acc, kc);
+        }
+        for (; j < cnt; j += S) pair<KID, ADJ, false, CUT, true>(sm.st, j, p[0], p[1], p[2], tn, acc, kc);
     };
     if (SRC_SURF)
         stream_surfaces(sm.st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
