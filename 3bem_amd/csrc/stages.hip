@@ -43,12 +43,18 @@
 
 namespace tbem {
 
-// SoA source tile: FP64 coordinates, normals and densities in VT.
+// SoA source tile: FP64 coordinates, normals and densities in VT; sv: normal . density
+// (FP64 tiles of three components, kop_pt).
+template <class VT, int R, bool NRM>
+constexpr bool tile_has_sv() {
+    return NRM && R == 3 && std::is_same<VT, double>::value;
+}
 template <class VT, int R, bool NRM, int NB>
 struct Tile {
     double x[NB], y[NB], z[NB];
     VT nx[NRM ? NB : 1], ny[NRM ? NB : 1], nz[NRM ? NB : 1];
     VT d[R][NB];
+    VT sv[tile_has_sv<VT, R, NRM>() ? NB : 1];
 };
 
 // LDS of a stage kernel: the point tile (values in PT), the surface tile (FP64),
@@ -182,6 +188,7 @@ __device__ inline void store_tile(Tile<VT, R, NRM, NB>& tl, int slot, const SrcR
     tl.z[slot] = r.z;
     if (NRM) { tl.nx[slot] = VT(r.nx); tl.ny[slot] = VT(r.ny); tl.nz[slot] = VT(r.nz); }
     for (int q = 0; q < R; q++) tl.d[q][slot] = VT(r.d[q]);
+    if constexpr (tile_has_sv<VT, R, NRM>()) tl.sv[slot] = r.nx * r.d[0] + r.ny * r.d[1] + r.nz * r.d[2];
 }
 
 // Streams the points of ranges e0..e1 (sorted points [rbeg[e], rbeg[e]+rcnt[e]))
@@ -366,6 +373,35 @@ __device__ __forceinline__ void pair(const Tile<VT, R, NRM, NB>& tl, int j, doub
         const T r2 = dx * dx + dy * dy + dz * dz;
         kop<KID, true, T, FAST, CUT, TWO>(dx, dy, dz, r2, sn, tn, v, acc, kc);
     }
+}
+
+// The leaf kernels' accumulator slots per target, and one point source on one target: the
+// regrouped FP64 form where the kernel has it.
+template <int KID, class T, bool ADJ>
+constexpr bool uses_pt() {
+    return has_pt(KID) && std::is_same<T, double>::value;
+}
+template <int KID, class T, bool ADJ>
+constexpr int leaf_slots() {
+    return uses_pt<KID, T, ADJ>() ? pt_slots<KID, ADJ>() : kernel_dim(KID);
+}
+template <int KID, bool ADJ, bool FAST, bool CUT, class T, class VT, int R, bool NRM, int NB>
+__device__ __forceinline__ void point_pair(const Tile<VT, R, NRM, NB>& tl, int j, double tx, double ty, double tz,
+                                           const T* tn, T* acc, const KC<T>& kc) {
+    if constexpr (uses_pt<KID, T, ADJ>()) {
+        const double sn[3] = {tl.nx[j], tl.ny[j], tl.nz[j]}, v[3] = {tl.d[0][j], tl.d[1][j], tl.d[2][j]};
+        // (d is the kernel's source minus its observation point)
+        kop_pt<KID, ADJ, FAST, CUT>(ADJ ? tx - tl.x[j] : tl.x[j] - tx, ADJ ? ty - tl.y[j] : tl.y[j] - ty,
+                                    ADJ ? tz - tl.z[j] : tl.z[j] - tz, tn, sn, v, tl.sv[j], acc, kc);
+    } else {
+        pair<KID, ADJ, FAST, CUT>(tl, j, tx, ty, tz, tn, acc, kc);
+    }
+}
+// A target's sum of component q, with the slot along its normal applied.
+template <int KID, class T, bool ADJ, class A>
+__device__ __forceinline__ double leaf_value(const A& acc, int q, const double* tn) {
+    if constexpr (leaf_slots<KID, T, ADJ>() > kernel_dim(KID)) return acc.value(q) + acc.value(3) * tn[q];
+    else return acc.value(q);
 }
 
 // ------------------------------------------------------------------ surface targets
@@ -558,7 +594,7 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
         const T an[3] = {T(an64[0]), T(an64[1]), T(an64[2])};
         const T bn[3] = {T(bn64[0]), T(bn64[1]), T(bn64[2])};
         drain_loads();
-        Acc<T, R> acA, acB;
+        Acc<T, leaf_slots<KID, T, ADJ>()> acA, acB;
         acA.init();
         acB.init();
         double sfA[SPLIT ? R : 1], sfB[SPLIT ? R : 1];
@@ -568,13 +604,13 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
             if (va) {
                 if (uni(tclose)) {
                     for (int j = slice; j < cnt; j += S) {
-                        pair<KID, ADJ, FAST, true>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
-                        pair<KID, ADJ, FAST, true>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
+                        point_pair<KID, ADJ, FAST, true>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
+                        point_pair<KID, ADJ, FAST, true>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
                     }
                 } else {  // no point of the tile within the cutoff of the leaf: same result without the test
                     for (int j = slice; j < cnt; j += S) {
-                        pair<KID, ADJ, FAST, false>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
-                        pair<KID, ADJ, FAST, false>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
+                        point_pair<KID, ADJ, FAST, false>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
+                        point_pair<KID, ADJ, FAST, false>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
                     }
                 }
             }
@@ -608,8 +644,8 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
         __syncthreads();
         for (int q = 0; q < R; q++) {
             const double ea = SPLIT ? sfA[q] : 0.0, eb = SPLIT ? sfB[q] : 0.0;
-            sm.red[q * NB + tid] = va ? acA.value(q) + ea : 0.0;
-            sm.red[(R + q) * NB + tid] = vb ? acB.value(q) + eb : 0.0;
+            sm.red[q * NB + tid] = va ? leaf_value<KID, T, ADJ>(acA, q, an64) + ea : 0.0;
+            sm.red[(R + q) * NB + tid] = vb ? leaf_value<KID, T, ADJ>(acB, q, bn64) + eb : 0.0;
         }
         __syncthreads();
         slice_sum<NB>(sm.red, sm.part, 2 * R, ntp, S, [&](int v, int g, double s) {
@@ -692,7 +728,7 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     const int f0 = uni(it->f0), f1 = uni(it->f1), v0 = uni(it->v0), v1 = uni(it->v1);
     const int se0 = uni(it->c0), se1 = uni(it->c1), self = uni(it->self), part = uni(it->part);
     drain_loads();
-    Acc<T, R> acA, acB;
+    Acc<T, leaf_slots<KID, T, ADJ>()> acA, acB;
     acA.init();
     acB.init();
     double sfA[SPLIT ? R : 1], sfB[SPLIT ? R : 1];
@@ -729,13 +765,13 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
             if (va) {
                 if (tclose) {
                     for (int j = slice; j < cnt; j += S) {
-                        pair<KID, ADJ, FAST, true>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
-                        pair<KID, ADJ, FAST, true>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
+                        point_pair<KID, ADJ, FAST, true>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
+                        point_pair<KID, ADJ, FAST, true>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
                     }
                 } else {
                     for (int j = slice; j < cnt; j += S) {
-                        pair<KID, ADJ, FAST, false>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
-                        pair<KID, ADJ, FAST, false>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
+                        point_pair<KID, ADJ, FAST, false>(sm.pt, j, ax, ay, az, an, acA.tile(), kc);
+                        point_pair<KID, ADJ, FAST, false>(sm.pt, j, bx, by, bz, bn, acB.tile(), kc);
                     }
                 }
             }
@@ -787,8 +823,8 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     wave_sync();
     for (int q = 0; q < R; q++) {
         const double ea = SPLIT ? sfA[q] : 0.0, eb = SPLIT ? sfB[q] : 0.0;
-        sm.red[q * 64 + lane] = va ? acA.value(q) + ea : 0.0;
-        sm.red[(R + q) * 64 + lane] = vb ? acB.value(q) + eb : 0.0;
+        sm.red[q * 64 + lane] = va ? leaf_value<KID, T, ADJ>(acA, q, an64) + ea : 0.0;
+        sm.red[(R + q) * 64 + lane] = vb ? leaf_value<KID, T, ADJ>(acB, q, bn64) + eb : 0.0;
     }
     wave_sync();
     if (lane < nslot) {
