@@ -732,14 +732,16 @@ static void close_flags(DevList& l, const int* leaves, const DevTree& tt, const 
 // kernel keeps 96% busy.)
 // A small problem has fewer such items than the chip has room for, and its longest one
 // sets the launch's length. The items of both kernels are therefore also cut where they
-// exceed the problem's total pairs divided by kWaveFill (kBlockFill) items, four per SIMD
-// (compute unit), but not below kWaveCapMin (kBlockCapMin) pairs, where an item's fixed
-// costs would take over. These cuts fall on whole LDS tiles (wave: kWaveTile sources;
+// exceed the kernel's total pairs divided by kWaveFill (kBlockFill) items, about four rounds
+// of what the chip holds at once, but not below kWaveCapMin (kBlockCapMin) pairs, where an
+// item's fixed costs would take over. These cuts fall on whole LDS tiles (wave: kWaveTile sources;
 // block_tile), so that the FP32 partial sum of every tile is the same as uncut.
 // Measured (whole passes): mesh of 9,102 points, hypersingular, mixed 1316 -> 823 us (its
 // block leaves 489 -> 57 us); sphere of 15,360 points, Laplace 310 -> 213 us (leaf waves
 // 67 -> 22 us, symmetric pairs 95 -> 38); 300,007 points, order 50, mixed, forward and
-// backward 6.10 -> 4.30 ms; from about 1e9 pairs on nothing is cut that was not before.
+// backward 6.10 -> 4.30 ms (one round of the whole problem's pairs); then 3.84 -> 3.62 ms,
+// and the double layer, 61,440 points, order 35, 1049 -> 937 us, with four rounds of each
+// kernel's own pairs.
 // Lays out work items (work, item), given in tree order, for a launch whose workgroup
 // b runs on XCD b % 8 (the hardware deals workgroups to the XCDs in turn), g items per
 // workgroup. The items are cut into 8 runs of about equal work, one per XCD, so that
@@ -773,8 +775,8 @@ static std::vector<I> xcd_layout(const std::vector<std::pair<long, I>>& items, i
 }
 
 constexpr int kWaveChunkLeaf = 64;
-constexpr long kWaveFill = 4096, kWaveCapMin = 4096;
-constexpr long kBlockFill = 2048, kBlockCapMin = 16384;
+constexpr long kWaveFill = 16384, kWaveCapMin = 4096;
+constexpr long kBlockFill = 8192, kBlockCapMin = 16384;
 
 static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
                          const HostList& surf, int n_e, int block_tile, LeafSplit& out, hipStream_t s) {
@@ -786,10 +788,14 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
         return p0 < p1 ? (long)pts.rpre[p1 - 1] + pts.rcnt[p1 - 1] : 0;
     };
     auto cells_of = [&](size_t k) { return surf.ptr.empty() ? 0 : surf.ptr[k + 1] - surf.ptr[k]; };
-    long total = 0;
-    for (size_t k = 0; k < leaves.size(); k++)
-        total += (long)tt.count[leaves[k]] * (points_of(k) + (long)n_e * (cells_of(k) + 1));
-    const long wave_cap = std::max(kWaveCapMin, total / kWaveFill), block_cap = std::max(kBlockCapMin, total / kBlockFill);
+    auto on_wave = [](long m, long pairs) { return m <= (pairs <= kWavePairsMax ? kWaveLeafMax : kWaveChunkLeaf); };
+    long wave_total = 0, block_total = 0;
+    for (size_t k = 0; k < leaves.size(); k++) {
+        const long m = tt.count[leaves[k]], pairs = m * (points_of(k) + (long)n_e * (cells_of(k) + 1));
+        (on_wave(m, pairs) ? wave_total : block_total) += pairs;
+    }
+    const long wave_cap = std::max(kWaveCapMin, wave_total / kWaveFill),
+               block_cap = std::max(kBlockCapMin, block_total / kBlockFill);
     long part = 0;
     for (size_t k = 0; k < leaves.size(); k++) {
         const int pos = (int)k;
@@ -800,7 +806,7 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
         const int c0 = surf.ptr.empty() ? 0 : surf.ptr[k], c1 = c0 + cells_of(k);
         const long src = np + (long)n_e * (c1 - c0 + 1);
         const long nc = (m * src + kWavePairsMax - 1) / kWavePairsMax;
-        const bool wave = m <= (nc <= 1 ? kWaveLeafMax : kWaveChunkLeaf);
+        const bool wave = on_wave(m, m * src);
         if (!wave) b.push_back({m * src, pos});
         // runs of at most `per` sources, each cut further into chunks of at most `sub`
         // points, whole tiles from the run's start
