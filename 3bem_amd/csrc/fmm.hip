@@ -40,6 +40,12 @@ constexpr size_t kM2lOutputBudget = size_t(6) << 30;
 // at most kWaveLeafMax points: one work item each, or chunks of a large one) and the
 // one-workgroup kernel (the rest, whole or in chunks), both ordered by decreasing work
 // (split_leaves).
+// Below this many operator rows the surface stages apply the C2E product themselves
+// (SurfStage.c2e) instead of a level GEMM of its own per stage and level; it needs a row per
+// thread of kSurfBlock. From here on the MFMA products of the classes and levels take over.
+constexpr int kFuseC2eMax = 48;
+static_assert(kFuseC2eMax <= kSurfBlock, "one row per thread");
+
 struct LeafSplit {
     DevBuf<WaveItem> items, block_items;
     DevBuf<WaveLeafParts> parts;  // the wave items' cut leaves, then the block items'
@@ -88,6 +94,10 @@ struct FmmPlan {
     DevPoints sp, op;
     DevBuf<double> d_unit, d_inner, d_outer;
     DevBuf<double> uc2e, dc2e;
+    // below kFuseC2eMax rows the surface stages apply the C2E themselves: transposed copies
+    // per level (the forward's; the adjoint reads uc2e and dc2e)
+    bool fuse_c2e = false;
+    DevBuf<double> uc2e_t, dc2e_t;
     std::vector<double> h_uc2e, h_dc2e;
     TaskLists tl;
     // forward lists
@@ -1130,6 +1140,20 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     }
     P->h_uc2e = P->uc2e.to_host(s);
     P->h_dc2e = P->dc2e.to_host(s);
+    P->fuse_c2e = P->blk < kFuseC2eMax;
+    if (P->fuse_c2e) {
+        auto transposed = [&](const std::vector<double>& h, DevBuf<double>& d) {
+            std::vector<double> t(h.size());
+            const size_t n = P->blk;
+            for (size_t L = 0; L < h.size() / (n * n); L++)
+                for (size_t r = 0; r < n; r++)
+                    for (size_t k = 0; k < n; k++) t[(L * n + k) * n + r] = h[(L * n + r) * n + k];
+            d.upload(t, s);
+            TBEM_HIP(hipStreamSynchronize(s));  // t goes out of scope
+        };
+        transposed(P->h_uc2e, P->uc2e_t);
+        transposed(P->h_dc2e, P->dc2e_t);
+    }
     if (keep_fac) {
         for (int k = 0; k < 2; k++) {
             if (up_fac[k].n) P->h_fac[k] = up_fac[k].to_host(s);
@@ -1338,6 +1362,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     // the up-check potentials of a stage's cells -> equivalent densities, and, for
     // the MFMA M2L, the modal FP32 input Bu * check
     auto up_c2e = [&](const CellTiles& T) {
+        if (P.fuse_c2e) return;  // done by the stage
         launch_level_gemm(T, P.blk, P.uc2e.p, false, W.fld.p, nullptr, W.mult.p, nullptr, false, s);
         if (mfma) launch_level_gemm(T, P.blk, P.m2l_mfma.Bu.p, false, W.fld.p, nullptr, nullptr, W.chk_up.p, false, s);
     };
@@ -1346,12 +1371,20 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         launch_level_gemm(T, P.blk, P.dc2e.p, false, W.fld.p, nullptr, W.locals.p, nullptr, true, s);
     };
 
+    auto fuse_up = [&](SurfStage& a) {
+        if (P.fuse_c2e) { a.c2e = P.uc2e_t.p; a.c2e_out = W.mult.p; a.c2e_add = 0; }
+    };
+    auto fuse_down = [&](SurfStage& a) {
+        if (P.fuse_c2e) { a.c2e = P.dc2e_t.p; a.c2e_out = W.locals.p; a.c2e_add = 1; }
+    };
+
     // P2M (cpp/fmm.cpp:162-202): points of each source leaf -> up-check -> UC2E
     SurfStage a = surf_base(P);
     set_list(a, P.p2m);
     a.tt = view(P.dst); a.t_surf = P.d_outer.p;
     a.st = view(P.dst); a.sp = view(P.sp); a.dens = W.dens.p; a.n_src_pts = Ns;
     a.out = W.fld.p;
+    fuse_up(a);
     launch_surf_stage(P.kid, false, false, false, a, P.kc, s);
     up_c2e(P.t_p2m);
     TBEM_HIP(hipEventRecord(W.ev[2], s));
@@ -1367,6 +1400,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             m.tt = view(P.dst); m.t_surf = P.d_outer.p;
             m.st = view(P.dst); m.s_surf = P.d_inner.p; m.s_coeff = W.mult.p;
             m.out = W.fld.p;
+            fuse_up(m);
             launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         }
         up_c2e(P.t_m2m[L]);
@@ -1394,17 +1428,19 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         m.st = view(P.dst); m.s_surf = P.d_inner.p; m.s_coeff = W.mult.p;
         m.out = W.fld.p;
         m.no_cutoff = P.m2l_no_cutoff;
+        fuse_down(m);
         launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         TBEM_HIP(hipEventRecord(W.ev[9], s));
-        down_c2e(P.t_m2l);
+        if (!P.fuse_c2e) down_c2e(P.t_m2l);
     }
     SurfStage pl = surf_base(P);
     set_list(pl, P.p2l);
     pl.tt = view(P.dot); pl.t_surf = P.d_inner.p;
     pl.st = view(P.dst); pl.sp = view(P.sp); pl.dens = W.dens.p; pl.n_src_pts = Ns;
     pl.out = W.fld.p;
+    fuse_down(pl);
     launch_surf_stage(P.kid, false, false, false, pl, P.kc, s);
-    down_c2e(P.t_p2l);
+    if (!P.fuse_c2e) down_c2e(P.t_p2l);
     TBEM_HIP(hipEventRecord(W.ev[4], s));
 
     // L2L (cpp/fmm.cpp:384-413), root first
@@ -1418,9 +1454,10 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             l.tt = view(P.dot); l.t_surf = P.d_inner.p;
             l.st = view(P.dot); l.s_surf = P.d_outer.p; l.s_coeff = W.locals.p;
             l.out = W.fld.p;
+            fuse_down(l);
             launch_surf_stage(P.kid, true, false, false, l, P.kc, s);
         }
-        down_c2e(P.t_olev[L]);
+        if (!P.fuse_c2e) down_c2e(P.t_olev[L]);
     }
     TBEM_HIP(hipEventRecord(W.ev[5], s));
 }
@@ -1612,10 +1649,15 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
         launch_leaf_stage<T>(P.kid, true, f, P.kc, W.side, true);
         TBEM_HIP(hipEventRecord(W.join, W.side));
     }
-    launch_fill(W.lbar.p, nco, 0.0, s);
-    launch_fill(W.cbar.p, nco, 0.0, s);
+    // (with the C2E in the stages every cell's cbar and ebar is written: a leaf's by the L2P^T
+    // stage, a parent's by the L2L^T one, and below the root ebar by the M2M^T one)
+    const bool fuse = P.fuse_c2e;
+    if (!fuse) {
+        launch_fill(W.lbar.p, nco, 0.0, s);
+        launch_fill(W.cbar.p, nco, 0.0, s);
+        launch_fill(W.ebar.p, ncs, 0.0, s);
+    }
     launch_fill(W.mbar.p, ncs, 0.0, s);
-    launch_fill(W.ebar.p, ncs, 0.0, s);
 
     // L2P^T: observation points -> down-equivalent surface of their leaf
     SurfStage a = surf_base(P);
@@ -1623,11 +1665,12 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
     a.tt = view(P.dot); a.t_surf = P.d_outer.p;
     a.st = view(P.dot); a.sp = view(P.op); a.dens = W.gsort.p; a.n_src_pts = No;
     a.out = W.lbar.p;
+    if (fuse) { a.c2e = P.dc2e.p; a.c2e_out = W.cbar.p; }
     launch_surf_stage(P.kid, false, false, true, a, P.kc, s);
 
     // L2L^T, deepest level first: cbar = DC2E^T lbar, then push to parents
     for (int L = P.ot.n_levels - 1; L >= 0; L--) {
-        launch_level_gemm(P.t_olev[L], P.blk, P.dc2e.p, true, W.lbar.p, nullptr, W.cbar.p, nullptr, false, s);
+        if (!fuse) launch_level_gemm(P.t_olev[L], P.blk, P.dc2e.p, true, W.lbar.p, nullptr, W.cbar.p, nullptr, false, s);
         if (L == 0) break;
         if (P.l2l_ops[L].enabled) {  // lbar[parent] += sum over its children of K^T cbar[child]
             m2l_adjoint64(P.l2l_ops[L], W.cbar.p, W.ty.p, W.lbar.p, s);
@@ -1638,7 +1681,8 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
         l.tt = view(P.dot); l.t_surf = P.d_outer.p;
         l.st = view(P.dot); l.s_surf = P.d_inner.p; l.s_coeff = W.cbar.p;
         l.out = W.lbar.p;
-        launch_surf_stage(P.kid, true, true, true, l, P.kc, s);
+        if (fuse) { l.c2e = P.dc2e.p; l.c2e_out = W.cbar.p; }
+        launch_surf_stage(P.kid, true, !fuse, true, l, P.kc, s);
     }
 
     // M2L^T into mbar (FP64), or, on MFMA, e2 = Bu^T M_c^T Vd^T lbar, added to ebar below
@@ -1669,8 +1713,9 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
 
     // M2M^T, root first: ebar = UC2E^T mbar, then push to children
     for (int L = 0; L < P.st.n_levels; L++) {
-        launch_level_gemm(A.t_slev[L], P.blk, P.uc2e.p, true, W.mbar.p, mfma ? W.e2.p : nullptr, W.ebar.p, nullptr,
-                          false, s);
+        if (!fuse || L == 0)
+            launch_level_gemm(A.t_slev[L], P.blk, P.uc2e.p, true, W.mbar.p, mfma ? W.e2.p : nullptr, W.ebar.p, nullptr,
+                              false, s);
         if (L + 1 >= P.st.n_levels) break;
         if (P.m2m_ops[L].enabled) {  // mbar[child] += K^T ebar[parent]
             m2l_adjoint64(P.m2m_ops[L], W.ebar.p, W.ty.p, W.mbar.p, s);
@@ -1681,6 +1726,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
         c.tt = view(P.dst); c.t_surf = P.d_inner.p;
         c.st = view(P.dst); c.s_surf = P.d_outer.p; c.s_coeff = W.ebar.p;
         c.out = W.mbar.p;
+        if (fuse) { c.c2e = P.uc2e.p; c.c2e_out = W.ebar.p; }
         launch_surf_stage(P.kid, true, true, true, c, P.kc, s);
     }
 

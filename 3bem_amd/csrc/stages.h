@@ -106,6 +106,13 @@ struct SurfStage {
     int n_e, blk;
     double* out;            // blk per cell of tt: the raw check potentials (= or += with add)
     const int* order;       // the items' launch order (null: as listed), the most work first
+    // With c2e given (operators of at most kSurfBlock rows), the check-to-equivalent product of
+    // the cell's potentials follows in the same launch instead of the store to out:
+    // c2e_out[cell] (= or += with c2e_add) C field, field first added to out[cell] with add;
+    // C[row][k] of the cell's level at c2e[(level * blk + k) * blk + row].
+    const double* c2e;
+    double* c2e_out;
+    int c2e_add;
     int no_cutoff;          // surface sources: every pair is known to lie beyond the r2 < 1e-12
                             // cutoff, so the kernels leave the test out (same result)
 };

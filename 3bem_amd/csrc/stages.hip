@@ -405,6 +405,26 @@ __device__ __forceinline__ double leaf_value(const A& acc, int q, const double* 
 }
 
 // ------------------------------------------------------------------ surface targets
+// Row r of a level's check-to-equivalent operator (m: its k-major copy at row r) times the n
+// potentials in LDS, one FMA after the other in k as k_level_gemm adds them (the same bits).
+// The rows' loads are coalesced and, a level's operator being small, come from the CU's cache.
+// Used below kFuseC2eMax rows, where a launch of its own per level costs more than the product:
+// sphere of 15,360 points, order 5 195 -> 156 us a pass, double layer, 61,440 points, order 35,
+// forward and backward 937 -> 848 us, 1M points, order 6 2777 -> 2715 us.
+__device__ __forceinline__ double c2e_row(const double* __restrict__ m, const double* field, int n) {
+    double s = 0;
+    int k = 0;
+    for (; k + 8 <= n; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = m[(size_t)(k + u) * n];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s = fma(v[u], field[k + u], s);
+    }
+    for (; k < n; k++) s = fma(m[(size_t)k * n], field[k], s);
+    return s;
+}
+
 // CUT = false (surface sources only): the r2 < 1e-12 cutoff test is left out, when
 // the plan has shown every pair of the stage to be farther apart (SurfStage.no_cutoff).
 template <int KID, bool SRC_SURF, bool ADJ, bool DUAL, bool CUT = true>
@@ -474,7 +494,19 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
         __syncthreads();
     }
     double* o = a.out + (size_t)cell * a.blk;
-    for (int row = tid; row < a.blk; row += NB) o[row] = add ? o[row] + field[row] : field[row];
+    if (!a.c2e) {
+        for (int row = tid; row < a.blk; row += NB) o[row] = add ? o[row] + field[row] : field[row];
+        return;
+    }
+    if (add) {
+        if (tid < a.blk) field[tid] = o[tid] + field[tid];
+        __syncthreads();
+    }
+    if (tid < a.blk) {
+        const double s = c2e_row(a.c2e + (size_t)lvl * a.blk * a.blk + tid, field, a.blk);
+        double* e = a.c2e_out + (size_t)cell * a.blk + tid;
+        *e = a.c2e_add ? *e + s : s;
+    }
 }
 
 // The same stage for kSurfBlock / 2 < n_e <= kSurfOneMax with one target per lane and a
