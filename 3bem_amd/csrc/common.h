@@ -96,4 +96,15 @@ inline int div_up(size_t a, size_t b) { return (int)((a + b - 1) / b); }
 // that were active in a loop's last partial iteration.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// Device-side times of a pass's stages: a kernel that begins a stage writes the clock as its
+// first workgroup starts, one that ends the pass as its last workgroup (by index) is through.
+// A null pointer writes nothing. (A recorded event is a packet and a host call of its own
+// between two launches.)
+__device__ __forceinline__ void stamp_start(unsigned long long* t) {
+    if (t && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *t = wall_clock64();
+}
+__device__ __forceinline__ void stamp_end(unsigned long long* t) {
+    if (t && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *t = wall_clock64();
+}
+
 }  // namespace tbem

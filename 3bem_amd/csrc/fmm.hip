@@ -202,8 +202,15 @@ struct Work {
     DevBuf<double> wpart;   // chunk sums of the leaf kernels (LeafSplit::part_size)
     DevBuf<double> wsym;    // target sums of the symmetric pairs' chunks (FmmPlan::sym.part_size)
     DevBuf<double> wrev;    // reverse sums of the symmetric pairs (R rows of FmmPlan::sym.n_rev)
-    hipEvent_t ev[12];  // 0..7 stage boundaries; 8, 9 around the M2L translation kernel; 10, 11
-                        // around the point-pair (P2P) launch on the side stream
+    // Stage boundaries 0..7; 8, 9 around the M2L translation kernel; 10, 11 around the
+    // point-pair (P2P) launch on the side stream. Where the surface stages apply the C2E (small
+    // operators, where a pass may be as short as its launches) 0..9 are stamps in ts that the
+    // stages' own kernels write, else events. A sphere of 15,360 points, order 5, host-bound:
+    // 142 us a pass with the ten events, 122 with the stamps; 61k points, order 35, 848 -> 822.
+    hipEvent_t ev[12];
+    DevBuf<unsigned long long> ts;
+    double ts_per_ms = 0;
+    bool stamped = false;  // the last forward's boundaries are in ts
     hipEvent_t done = nullptr;  // end of the last call's work, on whichever stream it ran
     bool timed = false;
     // The forward's P2P needs only the gathered densities, so it can run on a side
@@ -225,7 +232,15 @@ struct Work {
     uint64_t far_token = 0, next_token = 0;
     explicit Work(const FmmPlan& P) {
         TBEM_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        for (auto& e: ev) TBEM_HIP(hipEventCreate(&e));
+        // (timing only: nothing waits for them, so they need no cache release)
+        for (auto& e: ev) TBEM_HIP(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
+        if (P.fuse_c2e) {
+            ts.alloc(kStamps);
+            int dev = 0, khz = 0;
+            TBEM_HIP(hipGetDevice(&dev));
+            TBEM_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+            ts_per_ms = khz;
+        }
         TBEM_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         TBEM_HIP(hipEventRecord(done, stream));
         TBEM_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
@@ -1354,9 +1369,15 @@ template <class F = std::nullptr_t>
 static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, bool mfma, F&& after_gather = nullptr) {
     const int R = P.R;
     const int Ns = (int)P.n_src;
-    TBEM_HIP(hipEventRecord(W.ev[0], s));
-    launch_gather_dens(x, P.sp.perm.p, P.sp.w.p, Ns, R, W.dens.p, s);
-    TBEM_HIP(hipEventRecord(W.ev[1], s));
+    // boundary k: a stamp of the kernel that begins the stage, or an event
+    auto st = [&](int k) { return P.fuse_c2e ? W.ts.p + k : nullptr; };
+    auto mark = [&](int k) {
+        if (!P.fuse_c2e) TBEM_HIP(hipEventRecord(W.ev[k], s));
+    };
+    W.stamped = P.fuse_c2e;
+    mark(0);
+    launch_gather_dens(x, P.sp.perm.p, P.sp.w.p, Ns, R, W.dens.p, s, st(0));
+    mark(1);
     if constexpr (!std::is_same<typename std::decay<F>::type, std::nullptr_t>::value) after_gather();
 
     // the up-check potentials of a stage's cells -> equivalent densities, and, for
@@ -1385,9 +1406,10 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     a.st = view(P.dst); a.sp = view(P.sp); a.dens = W.dens.p; a.n_src_pts = Ns;
     a.out = W.fld.p;
     fuse_up(a);
+    a.stamp = st(1);
     launch_surf_stage(P.kid, false, false, false, a, P.kc, s);
     up_c2e(P.t_p2m);
-    TBEM_HIP(hipEventRecord(W.ev[2], s));
+    mark(2);
 
     // M2M (cpp/fmm.cpp:204-251), deepest parents first
     for (int L = P.st.n_levels - 2; L >= 0; L--) {
@@ -1401,15 +1423,16 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             m.st = view(P.dst); m.s_surf = P.d_inner.p; m.s_coeff = W.mult.p;
             m.out = W.fld.p;
             fuse_up(m);
+            if (L == P.st.n_levels - 2) m.stamp = st(2);
             launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         }
         up_c2e(P.t_m2m[L]);
     }
-    TBEM_HIP(hipEventRecord(W.ev[3], s));
+    mark(3);
 
     // M2L (cpp/fmm.cpp:362-382) and P2L (cpp/fmm.cpp:296-330) into locals
-    launch_fill(W.locals.p, W.locals.n, 0.0, s);
-    TBEM_HIP(hipEventRecord(W.ev[8], s));
+    launch_fill(W.locals.p, W.locals.n, 0.0, s, st(3), st(8));
+    mark(8);
     if (mfma) {
         // Vd M_c Bu check = DC2E K_c UC2E check = the FP64 stage's DC2E K_c mult
         YLease y(P, s);
@@ -1419,7 +1442,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         // FP64 class operators: check potential = sum over pairs of K_c mult, then DC2E
         YLease y(P, s);
         m2l_forward64(P.m2l_mfma, P.m2l.items.p, P.m2l.ptr.p, P.m2l.cell.p, W.mult.p, P.m2l_y64.p, W.fld.p, s,
-                      W.ev[9]);
+                      P.fuse_c2e ? nullptr : W.ev[9], st(9));
         down_c2e(P.t_m2l);
     } else {
         SurfStage m = surf_base(P);
@@ -1430,7 +1453,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         m.no_cutoff = P.m2l_no_cutoff;
         fuse_down(m);
         launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
-        TBEM_HIP(hipEventRecord(W.ev[9], s));
+        mark(9);
         if (!P.fuse_c2e) down_c2e(P.t_m2l);
     }
     SurfStage pl = surf_base(P);
@@ -1439,9 +1462,10 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     pl.st = view(P.dst); pl.sp = view(P.sp); pl.dens = W.dens.p; pl.n_src_pts = Ns;
     pl.out = W.fld.p;
     fuse_down(pl);
+    if (!P.m2l_mfma.enabled) pl.stamp = st(9);
     launch_surf_stage(P.kid, false, false, false, pl, P.kc, s);
     if (!P.fuse_c2e) down_c2e(P.t_p2l);
-    TBEM_HIP(hipEventRecord(W.ev[4], s));
+    mark(4);
 
     // L2L (cpp/fmm.cpp:384-413), root first
     for (int L = 1; L < P.ot.n_levels; L++) {
@@ -1455,11 +1479,12 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             l.st = view(P.dot); l.s_surf = P.d_outer.p; l.s_coeff = W.locals.p;
             l.out = W.fld.p;
             fuse_down(l);
+            if (L == 1) l.stamp = st(4);
             launch_surf_stage(P.kid, true, false, false, l, P.kc, s);
         }
         if (!P.fuse_c2e) down_c2e(P.t_olev[L]);
     }
-    TBEM_HIP(hipEventRecord(W.ev[5], s));
+    mark(5);
 }
 
 static void set_split(LeafStage& f, const LeafSplit& sp, Work& W) {
@@ -1522,6 +1547,7 @@ static void forward_T(const FmmPlan& P, Work& W, const double* x, double* y, hip
         return;
     }
     const bool mfma = std::is_same<T, float>::value && P.m2l_mfma.enabled && !P.m2l_mfma.fp64;
+    auto st = [&](int k) { return P.fuse_c2e ? W.ts.p + k : nullptr; };
     W.split_last = W.overlap;
     if (W.overlap) {
         // P2P on the side stream once the densities are gathered, beside the far field
@@ -1545,17 +1571,19 @@ static void forward_T(const FmmPlan& P, Work& W, const double* x, double* y, hip
         set_split(f, P.surf_split, W);
         f.rp_ptr = nullptr;
         f.accumulate = 1;
+        f.stamp = st(5);
         launch_leaf_stage<double>(P.kid, false, f, P.kc, s, true);
     } else {
         farfield(P, W, x, s, mfma);
         W.far_token = ++W.next_token;
         LeafStage f = leaf_stage_args(P, W);
         use_sym(f, P, W);
+        f.stamp = st(5);
         launch_leaf_stage<T>(P.kid, false, f, P.kc, s, true);
     }
-    TBEM_HIP(hipEventRecord(W.ev[6], s));
-    launch_scatter_out(W.out_sorted.p, P.op.perm.p, No, R, y, s);
-    TBEM_HIP(hipEventRecord(W.ev[7], s));
+    if (!P.fuse_c2e) TBEM_HIP(hipEventRecord(W.ev[6], s));
+    launch_scatter_out(W.out_sorted.p, P.op.perm.p, No, R, y, s, st(6), st(7));
+    if (!P.fuse_c2e) TBEM_HIP(hipEventRecord(W.ev[7], s));
     W.timed = true;
 }
 
@@ -1839,6 +1867,22 @@ static int guard(F&& f) {
         set_last_error(e.what());
         return TBEM_E_INVALID;
     }
+}
+
+// The last forward's stamps in milliseconds from the first. A stage without a kernel left
+// none: it takes the next boundary's (the M2L's end, 9, comes before 4).
+static std::array<double, kStamps> stamps_ms(Work& W) {
+    TBEM_HIP(hipEventSynchronize(W.done));
+    const std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
+    std::array<double, kStamps> t{};
+    const int order[kStamps] = {0, 1, 2, 3, 8, 9, 4, 5, 6, 7};
+    double next = 0;
+    for (int i = kStamps - 1; i >= 0; i--) {
+        const int k = order[i];
+        if (raw[k]) next = (double)(long long)(raw[k] - raw[0]) / W.ts_per_ms;
+        t[k] = next;
+    }
+    return t;
 }
 
 static void host_roundtrip(tbem_fmm_s* h, bool adj, const double* in, double* out) {
@@ -2187,11 +2231,16 @@ int tbem_fmm_stage_times(tbem_fmm_t h, double* ms) {
         TBEM_REQUIRE(h && ms, TBEM_E_INVALID, "null argument");
         Work& W = *h->work;
         TBEM_REQUIRE(W.timed, TBEM_E_INVALID, "no timed apply yet");
-        TBEM_HIP(hipEventSynchronize(W.ev[7]));
-        for (int k = 0; k < 7; k++) {
-            float t = 0;
-            TBEM_HIP(hipEventElapsedTime(&t, W.ev[k], W.ev[k + 1]));
-            ms[k] = t;
+        if (W.stamped) {
+            const std::array<double, kStamps> t = stamps_ms(W);
+            for (int k = 0; k < 7; k++) ms[k] = t[k + 1] - t[k];
+        } else {
+            TBEM_HIP(hipEventSynchronize(W.ev[7]));
+            for (int k = 0; k < 7; k++) {
+                float t = 0;
+                TBEM_HIP(hipEventElapsedTime(&t, W.ev[k], W.ev[k + 1]));
+                ms[k] = t;
+            }
         }
         if (W.split_last) {  // the leaf stage ran as P2P (side stream) + M2P/L2P
             float t = 0;
@@ -2214,6 +2263,11 @@ int tbem_fmm_m2l_ms(tbem_fmm_t h, double* ms) {
         TBEM_REQUIRE(h && ms, TBEM_E_INVALID, "null argument");
         Work& W = *h->work;
         TBEM_REQUIRE(W.timed, TBEM_E_INVALID, "no timed apply yet");
+        if (W.stamped) {
+            const std::array<double, kStamps> t = stamps_ms(W);
+            *ms = t[9] - t[8];
+            return;
+        }
         TBEM_HIP(hipEventSynchronize(W.ev[7]));
         float t = 0;
         TBEM_HIP(hipEventElapsedTime(&t, W.ev[8], W.ev[9]));

@@ -71,9 +71,11 @@ void build_m2l_mfma(M2lMfma& M, int kid, const KConst& kc, const HostTree& ot, c
 void m2l_forward32(const M2lMfma& M, const int* items, const int* ptr, const int* pair_src, const CellTiles& targets,
                    const float* chk_up, float* Y, double* z, double* locals, hipStream_t s, hipEvent_t kernel_end);
 // FP64 path, forward: slice by slice, Y[p] = K_{class(p)} * mult[src(p)] (FP64 MFMA)
-// and fld[t] = sum of the target's Y in pair order.
+// and fld[t] = sum of the target's Y in pair order. stamp, if given, takes the time after
+// the last slice's MFMA kernel (see stamp_start).
 void m2l_forward64(const M2lMfma& M, const int* items, const int* ptr, const int* pair_src, const double* mult,
-                   double* Y, double* fld, hipStream_t s, hipEvent_t kernel_end);
+                   double* Y, double* fld, hipStream_t s, hipEvent_t kernel_end,
+                   unsigned long long* stamp = nullptr);
 // Mixed path, transpose: w[t] = float(Vd[level t]^T lbar[t]) for the M2L targets,
 // then slice by slice Y[p] = M_c^T w[tgt(p)] and z[s] (+)= the source's Y in the
 // slice, and e2[s] = Bu[level s]^T z[s] for the sources with pairs (z: scratch).

@@ -418,7 +418,8 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
 __global__ __launch_bounds__(256) void k_m2l_pair_sum64(const int* __restrict__ items, const int* __restrict__ ptr,
                                                         const int* __restrict__ pairs, const double* __restrict__ Y,
                                                         int ystride, int blk, int ybase, int pb, int pe, int add,
-                                                        double* __restrict__ out) {
+                                                        double* __restrict__ out, unsigned long long* stamp) {
+    stamp_start(stamp);
     extern __shared__ double part64[];  // npar * ystride partial sums (npar > 1 only)
     const int k = blockIdx.x;
     const int t = uni(items[k]);
@@ -1000,7 +1001,7 @@ static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const dou
 // the forward sums of slice q: its items' pairs, out[t] = sum (FP32 Y into FP64 z, or FP64 Y)
 template <class T>
 static void forward_sum_slice(const M2lMfma& M, int q, const int* items, const int* ptr, const T* Y, double* out,
-                              hipStream_t s) {
+                              hipStream_t s, unsigned long long* stamp = nullptr) {
     const int k0 = M.slice_items[q], nk = M.slice_items[q + 1] - k0;
     if (nk == 0) return;
     if constexpr (std::is_same<T, float>::value) {
@@ -1009,7 +1010,7 @@ static void forward_sum_slice(const M2lMfma& M, int q, const int* items, const i
                            items + k0, ptr + k0, nullptr, Y, M.ystride, M.blk, M.slice_pairs[q], 0, 0, 0, out);
     } else {
         hipLaunchKernelGGL(k_m2l_pair_sum64, dim3(nk), dim3(256), pair_sum64_shm(M.ystride), s, items + k0,
-                           ptr + k0, nullptr, Y, M.ystride, M.blk, M.slice_pairs[q], 0, 0, 0, out);
+                           ptr + k0, nullptr, Y, M.ystride, M.blk, M.slice_pairs[q], 0, 0, 0, out, stamp);
     }
     TBEM_LAUNCH_CHECK();
 }
@@ -1027,7 +1028,8 @@ static void adjoint_sum_slice(const M2lMfma& M, int q, const T* Y, double* out, 
                            M.adj_items.p, M.adj_ptr.p, M.adj_pairs.p, Y, M.ystride, M.blk, pb, pb, pe, add, out);
     } else {
         hipLaunchKernelGGL(k_m2l_pair_sum64, dim3(M.n_adj), dim3(256), pair_sum64_shm(M.ystride), s,
-                           M.adj_items.p, M.adj_ptr.p, M.adj_pairs.p, Y, M.ystride, M.blk, pb, pb, pe, add, out);
+                           M.adj_items.p, M.adj_ptr.p, M.adj_pairs.p, Y, M.ystride, M.blk, pb, pb, pe, add, out,
+                           (unsigned long long*)nullptr);
     }
     TBEM_LAUNCH_CHECK();
 }
@@ -1044,12 +1046,12 @@ void m2l_forward32(const M2lMfma& M, const int* items, const int* ptr, const int
 }
 
 void m2l_forward64(const M2lMfma& M, const int* items, const int* ptr, const int* pair_src, const double* mult,
-                   double* Y, double* fld, hipStream_t s, hipEvent_t kernel_end) {
+                   double* Y, double* fld, hipStream_t s, hipEvent_t kernel_end, unsigned long long* stamp) {
     if (!M.enabled || !M.fp64) return;
     for (int q = 0; q < M.n_slices; q++) {
         mfma64_slice(M, q, pair_src, mult, Y, false, s);
         if (kernel_end && q + 1 == M.n_slices) TBEM_HIP(hipEventRecord(kernel_end, s));
-        forward_sum_slice<double>(M, q, items, ptr, Y, fld, s);
+        forward_sum_slice<double>(M, q, items, ptr, Y, fld, s, q + 1 == M.n_slices ? stamp : nullptr);
     }
 }
 

@@ -113,6 +113,7 @@ struct SurfStage {
     const double* c2e;
     double* c2e_out;
     int c2e_add;
+    unsigned long long* stamp;  // see stamp_start
     int no_cutoff;          // surface sources: every pair is known to lie beyond the r2 < 1e-12
                             // cutoff, so the kernels leave the test out (same result)
 };
@@ -161,6 +162,7 @@ struct LeafStage {
     int n_e, blk;
     double* out_sorted;
     int accumulate;         // out_sorted += (instead of =) the stage's sums
+    unsigned long long* stamp;  // see stamp_start (the first kernel of the stage)
     // The leaf positions a gradient launch serves (null: 0 .. n_leaves-1, one workgroup each).
     const int* order;
     int n_order;
@@ -228,10 +230,14 @@ void launch_range_close(int n_items, const int* leaves, const TreeView& tt, cons
                         const int* rbeg, const int* rcnt, const PtsView& sp, double margin, int* close,
                         hipStream_t s);
 
+// ts (optional): kStamps stamps, cleared, and the first set as the kernel starts
+constexpr int kStamps = 10;
 void launch_gather_dens(const double* x, const int* perm, const double* w, int n, int R,
-                        double* dens, hipStream_t s);
+                        double* dens, hipStream_t s, unsigned long long* ts = nullptr);
+// t0, t1 (optional): stamps of the kernel's start and end
 void launch_scatter_out(const double* out_sorted, const int* perm, int n, int R, double* y,
-                        hipStream_t s);
-void launch_fill(double* p, size_t n, double v, hipStream_t s);
+                        hipStream_t s, unsigned long long* t0 = nullptr, unsigned long long* t1 = nullptr);
+void launch_fill(double* p, size_t n, double v, hipStream_t s, unsigned long long* t0 = nullptr,
+                 unsigned long long* t1 = nullptr);
 
 }  // namespace tbem

@@ -434,6 +434,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     __shared__ StageSmem<double, R, NRM, NB, (DUAL ? 2 : 1) * R> sm;
     extern __shared__ double field[];  // R * n_e
+    stamp_start(a.stamp);
     const int item = a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
     const int cell = uni(a.items[item]);
     const int lvl = uni(a.tt.level[cell]);
@@ -589,6 +590,7 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
     __shared__ StageSmem<T, R, NRM, NB, 2 * R> sm;
+    stamp_start(a.stamp);
     const WaveItem* it = a.split ? a.block_items + blockIdx.x : nullptr;
     const int pos = it ? uni(it->pos) : (int)blockIdx.x;
     if (pos < 0) return;  // padding of the layout (the whole workgroup)
@@ -738,6 +740,7 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
     __shared__ WaveSmem<T, R, NRM> smw[kWaveBlock / 64];
+    stamp_start(a.stamp);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int idx = blockIdx.x * (kWaveBlock / 64) + w;
     if (idx >= a.n_wave) return;  // the whole wave: nothing below synchronizes the block
@@ -1640,7 +1643,9 @@ __global__ __launch_bounds__(WR* WC * 64) void k_level_gemm(int n, const int* __
 }
 
 __global__ void k_gather_dens(const double* __restrict__ x, const int* __restrict__ perm,
-                              const double* __restrict__ w, int n, int R, double* __restrict__ dens) {
+                              const double* __restrict__ w, int n, int R, double* __restrict__ dens,
+                              unsigned long long* ts) {
+    if (ts && blockIdx.x == 0 && threadIdx.x < kStamps) ts[threadIdx.x] = threadIdx.x == 0 ? wall_clock64() : 0ull;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int g = perm[i];
@@ -1649,16 +1654,20 @@ __global__ void k_gather_dens(const double* __restrict__ x, const int* __restric
 }
 
 __global__ void k_scatter_out(const double* __restrict__ out_sorted, const int* __restrict__ perm, int n,
-                              int R, double* __restrict__ y) {
+                              int R, double* __restrict__ y, unsigned long long* t0, unsigned long long* t1) {
+    stamp_start(t0);
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int g = perm[i];
     for (int q = 0; q < R; q++) y[(size_t)q * n + g] = out_sorted[(size_t)q * n + i];
+    stamp_end(t1);
 }
 
-__global__ void k_fill(double* __restrict__ p, size_t n, double v) {
+__global__ void k_fill(double* __restrict__ p, size_t n, double v, unsigned long long* t0, unsigned long long* t1) {
+    stamp_start(t0);
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
         p[i] = v;
+    stamp_end(t1);
 }
 
 CellTiles make_cell_tiles(const std::vector<int>& cells_in, const HostTree& t, hipStream_t s) {
@@ -1764,22 +1773,23 @@ void launch_range_close(int n_items, const int* leaves, const TreeView& tt, cons
 }
 
 void launch_gather_dens(const double* x, const int* perm, const double* w, int n, int R, double* dens,
-                        hipStream_t s) {
+                        hipStream_t s, unsigned long long* ts) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_gather_dens, dim3(div_up(n, 256)), dim3(256), 0, s, x, perm, w, n, R, dens);
+    hipLaunchKernelGGL(k_gather_dens, dim3(div_up(n, 256)), dim3(256), 0, s, x, perm, w, n, R, dens, ts);
     TBEM_LAUNCH_CHECK();
 }
 
-void launch_scatter_out(const double* out_sorted, const int* perm, int n, int R, double* y, hipStream_t s) {
+void launch_scatter_out(const double* out_sorted, const int* perm, int n, int R, double* y, hipStream_t s,
+                        unsigned long long* t0, unsigned long long* t1) {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_scatter_out, dim3(div_up(n, 256)), dim3(256), 0, s, out_sorted, perm, n, R, y);
+    hipLaunchKernelGGL(k_scatter_out, dim3(div_up(n, 256)), dim3(256), 0, s, out_sorted, perm, n, R, y, t0, t1);
     TBEM_LAUNCH_CHECK();
 }
 
-void launch_fill(double* p, size_t n, double v, hipStream_t s) {
+void launch_fill(double* p, size_t n, double v, hipStream_t s, unsigned long long* t0, unsigned long long* t1) {
     if (n == 0) return;
     int blocks = (int)std::min<size_t>(4096, (n + 255) / 256);
-    hipLaunchKernelGGL(k_fill, dim3(blocks), dim3(256), 0, s, p, n, v);
+    hipLaunchKernelGGL(k_fill, dim3(blocks), dim3(256), 0, s, p, n, v, t0, t1);
     TBEM_LAUNCH_CHECK();
 }
 
@@ -1857,6 +1867,7 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
         }
         LeafStage bl = a;
         bl.split_rest = 1;
+        if (a.n_wave > 0) bl.stamp = nullptr;
         leaf_launch<KID, T>(adj, fast, bl, c, s);  // block_items, then the parts of both
         if (a.sy_items && a.rp_ptr) {  // the pairs left out of the rp_* lists, then their reverse sums
             TBEM_REQUIRE((KID == K_EU || KID == K_LS) && fast, TBEM_E_INVALID,
