@@ -81,6 +81,7 @@ struct FmmPlan {
         DevBuf<WaveItem> items;         // the owners, whole or in chunks (pos, v0, v1, part)
         DevBuf<WaveLeafParts> g_parts;  // per receiving or cut position, its chunks
         int n_items = 0, n_g = 0, n_leaves = 0;
+        int slots = 0;  // 64 + the most points of an owner (k_leaf_sym's LDS)
         size_t part_size = 0;           // doubles of the chunks' target sums (Work::wsym)
         size_t n_rev = 0;
         double pairs = 0;  // unordered point pairs
@@ -1010,6 +1011,7 @@ static void build_sym(FmmPlan& P, const HostTree& T, const std::vector<std::arra
                                 WaveItem{k, 0, 0, (int)v, (int)std::min(n, v + per), 0, 0, 0, (int)part}});
         }
         Y.n_leaves++;
+        Y.slots = std::max(Y.slots, 64 + (int)m);
         Y.pairs += (double)n * T.count[leaves[k]];
         n_rev += (size_t)n;
         TBEM_REQUIRE(n_rev <= (size_t)INT32_MAX, TBEM_E_UNSUPPORTED, "symmetric pairs: too many slots");
@@ -1513,7 +1515,7 @@ static void use_sym(LeafStage& f, const FmmPlan& P, Work& W, const FmmPlan::AdjL
     f.rp_pre = o.rpre.p; f.rp_close = o.rclose.p;
     set_split(f, A ? A->sym_split : Y.split, W);
     f.sy_ptr = Y.own.ptr.p; f.sy_beg = Y.own.rbeg.p; f.sy_cnt = Y.own.rcnt.p; f.sy_pre = Y.own.rpre.p;
-    f.sy_base = Y.base.p; f.sy_items = Y.items.p; f.n_sy_items = Y.n_items; f.sy_part_buf = W.wsym.p;
+    f.sy_base = Y.base.p; f.sy_items = Y.items.p; f.n_sy_items = Y.n_items; f.sy_slots = Y.slots; f.sy_part_buf = W.wsym.p;
     f.sg_pos = Y.g_pos.p; f.sg_ptr = Y.g_ptr.p; f.sg_off = Y.g_off.p; f.sg_parts = Y.g_parts.p; f.n_sg = Y.n_g;
     f.rev = W.wrev.p; f.n_rev = Y.n_rev;
 }

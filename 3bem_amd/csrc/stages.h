@@ -35,7 +35,7 @@ constexpr int leaf_block() {
 }
 template <int KID, class T>
 constexpr int leaf_waves() {
-    return leaf_narrow<KID, T>() ? 3 : ((KID == 4 || KID == 5) ? 4 : 1);
+    return leaf_narrow<KID, T>() ? 3 : ((KID >= 3 && KID <= 5) ? 4 : 1);
 }
 constexpr int kGradBlock = 256;  // observation-coordinate gradient of the point-target stage
 constexpr int kWaveBlock = 256;        // k_leaf_wave: four work items per workgroup
@@ -47,7 +47,6 @@ constexpr int kPartsBlock = 128;       // k_leaf_parts
 constexpr int kSymBlock = 256;         // k_leaf_sym: four waves per leaf
 constexpr int kSymLeafMin = 16;        // k_leaf_sym takes leaves of kSymLeafMin .. kSymLeafMax
 constexpr int kSymLeafMax = 256;       // points (the plan chooses which, per kernel)
-constexpr int kSymSlots = kSymLeafMax + 64;  // k_leaf_sym's target slots per wave and component
 constexpr int kSymSrc = 3;             // k_leaf_sym: sources per lane
 
 // One work item of k_leaf_wave (and of k_leaf_stage, LeafStage.block_items): the leaf at
@@ -191,7 +190,7 @@ struct LeafStage {
     // its own chunks' (sg_parts, n = 0: not cut).
     const int *sy_ptr, *sy_beg, *sy_cnt, *sy_pre, *sy_base;
     const WaveItem* sy_items;
-    int n_sy_items;
+    int n_sy_items, sy_slots;  // sy_slots: 64 + the most points of an owner
     double* sy_part_buf;
     const int *sg_pos, *sg_ptr, *sg_off;
     const WaveLeafParts* sg_parts;

@@ -577,8 +577,8 @@ __global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double
 // sources accumulate in T (acA, acB); surface sources in FP64 (sfA, sfB, which
 // are acA, acB themselves when T is double). Register budget: at 512 threads per
 // workgroup, <= 128 VGPRs keeps two workgroups per CU; one more register halves
-// the resident waves (the elastic-U FP32 instance at 139 VGPRs ran 1.5x slower),
-// so leaf_waves() makes the compiler hold that budget (leaf_block() for the rest).
+// the resident waves (the elastic-U FP32 instance at 139 VGPRs ran 1.5x slower, at 142 and
+// FP64 at 144 1.25x), so leaf_waves() makes the compiler hold that budget (leaf_block() for the rest).
 // CLOSE: tiles without close points (LeafStage.rp_close) skip the cutoff test; the
 // instances without it have one pair loop and fewer registers, which pays where
 // leaves are small and per-leaf work dominates.
@@ -913,19 +913,20 @@ __global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, double 
 // evaluates each pair with the points of the leaves it owns (the sources; every
 // unordered leaf pair has one owner) once. A wave takes 64 x kSymSrc sources at a
 // time, kSymSrc per lane, and visits the m targets in the rotated order
-// t = (r + k) mod m, r = lane mod m: the lanes of one group (lane / m; one group when
-// m >= 64) update distinct targets at every step, and each group has its own copy of
-// the wave's target sums in LDS (one LDS add per component and step; a slot's adds
-// arrive in instruction order, the same on every run); the source sums stay in
+// (lane + k) mod m, k = 0 .. m - 1, adding to slot lane + k of the wave's target sums in
+// LDS: the lanes of a step add to distinct slots (one LDS add per component and step; a
+// slot's adds arrive in instruction order, the same on every run); the source sums stay in
 // registers over all m targets, then go to the reverse buffer at the source's slot;
 // k_sym_gather adds those slots in list order.
 // The transpose runs the same pairs (U^T = U) with each sum times t_weight, the
 // source weight of the point it goes to.
-struct alignas(16) SymTarget {
-    double x, y, z, v0, v1, v2;
-};
 // (T: the pair arithmetic; positions stay FP64, so the displacement is exact before
 // it is rounded to T, as in the other point-pair kernels)
+// Bound: vector issue (Kelvin U 34 instructions a pair and the root, Laplace 13). The LDS
+// is sized by the largest owner (64 + m slots of a record and four sums), so that registers
+// and not LDS set the waves per SIMD: 4 and 5, where slots for kSymLeafMax points with room
+// for three components left 3. Measured, 4M points in clusters, Laplace FP32: 14.6 -> 12.6
+// ms; Kelvin U FP64 issues as fast with three (2M points, 10.2 ms both).
 template <class T>
 struct SymSource {
     double x, y, z;
@@ -998,7 +999,11 @@ __device__ inline void sym_load(SymSource<T>& s, int p, int n, int e0, int e1, c
     s.r2 = T(0);
 }
 
-// Step k takes slot r + k of the records and of the group's sums: records repeat the
+// A target's record: x, y | z, v0 | v1, v2 (the last for three components only)
+template <int R>
+constexpr int kSymRecord = R > 1 ? 3 : 2;
+
+// Step k takes slot lane + k of the records and of the wave's sums: records repeat the
 // targets past slot m (slot s holds target s mod m), and the sums of slots m.. are
 // folded onto their targets at the end. The target sums are FP64 in LDS whatever T is.
 template <int KID, class T, bool CUT>
@@ -1009,32 +1014,37 @@ __device__ __forceinline__ void sym_step(SymSource<T>* sv, double2 A, double2 B,
     sym_pair<KID, T, CUT, true>(sv[0], A.x, A.y, B.x, tv0, tv1, tv2, u2, f);
     for (int u = 1; u < kSymSrc; u++) sym_pair<KID, T, CUT, false>(sv[u], A.x, A.y, B.x, tv0, tv1, tv2, u2, f);
     for (int q = 0; q < R; q++)
-        __hip_atomic_fetch_add(acc + q * kSymSlots, (double)f[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(acc + q, (double)f[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Two steps per iteration, both records read first: LDS operations complete in
 // order, so a read issued after a step's adds waits for them; this waits once per two.
 template <int KID, class T, bool CUT>
-__device__ __forceinline__ void sym_block(SymSource<T>* sv, const SymTarget* tg, double* fa, int m, int r, T u2) {
-    const double2* rec = reinterpret_cast<const double2*>(tg + r);
-    double* acc = fa + r;
+__device__ __forceinline__ void sym_block(SymSource<T>* sv, const double2* tg, double* fa, int m, T u2) {
+    constexpr int R = kernel_dim(KID), NT = kSymRecord<R>;
+    const int lane = threadIdx.x & 63;
+    const double2* rec = tg + NT * lane;
+    double* acc = fa + R * lane;
     int k = 0;
     for (; k + 2 <= m; k += 2) {
-        const double2 A0 = rec[0], B0 = rec[1], C0 = rec[2], A1 = rec[3], B1 = rec[4], C1 = rec[5];
+        const double2 A0 = rec[0], B0 = rec[1], C0 = rec[NT - 1];
+        const double2 A1 = rec[NT], B1 = rec[NT + 1], C1 = rec[2 * NT - 1];
         sym_step<KID, T, CUT>(sv, A0, B0, C0, acc, u2);
-        sym_step<KID, T, CUT>(sv, A1, B1, C1, acc + 1, u2);
-        rec += 6;
-        acc += 2;
+        sym_step<KID, T, CUT>(sv, A1, B1, C1, acc + R, u2);
+        rec += 2 * NT;
+        acc += 2 * R;
     }
-    if (k < m) sym_step<KID, T, CUT>(sv, rec[0], rec[1], rec[2], acc, u2);
+    if (k < m) sym_step<KID, T, CUT>(sv, rec[0], rec[1], rec[NT - 1], acc, u2);
 }
 
 template <int KID, class T>
 __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, double scale) {
     constexpr int NW = kSymBlock / 64;
     constexpr int R = kernel_dim(KID);
-    __shared__ SymTarget tg[kSymSlots];
-    __shared__ double facc[NW][3 * kSymSlots];
+    constexpr int NT = kSymRecord<R>;
+    const int S = a.sy_slots;        // slots: lane + k < 64 + m <= S
+    extern __shared__ double2 tg[];  // the records, then each wave's sums (R per slot)
+    double* const facc = reinterpret_cast<double*>(tg + NT * S);
     const WaveItem* it = a.sy_items + blockIdx.x;
     const int pos = uni(it->pos);
     if (pos < 0) return;  // padding of the layout (the whole workgroup)
@@ -1044,21 +1054,14 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
     const int n0 = uni(it->v0), n = uni(it->v1), part = uni(it->part);  // the owned points it takes
     const size_t base = (size_t)uni(a.sy_base[pos]);
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    // slots per group copy (r + k < S), the copies, and this lane's group and offset:
-    // C * S <= 128 + 2m <= kSymSlots below 64 targets, S = m + 64 <= kSymSlots above
-    const int S = m < 64 ? 2 * m : m + 64, C = m < 64 ? (64 + m - 1) / m : 1;
-    const int gc = lane / m, gr = lane - gc * m;
     const size_t ns = (size_t)a.n_ps;
-    for (int i = tid; i < S; i += kSymBlock) {
-        const int j = b + (i < m ? i : i - m);
-        SymTarget t;
-        t.x = a.tp.x[j]; t.y = a.tp.y[j]; t.z = a.tp.z[j];
-        t.v0 = a.pdens[j];
-        t.v1 = R > 1 ? a.pdens[ns + j] : 0.0;
-        t.v2 = R > 1 ? a.pdens[2 * ns + j] : 0.0;
-        tg[i] = t;
+    for (int i = tid; i < m + 64; i += kSymBlock) {
+        const int j = b + i % m;
+        tg[NT * i] = double2{a.tp.x[j], a.tp.y[j]};
+        tg[NT * i + 1] = double2{a.tp.z[j], a.pdens[j]};
+        if (R > 1) tg[NT * i + 2] = double2{a.pdens[ns + j], a.pdens[2 * ns + j]};
     }
-    for (int i = tid; i < NW * 3 * kSymSlots; i += kSymBlock) (&facc[0][0])[i] = 0.0;
+    for (int i = tid; i < NW * R * S; i += kSymBlock) facc[i] = 0.0;
     // the box of the leaf's points (one per thread: m <= kSymBlock)
     static_assert(kSymLeafMax <= kSymBlock, "one target per thread");
     __shared__ double wbox[NW][6];
@@ -1085,14 +1088,14 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
             bx[3 + c] = fmax(bx[3 + c], wbox[v][3 + c]);
         }
     }
-    double* fa = facc[w] + gc * S;
+    double* fa = facc + w * R * S;
     constexpr int PB = 64 * kSymSrc;  // stream positions per wave block
     for (int p0 = n0 + w * PB; p0 < n; p0 += NW * PB) {
         SymSource<T> sv[kSymSrc];
         int close = 0;
         for (int u = 0; u < kSymSrc; u++) sym_load<R>(sv[u], p0 + 64 * u + lane, n, e0, e1, a, bx, close);
-        if (__ballot(close) != 0ull) sym_block<KID, T, true>(sv, tg, fa, m, gr, kc.u2);
-        else sym_block<KID, T, false>(sv, tg, fa, m, gr, kc.u2);
+        if (__ballot(close) != 0ull) sym_block<KID, T, true>(sv, tg, fa, m, kc.u2);
+        else sym_block<KID, T, false>(sv, tg, fa, m, kc.u2);
         for (int u = 0; u < kSymSrc; u++) {
             const int p = p0 + 64 * u + lane;
             if (p >= n) continue;
@@ -1109,11 +1112,7 @@ __global__ __launch_bounds__(kSymBlock) void k_leaf_sym(LeafStage a, KC<T> kc, d
         const int q = o / m, i = o - q * m;
         double s = 0;
         for (int v = 0; v < NW; v++)
-            for (int c = 0; c < C; c++) {
-                const double* f = &facc[v][q * kSymSlots + c * S];
-                s += f[i];
-                if (i + m < S) s += f[i + m];
-            }
+            for (int t = i; t < m + 64; t += m) s += facc[(v * S + t) * R + q];
         if (part >= 0) {  // k_sym_gather adds the leaf's chunks
             a.sy_part_buf[(size_t)part + o] = s;
             continue;
@@ -1873,9 +1872,12 @@ static void leaf_launch(bool adj, bool fast, const LeafStage& a, const KConst& c
             TBEM_REQUIRE((KID == K_EU || KID == K_LS) && fast, TBEM_E_INVALID,
                          "symmetric pairs: Kelvin U and the Laplace single layer only");
             if (a.n_sy_items > 0) {
-                if constexpr (KID == K_EU || KID == K_LS)
-                    hipLaunchKernelGGL((k_leaf_sym<KID, T>), dim3(a.n_sy_items), dim3(kSymBlock), 0, s, a, kc,
+                if constexpr (KID == K_EU || KID == K_LS) {
+                    constexpr int R = kernel_dim(KID);
+                    const size_t shm = (size_t)a.sy_slots * (2 * kSymRecord<R> + R * (kSymBlock / 64)) * sizeof(double);
+                    hipLaunchKernelGGL((k_leaf_sym<KID, T>), dim3(a.n_sy_items), dim3(kSymBlock), shm, s, a, kc,
                                        scale);
+                }
                 TBEM_LAUNCH_CHECK();
             }
             if (a.n_sg > 0) {
