@@ -19,6 +19,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <shared_mutex>
 #include <type_traits>
 
@@ -134,6 +135,7 @@ struct FmmPlan {
     size_t tr_y = 0;             // their largest per-pair output, in doubles (a per-handle buffer)
     // GEMM tiles of the C2E products: the cells each stage writes
     CellTiles t_p2m, t_m2l, t_p2l;
+    CellTiles t_src;                       // every source cell (mixed precision)
     std::vector<CellTiles> t_m2m;          // by source level: the M2M parents
     std::vector<CellTiles> t_olev;         // every cell of each observation level
     double p2p_pairs = 0;
@@ -1196,6 +1198,11 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     auto note_y = [&](const M2lMfma& M) {
         if (M.enabled) P->tr_y = std::max(P->tr_y, (size_t)M.y_pairs * M.ystride);
     };
+    if (P->precision == TBEM_MIXED) {
+        std::vector<int> all(ST.n_cells);
+        std::iota(all.begin(), all.end(), 0);
+        P->t_src = make_cell_tiles(all, ST, s);
+    }
     P->m2m.resize(ST.n_levels);
     P->t_m2m.resize(ST.n_levels);
     P->m2m_ops.resize(ST.n_levels);
@@ -1382,12 +1389,10 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     mark(1);
     if constexpr (!std::is_same<typename std::decay<F>::type, std::nullptr_t>::value) after_gather();
 
-    // the up-check potentials of a stage's cells -> equivalent densities, and, for
-    // the MFMA M2L, the modal FP32 input Bu * check
+    // the up-check potentials of a stage's cells -> equivalent densities
     auto up_c2e = [&](const CellTiles& T) {
         if (P.fuse_c2e) return;  // done by the stage
         launch_level_gemm(T, P.blk, P.uc2e.p, false, W.fld.p, nullptr, W.mult.p, nullptr, false, s);
-        if (mfma) launch_level_gemm(T, P.blk, P.m2l_mfma.Bu.p, false, W.fld.p, nullptr, nullptr, W.chk_up.p, false, s);
     };
     // down-check potentials -> added to the down-equivalent densities
     auto down_c2e = [&](const CellTiles& T) {
@@ -1430,6 +1435,10 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         }
         up_c2e(P.t_m2m[L]);
     }
+    // for the FP32 M2L, its modal input Bu * check of every cell (fld still holds all of them):
+    // one launch, not one beside each level's UC2E, which a small problem's chain of levels
+    // waits for (9,102 points: five launches of 7 us)
+    if (mfma) launch_level_gemm(P.t_src, P.blk, P.m2l_mfma.Bu.p, false, W.fld.p, nullptr, nullptr, W.chk_up.p, false, s);
     mark(3);
 
     // M2L (cpp/fmm.cpp:362-382) and P2L (cpp/fmm.cpp:296-330) into locals
@@ -1703,7 +1712,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
         if (!fuse) launch_level_gemm(P.t_olev[L], P.blk, P.dc2e.p, true, W.lbar.p, nullptr, W.cbar.p, nullptr, false, s);
         if (L == 0) break;
         if (P.l2l_ops[L].enabled) {  // lbar[parent] += sum over its children of K^T cbar[child]
-            m2l_adjoint64(P.l2l_ops[L], W.cbar.p, W.ty.p, W.lbar.p, s);
+            m2l_adjoint64(P.l2l_ops[L], P.l2l[L].cell.p, W.cbar.p, W.ty.p, W.lbar.p, s);
             continue;
         }
         SurfStage l = surf_base(P);
@@ -1723,7 +1732,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
     } else if (P.m2l_mfma.enabled && P.m2l_mfma.fp64) {
         // FP64 class operators: mbar[s] += sum over the pairs of s of K_c^T cbar[t]
         YLease y(P, s);
-        m2l_adjoint64(P.m2l_mfma, W.cbar.p, P.m2l_y64.p, W.mbar.p, s);
+        m2l_adjoint64(P.m2l_mfma, P.m2l.cell.p, W.cbar.p, P.m2l_y64.p, W.mbar.p, s);
     } else {
         SurfStage m = surf_base(P);
         set_list(m, A.m2l);
@@ -1748,7 +1757,7 @@ static void adjoint_T(const FmmPlan& P, Work& W, const double* g, double* xbar, 
                               false, s);
         if (L + 1 >= P.st.n_levels) break;
         if (P.m2m_ops[L].enabled) {  // mbar[child] += K^T ebar[parent]
-            m2l_adjoint64(P.m2m_ops[L], W.ebar.p, W.ty.p, W.mbar.p, s);
+            m2l_adjoint64(P.m2m_ops[L], P.m2m[L].cell.p, W.ebar.p, W.ty.p, W.mbar.p, s);
             continue;
         }
         SurfStage c = surf_base(P);

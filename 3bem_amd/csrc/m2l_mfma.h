@@ -41,6 +41,9 @@ struct M2lMfma {
     int n_adj = 0;          // transpose: source cells with pairs, and their pairs (CSR)
     DevBuf<int> adj_items, adj_ptr, adj_pairs;
     CellTiles adj_tiles;    // adj_items as GEMM tiles
+    // every target (transpose: source) cell is in one pair, as L2L's and M2M^T's are: its
+    // product needs no sum and goes straight to the cell
+    bool one = false, adj_one = false;
     double plan_seconds = 0;
 };
 
@@ -82,6 +85,6 @@ void m2l_forward64(const M2lMfma& M, const int* items, const int* ptr, const int
 void m2l_adjoint32(const M2lMfma& M, const CellTiles& targets, const double* lbar, float* w, float* Y, double* z,
                    double* e2, hipStream_t s);
 // FP64 path, transpose: mbar[s] += sum over the pairs of source s of K_c^T cbar[tgt(p)].
-void m2l_adjoint64(const M2lMfma& M, const double* cbar, double* Y, double* mbar, hipStream_t s);
+void m2l_adjoint64(const M2lMfma& M, const int* pair_src, const double* cbar, double* Y, double* mbar, hipStream_t s);
 
 }  // namespace tbem

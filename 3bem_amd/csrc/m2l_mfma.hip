@@ -354,13 +354,15 @@ __device__ __forceinline__ void m2l_row_tile64(const double* __restrict__ A, con
 // The FP64 MFMA leaves D[4*r + lq][lr] in register r of lane (lq, lr) (not the f32
 // 16x16x4 order). The staged columns are its A operand and the operator's rows its B
 // operand (the same lane layout), so Y[pair ct*16 + 4*r + lq][rt*16 + lr] = D[4*r + lq][lr]
-// and the 16 lanes lr write 128 contiguous bytes of a pair.
+// and the 16 lanes lr write 128 contiguous bytes of a pair. With dst, a pair's row goes to
+// row dst[pair] of Y (= or += with add; ystride = n there) and not to its own.
 template <int NW, int kPre>
 __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, int ystride,
                                                      const double* __restrict__ S, const int* __restrict__ ucls,
                                                      const int* __restrict__ uoff, const int* __restrict__ ucnt,
                                                      const int* __restrict__ colpair, const int* __restrict__ pair_src,
-                                                     int ybase, const double* __restrict__ x, double* __restrict__ Y) {
+                                                     int ybase, const double* __restrict__ x, double* __restrict__ Y,
+                                                     const int* __restrict__ dst, int add) {
     extern __shared__ double Bd[];  // [kt*4][kUnitCols64]
     const int u = blockIdx.x;
     const int cls = uni(ucls[u]), off = uni(uoff[u]), cnt = uni(ucnt[u]);
@@ -370,6 +372,11 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
     // waves stride over the k-steps
     constexpr int RPW = 64 / kUnitCols64;  // k-steps per wave and pass
     const int c = lane % kUnitCols64, h = lane / kUnitCols64;
+    // (the first row tile's first k-steps are on their way meanwhile)
+    const double* Acls = S + (size_t)cls * mt * kt * 64 + lane;
+    const int rt0 = blockIdx.y * NW + wave, step = gridDim.y * NW;
+    double cur[kPre];
+    for (int i = 0; i < kPre; i++) cur[i] = (rt0 < mt && i < kt) ? Acls[((size_t)rt0 * kt + i) * 64] : 0.0;
     const double* col = c < cnt ? x + (size_t)pair_src[colpair[off + c]] * n : nullptr;
     stage_quads<double>(col, n, kt, RPW * wave + h, RPW * NW, [&](int q, int i, double v) {
         Bd[(4 * q + i) * kUnitCols64 + c] = v;
@@ -380,18 +387,14 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
     const double* b = Bd + lq * kUnitCols64 + lr;
     constexpr int MAXCT = kUnitCols64 / 16;
     const int nct = (cnt + 15) / 16;  // 1 .. MAXCT (uniform)
-    const double* Acls = S + (size_t)cls * mt * kt * 64 + lane;
     int yp[MAXCT][4];  // the lane's pairs' rows of Y (-1: none)
 #pragma unroll
     for (int ct = 0; ct < MAXCT; ct++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int nn = ct * 16 + 4 * r + lq;
-            yp[ct][r] = nn < cnt ? colpair[off + nn] - ybase : -1;
+            yp[ct][r] = nn >= cnt ? -1 : dst ? dst[colpair[off + nn]] : colpair[off + nn] - ybase;
         }
-    const int rt0 = blockIdx.y * NW + wave, step = gridDim.y * NW;
-    double cur[kPre];
-    for (int i = 0; i < kPre; i++) cur[i] = (rt0 < mt && i < kt) ? Acls[((size_t)rt0 * kt + i) * 64] : 0.0;
     for (int rt = rt0; rt < mt; rt += step) {
         f64x4 acc[MAXCT] = {};
         const double* A = Acls + (size_t)rt * kt * 64;
@@ -403,8 +406,12 @@ __global__ __launch_bounds__(NW * 64) void k_m2l_mfma64(int n, int mt, int kt, i
 #pragma unroll
         for (int ct = 0; ct < MAXCT; ct++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (yp[ct][r] >= 0) Y[(size_t)yp[ct][r] * ystride + rt * 16 + lr] = acc[ct][r];
+            for (int r = 0; r < 4; r++) {
+                const int row = rt * 16 + lr;
+                if (yp[ct][r] < 0 || (dst && row >= n)) continue;
+                double* o = Y + (size_t)yp[ct][r] * ystride + row;
+                *o = add ? *o + acc[ct][r] : acc[ct][r];
+            }
     }
 }
 
@@ -911,8 +918,11 @@ void build_m2l_mfma(M2lMfma& M, int kid, const KConst& kc, const HostTree& ot, c
         M.n_adj = na;
         M.adj_tiles = make_cell_tiles(adj_items, st, s);
         M.adj_pairs = std::move(spairs);
+        M.adj_one = na == n_pairs;
     }
     TBEM_HIP(hipStreamSynchronize(s));
+    M.one = true;
+    for (size_t k = 0; k + 1 < m2l.ptr.size(); k++) M.one = M.one && m2l.ptr[k + 1] - m2l.ptr[k] == 1;
     M.enabled = true;
     M.plan_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
 }
@@ -972,9 +982,10 @@ static void mfma32_slice(const M2lMfma& M, int q, const int* pair_src, const flo
 // 12 us (9,102 points).
 constexpr int kUnitsFill = 1024;
 
-// Y (slice q) = K_c * x[src(p)] (transpose: K_c^T * x[tgt(p)]), FP64 MFMA
+// Y (slice q) = K_c * x[src(p)] (transpose: K_c^T * x[tgt(p)]), FP64 MFMA; with dst, row
+// dst[p] of Y (blk values each) = or += (add) the pair's product
 static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const double* x, double* Y, bool transpose,
-                         hipStream_t s) {
+                         hipStream_t s, const int* dst = nullptr, bool add = false) {
     const SliceUnits U = slice_units(M, q);
     if (U.n == 0) return;
     const size_t shm = staged_bytes(M.blk, true);
@@ -982,19 +993,18 @@ static void mfma64_slice(const M2lMfma& M, int q, const int* pair_src, const dou
     const int* src = transpose ? M.pair_tgt.p : pair_src;
     const int nw = 3 * shm > kLdsPerCu ? kWaves64 : narrow_waves(M.mt);
     const dim3 g(U.n, std::max(1, std::min(div_up(M.mt, nw), kUnitsFill / U.n)));
-    if (nw == kWaves64)
-        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64, kPre64>), g, dim3(kWaves64 * 64), shm, s, M.blk, M.mt,
-                           M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
-    else if (nw == 5)
-        hipLaunchKernelGGL((k_m2l_mfma64<5, kPre64Narrow>), g, dim3(320), shm, s, M.blk, M.mt, M.kt,
-                           M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
-    else if (nw == 3)
-        hipLaunchKernelGGL((k_m2l_mfma64<3, kPre64Narrow>), g, dim3(192), shm, s, M.blk, M.mt, M.kt,
-                           M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x, Y);
-    else
-        hipLaunchKernelGGL((k_m2l_mfma64<kWaves64Narrow, kPre64Narrow>), g, dim3(kWaves64Narrow * 64), shm,
-                           s, M.blk, M.mt, M.kt, M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src,
-                           M.slice_pairs[q], x, Y);
+    auto launch = [&](auto waves, auto pre) {
+        constexpr int NW = decltype(waves)::value;
+        hipLaunchKernelGGL((k_m2l_mfma64<NW, decltype(pre)::value>), g, dim3(NW * 64), shm, s, M.blk, M.mt, M.kt,
+                           dst ? M.blk : M.ystride, S, U.ucls, U.uoff, U.ucnt, M.colpair.p, src, M.slice_pairs[q], x,
+                           Y, dst, add ? 1 : 0);
+    };
+    using std::integral_constant;
+    const integral_constant<int, kPre64Narrow> narrow{};
+    if (nw == kWaves64) launch(integral_constant<int, kWaves64>{}, integral_constant<int, kPre64>{});
+    else if (nw == 5) launch(integral_constant<int, 5>{}, narrow);
+    else if (nw == 3) launch(integral_constant<int, 3>{}, narrow);
+    else launch(integral_constant<int, kWaves64Narrow>{}, narrow);
     TBEM_LAUNCH_CHECK();
 }
 
@@ -1049,9 +1059,10 @@ void m2l_forward64(const M2lMfma& M, const int* items, const int* ptr, const int
                    double* Y, double* fld, hipStream_t s, hipEvent_t kernel_end, unsigned long long* stamp) {
     if (!M.enabled || !M.fp64) return;
     for (int q = 0; q < M.n_slices; q++) {
-        mfma64_slice(M, q, pair_src, mult, Y, false, s);
+        if (M.one) mfma64_slice(M, q, pair_src, mult, fld, false, s, M.pair_tgt.p);
+        else mfma64_slice(M, q, pair_src, mult, Y, false, s);
         if (kernel_end && q + 1 == M.n_slices) TBEM_HIP(hipEventRecord(kernel_end, s));
-        forward_sum_slice<double>(M, q, items, ptr, Y, fld, s, q + 1 == M.n_slices ? stamp : nullptr);
+        if (!M.one) forward_sum_slice<double>(M, q, items, ptr, Y, fld, s, q + 1 == M.n_slices ? stamp : nullptr);
     }
 }
 
@@ -1066,9 +1077,13 @@ void m2l_adjoint32(const M2lMfma& M, const CellTiles& targets, const double* lba
     if (M.n_adj > 0) launch_level_gemm(M.adj_tiles, M.blk, M.Bu.p, true, z, nullptr, e2, nullptr, false, s);
 }
 
-void m2l_adjoint64(const M2lMfma& M, const double* cbar, double* Y, double* mbar, hipStream_t s) {
+void m2l_adjoint64(const M2lMfma& M, const int* pair_src, const double* cbar, double* Y, double* mbar, hipStream_t s) {
     if (!M.enabled || !M.fp64) return;
     for (int q = 0; q < M.n_slices; q++) {
+        if (M.adj_one) {
+            mfma64_slice(M, q, nullptr, cbar, mbar, true, s, pair_src, true);
+            continue;
+        }
         mfma64_slice(M, q, nullptr, cbar, Y, true, s);
         adjoint_sum_slice<double>(M, q, Y, mbar, true, s);
     }
