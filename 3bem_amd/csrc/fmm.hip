@@ -1368,6 +1368,8 @@ static void set_list(SurfStage& a, const DevList& l) {
     a.rcnt = l.rcnt.p;
     a.rpre = l.rpre.p;
     a.order = l.by_work.p;
+    a.longest = l.longest;
+    a.n_cells = l.n_cells;
 }
 
 // gather, upward pass, M2L/P2L and L2L: everything the leaf stage consumes. FP64,

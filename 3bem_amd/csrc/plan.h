@@ -127,7 +127,8 @@ struct HostList {
     std::vector<int> items, ptr, cell, rbeg, rcnt, rpre;
 };
 struct DevList {
-    int n_items = 0;
+    int n_items = 0, longest = 0;  // longest: the most cells of an item
+    size_t n_cells = 0;
     DevBuf<int> items, ptr, cell, rbeg, rcnt, rpre;
     DevBuf<int> by_work; // item indices, the most cells first (order_by_work; empty: as listed)
     DevBuf<int> rclose;  // point-range lists of the point-target stage: launch_range_close

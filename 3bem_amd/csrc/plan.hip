@@ -94,6 +94,9 @@ void DevList::order_by_work(const std::vector<int>& p, hipStream_t s) {
 }
 
 void DevList::upload(const HostList& l, hipStream_t s) {
+    longest = 0;
+    n_cells = l.cell.size();
+    for (size_t k = 0; k + 1 < l.ptr.size(); k++) longest = std::max(longest, l.ptr[k + 1] - l.ptr[k]);
     n_items = (int)l.items.size();
     items.upload(l.items, s);
     ptr.upload(l.ptr, s);

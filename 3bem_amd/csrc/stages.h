@@ -105,6 +105,8 @@ struct SurfStage {
     int n_e, blk;
     double* out;            // blk per cell of tt: the raw check potentials (= or += with add)
     const int* order;       // the items' launch order (null: as listed), the most work first
+    int longest;            // surface sources: the most cells of an item, and of all of them
+    size_t n_cells;
     // With c2e given (operators of at most kSurfBlock rows), the check-to-equivalent product of
     // the cell's potentials follows in the same launch instead of the store to out:
     // c2e_out[cell] (= or += with c2e_add) C field, field first added to out[cell] with add;

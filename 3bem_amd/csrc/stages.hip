@@ -572,6 +572,108 @@ __global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double
     }
 }
 
+// The same sums again where few items, or a few long ones, leave the chip idle behind one
+// lane's chain of sources: the elastic kernels' surface sources. An item's targets go to
+// surf_parts(n_e) workgroups of at most 64 targets, and the four waves of each take every
+// fourth source of a chunk; what a source adds to a target goes to LDS, and one thread per
+// target and component adds the chunk in source order (slice by slice, as k_surf_one's lanes
+// do), so that the sums keep their bits. The traction and hypersingular kernels add a value
+// by a plain add; Kelvin U adds ri w in one FMA, so ri goes along. Two chunk buffers: one
+// barrier per chunk. Bound: vector issue, with the LDS round trip of a source beside its 50
+// instructions; chunks of eight sources, so that registers (128) and LDS (35 KB) leave four
+// waves per SIMD (chunks of 16 at two waves: 1427 us where this takes 1026).
+// (Rule: surf_launch.)
+template <int KID>
+constexpr int split_values() {
+    return KID == K_EU ? 4 : 3;
+}
+constexpr bool has_split(int kid) { return kid == K_EU || kid == K_ET || kid == K_EA || kid == K_EH; }
+static int surf_parts(int n_e) { return (n_e + 63) / 64; }
+
+template <int KID, bool ADJ, bool CUT>
+__global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> kc, double scale, int S, int add, int parts) {
+    constexpr int R = kernel_dim(KID), NV = split_values<KID>(), C = 8;
+    constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
+    static_assert(R == 3, "one wave per component adds");
+    __shared__ Tile<double, R, NRM, kSurfBlock> st;
+    __shared__ double inc[2][C][NV][64];
+    const int at = blockIdx.x / parts;  // an item's parts side by side, the longest items first
+    const int item = a.order ? uni(a.order[at]) : at;
+    const int cell = uni(a.items[item]);
+    const double rc = a.tt.level_r[uni(a.tt.level[cell])];
+    const int e0 = uni(a.ptr[item]), e1 = uni(a.ptr[item + 1]);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, n_e = a.n_e;
+    const int T = (n_e + parts - 1) / parts, t0 = (blockIdx.x % parts) * T;
+    const bool mine = lane < T && t0 + lane < n_e;
+    const int tg = mine ? t0 + lane : 0;
+    double p[3];
+    moved(rc, a.t_surf + 3 * tg, a.tt.cx[cell], a.tt.cy[cell], a.tt.cz[cell], p);
+    const double tn[3] = {a.unit[3 * tg], a.unit[3 * tg + 1], a.unit[3 * tg + 2]};
+    drain_loads();
+    // source j's addend(s) to the lane's target
+    auto values = [&](int j, double (*o)[64]) {
+        if constexpr (KID == K_EU) {
+            const double v[3] = {st.d[0][j], st.d[1][j], st.d[2][j]};
+            const double dx = ADJ ? p[0] - st.x[j] : st.x[j] - p[0];
+            const double dy = ADJ ? p[1] - st.y[j] : st.y[j] - p[1];
+            const double dz = ADJ ? p[2] - st.z[j] : st.z[j] - p[2];
+            const double r2 = dx * dx + dy * dy + dz * dz;
+            double ri = rsqrt_t(r2);
+            if constexpr (CUT) ri = (r2 < cutoff_r2<double>()) ? 0.0 : ri;
+            const double ri2 = ri * ri;
+            const double dv = dx * v[0] + dy * v[1] + dz * v[2];
+            const double t = dv * ri2;
+            o[0][lane] = mul_rounded(kc.u2, v[0]) + dx * t;
+            o[1][lane] = mul_rounded(kc.u2, v[1]) + dy * t;
+            o[2][lane] = mul_rounded(kc.u2, v[2]) + dz * t;
+            o[3][lane] = ri;
+        } else {
+            double x[3] = {-0.0, -0.0, -0.0};  // -0 + v is v
+            pair<KID, ADJ, false, CUT, true>(st, j, p[0], p[1], p[2], tn, x, kc);
+            o[0][lane] = x[0];
+            o[1][lane] = x[1];
+            o[2][lane] = x[2];
+        }
+    };
+    double acc[3] = {0.0, 0.0, 0.0};  // component w of the lane's target, per slice (S <= 3)
+    int buf = 0;
+    auto plus = [&](double s, int jj) {
+        if constexpr (KID == K_EU) return fma(inc[buf][jj][NV - 1][lane], inc[buf][jj][w][lane], s);
+        else return s + inc[buf][jj][w][lane];
+    };
+    auto compute = [&](int cnt) {
+        for (int c0 = 0; c0 < cnt; c0 += C) {
+            const int n = min(C, cnt - c0);
+#pragma unroll
+            for (int i = 0; i < C / 4; i++)
+                if (w + 4 * i < n) values(c0 + w + 4 * i, inc[buf][w + 4 * i]);
+            __syncthreads();
+            if (w < R) {
+                if (S == 1 && n == C) {
+#pragma unroll
+                    for (int jj = 0; jj < C; jj++) acc[0] = plus(acc[0], jj);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 3; k++)  // slice k: the tile's sources k, k + S, ..
+                        if (k < S)
+                            for (int jj = (k + S - c0 % S) % S; jj < n; jj += S) acc[k] = plus(acc[k], jj);
+                }
+            }
+            buf ^= 1;
+        }
+    };
+    stream_surfaces(st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
+    if (w < R && mine) {
+        double s = 0;
+        s += acc[0];
+        if (S > 1) s += acc[1];
+        if (S > 2) s += acc[2];
+        s *= scale;
+        double* o = a.out + (size_t)cell * a.blk + w * n_e + tg;
+        *o = add ? *o + s : s;
+    }
+}
+
 // -------------------------------------------------------------------- point targets
 // Two targets per lane: slot tg holds targets t0+tg and t0+nslot+tg. Point
 // sources accumulate in T (acA, acB); surface sources in FP64 (sfA, sfB, which
@@ -1800,6 +1902,14 @@ KC<double> kc_of<double>(const KConst& c) { return make_kc64(c); }
 template <>
 KC<float> kc_of<float>(const KConst& c) { return make_kc32(c); }
 
+// k_surf_one takes as long as its longest item's waves, or as all its waves take on the chip's
+// SIMDs: k_surf_split, a quarter more work but 1/4 of the chain and finer pieces, where the
+// first is kSurfSplit times the second. Traction, order 150: 454 items of up to 74 cells, 13,546
+// cells, M2L 1466 -> 1026 us, transposed 1306 -> 965; L2L^T and M2M (eight cells an item, up to
+// 256 items) 404 -> 270 us for five levels; the whole pass, both directions and gradient, 5356
+// -> 4330 us. Items of equal length that fill the chip stay (M2M of a deep tree's lowest level).
+constexpr double kSurfSimds = 1024, kSurfSplit = 1.3;
+
 template <int KID, class T>
 static void surf_launch(bool src_surf, bool add, bool adj, const SurfStage& a, const KConst& c, hipStream_t s) {
     if (a.n_items == 0) return;
@@ -1811,6 +1921,22 @@ static void surf_launch(bool src_surf, bool add, bool adj, const SurfStage& a, c
         const int S = kSurfBlock / ((a.n_e + 1) / 2);
         const dim3 w(div_up((size_t)a.n_e * S, 64) * 64);
         const int ad = add ? 1 : 0;
+        if constexpr (has_split(KID)) {
+            if (src_surf && (double)a.longest * kSurfSimds > kSurfSplit * (double)a.n_cells * (w.x / 64)) {
+                const int parts = surf_parts(a.n_e);
+                const dim3 gp((unsigned)a.n_items * parts), bp(256);
+                if (a.no_cutoff && !adj) hipLaunchKernelGGL((k_surf_split<KID, false, false>), gp, bp, 0, s, a, kc, scale, S, ad,
+                                   parts);
+                else if (a.no_cutoff) hipLaunchKernelGGL((k_surf_split<KID, true, false>), gp, bp, 0, s, a, kc, scale, S, ad,
+                                   parts);
+                else if (!adj) hipLaunchKernelGGL((k_surf_split<KID, false, true>), gp, bp, 0, s, a, kc, scale, S, ad,
+                                   parts);
+                else hipLaunchKernelGGL((k_surf_split<KID, true, true>), gp, bp, 0, s, a, kc, scale, S, ad,
+                                   parts);
+                TBEM_LAUNCH_CHECK();
+                return;
+            }
+        }
         if (src_surf && a.no_cutoff && !adj)
             hipLaunchKernelGGL((k_surf_one<KID, true, false, false>), g, w, 0, s, a, kc, scale, S, ad);
         else if (src_surf && a.no_cutoff)
