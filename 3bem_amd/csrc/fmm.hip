@@ -782,23 +782,26 @@ static std::vector<I> xcd_layout(const std::vector<std::pair<long, I>>& items, i
     constexpr int kXcds = 8;
     long total = 0;
     for (const auto& it: items) total += it.first;
-    std::vector<std::vector<std::pair<int, I>>> run(kXcds);
+    std::vector<std::vector<const std::pair<long, I>*>> run(kXcds);
     long acc = 0;
     for (const auto& it: items) {
         const int x = total > 0 ? (int)std::min<long>(kXcds - 1, (acc * kXcds) / total) : 0;
-        int cls = 0;
-        for (long w = it.first; w > 1; w >>= 1) cls++;
-        run[x].push_back({cls, it.second});
+        run[x].push_back(&it);
         acc += it.first;
     }
     size_t groups = 0;
-    for (auto& r: run) {
-        std::stable_sort(r.begin(), r.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
-        groups = std::max(groups, (r.size() + g - 1) / g);
-    }
+    for (const auto& r: run) groups = std::max(groups, (r.size() + g - 1) / g);
     std::vector<I> out(groups * kXcds * g, empty);
-    for (int x = 0; x < kXcds; x++)
-        for (size_t i = 0; i < run[x].size(); i++) out[((i / g) * kXcds + x) * g + i % g] = run[x][i].second;
+    auto cls = [](long w) { return w > 1 ? 63 - __builtin_clzl((unsigned long)w) : 0; };
+    for (int x = 0; x < kXcds; x++) {
+        size_t at[65] = {};  // the first place of each class, highest class first
+        for (const auto* it: run[x]) at[63 - cls(it->first) + 1]++;
+        for (int c = 1; c < 65; c++) at[c] += at[c - 1];
+        for (const auto* it: run[x]) {
+            const size_t i = at[63 - cls(it->first)]++;
+            out[((i / g) * kXcds + x) * g + i % g] = it->second;
+        }
+    }
     return out;
 }
 
@@ -808,8 +811,9 @@ constexpr long kBlockFill = 8192, kBlockCapMin = 16384;
 
 static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
                          const HostList& surf, int n_e, int block_tile, LeafSplit& out, hipStream_t s) {
-    std::vector<std::pair<long, WaveItem>> w, bi;
+    std::vector<std::pair<long, WaveItem>> w, bi, ch;
     std::vector<std::pair<long, int>> b;
+    w.reserve(leaves.size());
     std::vector<WaveLeafParts> wparts, bparts;
     auto points_of = [&](size_t k) {
         const int p0 = pts.ptr.empty() ? 0 : pts.ptr[k], p1 = pts.ptr.empty() ? 0 : pts.ptr[k + 1];
@@ -853,7 +857,7 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
             }
             continue;
         }
-        std::vector<std::pair<long, WaveItem>> ch;
+        ch.clear();
         const auto pre = pts.rpre.begin();
         for (long run = 0; run < np; run += per)
             for (long v = run, end = std::min(np, run + per); v < end; v += sub) {
