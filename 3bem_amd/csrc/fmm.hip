@@ -1893,7 +1893,8 @@ static std::array<double, kStamps> stamps_ms(Work& W) {
     const std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
     std::array<double, kStamps> t{};
     const int order[kStamps] = {0, 1, 2, 3, 8, 9, 4, 5, 6, 7};
-    double next = 0;
+    // (a gradient's own far field ends without a leaf stage: the last stamp stands for the rest)
+    double next = (double)(long long)(*std::max_element(raw.begin(), raw.end()) - raw[0]) / W.ts_per_ms;
     for (int i = kStamps - 1; i >= 0; i--) {
         const int k = order[i];
         if (raw[k]) next = (double)(long long)(raw[k] - raw[0]) / W.ts_per_ms;

@@ -318,10 +318,11 @@ int tbem_nbody_apply_dev(tbem_nbody_t h, const double* d_x, double* d_y, void* s
  * allocating library call). No counterpart in the reference: it is for callers that
  * cannot allocate device memory, such as code under HIP graph capture, tight
  * serving loops and harnesses that forbid allocation. The weighted source
- * densities are staged in a static device array of 4,194,304 doubles (32 MiB) that
- * each GPU the library runs on holds until the process ends: R * n_src above that
+ * densities are staged in a static device array of 4,194,304 doubles (32 MiB), the
+ * sums of the source parts in another of 2,097,152, that each GPU the library runs on
+ * holds until the process ends: R * n_src above the first
  * returns TBEM_E_UNSUPPORTED. The current device must be the handle's. Every call
- * on one GPU shares that array, so calls that overlap on one GPU (on different
+ * on one GPU shares these arrays, so calls that overlap on one GPU (on different
  * streams, or through different handles) race; calls ordered on one stream do
  * not. Same outputs as tbem_nbody_apply_dev, bit for bit. */
 int tbem_nbody_apply_noalloc(tbem_nbody_t h, const double* d_x, double* d_y, void* stream);
