@@ -1231,19 +1231,27 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     const bool fp64_classes = (P->precision == TBEM_FP64 || !m2l_mfma_size_ok(P->blk)) &&
                               d->translations == TBEM_TRANSLATIONS_AUTO && P->tree_layout != kTreesOwnBoxes &&
                               m2l_fp64_classes_pay(P->kid, P->n_e, m2l_h.cell.size());
-    if (P->precision == TBEM_MIXED || fp64_classes)
-        build_m2l_mfma(P->m2l_mfma, P->kid, P->kc, OT, ST, P->dot, P->dst, P->tree_layout != kTreesOwnBoxes,
-                       fp64_classes, d->m2l_output_budget ? d->m2l_output_budget : kM2lOutputBudget, m2l_h, P->m2l,
-                       P->surf, P->uc2e.p, P->dc2e.p, s, up_fac, down_fac);
+    try {
+        if (P->precision == TBEM_MIXED || fp64_classes)
+            build_m2l_mfma(P->m2l_mfma, P->kid, P->kc, OT, ST, P->dot, P->dst, P->tree_layout != kTreesOwnBoxes,
+                           fp64_classes, d->m2l_output_budget ? d->m2l_output_budget : kM2lOutputBudget, m2l_h, P->m2l,
+                           P->surf, P->uc2e.p, P->dc2e.p, s, up_fac, down_fac);
+        if (P->m2l_mfma.enabled) {
+            const size_t ny = (size_t)P->m2l_mfma.y_pairs * P->m2l_mfma.ystride;
+            if (P->m2l_mfma.fp64) P->m2l_y64.alloc(ny);
+            else P->m2l_y.alloc(ny);
+        }
+    } catch (const Error& e) {
+        // no memory for the class operators of a size that the surfaces serve too
+        if (e.code != TBEM_E_NOMEM || !fp64_classes || m2l_mfma_size_ok(P->blk)) throw;
+        (void)hipGetLastError();
+        P->m2l_mfma = M2lMfma{};
+        P->m2l_y64.release();
+    }
     clk.mark("m2l_mfma");
     TBEM_HIP(hipEventCreateWithFlags(&P->y_done, hipEventDisableTiming));
     TBEM_HIP(hipEventRecord(P->y_done, s));
     if (!P->m2l_mfma.enabled) P->m2l.order_by_work(m2l_h.ptr, s);
-    if (P->m2l_mfma.enabled) {
-        const size_t ny = (size_t)P->m2l_mfma.y_pairs * P->m2l_mfma.ystride;
-        if (P->m2l_mfma.fp64) P->m2l_y64.alloc(ny);
-        else P->m2l_y.alloc(ny);
-    }
     P->d_flag.alloc(1);
     const std::vector<int> p2l_items = cells_with(tl.p2l, 0, OT.n_cells);
     P->p2l.upload(list_from_pairs(p2l_items, OT.n_cells, tl.p2l, 0, &ST), s);

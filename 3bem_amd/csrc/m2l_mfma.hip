@@ -713,10 +713,15 @@ void build_m2l_mfma(M2lMfma& M, int kid, const KConst& kc, const HostTree& ot, c
     M.ystride = mt * 16;
     M.n_pairs = n_pairs;
     if (fp64) {
-        // the FP64 operators and their transposes must fit an eighth of the device
+        // The FP64 operators and their transposes must fit an eighth of the device. Below kMinBlk
+        // rows the surfaces serve the pairs too, without any memory: there the operators and the
+        // per-pair output must also fit a quarter of what is free, so that a plan that the
+        // surfaces could run never fails for them, and the handle's own buffers find room.
         size_t free_b = 0, total_b = 0;
         TBEM_HIP(hipMemGetInfo(&free_b, &total_b));
-        if ((size_t)nc * mt * kt * 64 * 2 * sizeof(double) > total_b / 8) return;
+        const size_t ops = (size_t)nc * mt * kt * 64 * 2 * sizeof(double);
+        const size_t out = std::min((size_t)n_pairs * M.ystride * sizeof(double), y_budget);
+        if (ops > total_b / 8 || (n < kMinBlk && ops + out > free_b / 4)) return;
     }
 
     // modal factors of UC2E (source tree levels) and DC2E (observation tree levels)

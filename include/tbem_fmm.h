@@ -122,8 +122,11 @@ typedef struct {
      * tree_boxes TBEM_TREES_COMMON_BOX). Elsewhere, and everywhere with
      * TBEM_TRANSLATIONS_SURFACES, the kernel is evaluated between the two surfaces of
      * every pair, as cpp/fmm.cpp:204-251, 362-413 do. Both are FP64 throughout and
-     * differ in rounding only. TBEM_MIXED's M2L always runs on its FP32 modal
-     * operators. */
+     * differ in rounding only. Below 48 rows (R*n_e) M2M and L2L stay on the surfaces,
+     * and the M2L takes the class operators, in either precision, where they are the
+     * faster (50,000 pairs and more) and they and their output (m2l_output_budget: up
+     * to 6 GiB where the surfaces need nothing) fit a quarter of the free device
+     * memory. From 48 rows on TBEM_MIXED's M2L runs on its FP32 modal operators. */
     int translations;
 
     /* Bytes the class M2L's per-pair output may take (no reference counterpart):
