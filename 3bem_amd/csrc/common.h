@@ -24,10 +24,12 @@ void set_last_error(const std::string& msg);
 #define TBEM_HIP(call)                                                                       \
     do {                                                                                     \
         hipError_t e_ = (call);                                                              \
-        if (e_ != hipSuccess)                                                                \
+        if (e_ != hipSuccess) {                                                              \
+            (void)hipGetLastError(); /* reported here, not by the next launch's check too */ \
             throw ::tbem::Error(e_ == hipErrorOutOfMemory ? TBEM_E_NOMEM : TBEM_E_HIP,       \
                                 std::string(#call) + ": " + hipGetErrorString(e_) + " at " + \
                                     __FILE__ + ":" + std::to_string(__LINE__));              \
+        }                                                                                    \
     } while (0)
 
 #define TBEM_REQUIRE(cond, code, msg)                       \

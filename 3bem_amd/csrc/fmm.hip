@@ -1244,7 +1244,6 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
     } catch (const Error& e) {
         // no memory for the class operators of a size that the surfaces serve too
         if (e.code != TBEM_E_NOMEM || !fp64_classes || m2l_mfma_size_ok(P->blk)) throw;
-        (void)hipGetLastError();
         P->m2l_mfma = M2lMfma{};
         P->m2l_y64.release();
     }
