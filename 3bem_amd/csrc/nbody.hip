@@ -9,6 +9,7 @@
 // alone are too few for the chip, the sources are cut into parts, one workgroup per
 // (chunk, part), whose sums k_leaf_parts adds in part order (split_sources).
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 
@@ -110,17 +111,40 @@ static HostList all_pairs(const HostTree& tgt, int n_src) {
 }
 
 // The work items of one direction: every target chunk against n_src sources, the sources
-// cut into equal parts so that the launch holds about kTargetItems workgroups: the kernel
-// keeps two to three per compute unit, and several rounds of them keep the last round's
-// idle units a small share. Bound: FP64 VALU issue once the chip is filled. Measured,
-// whole chunks -> parts: hypersingular, 20,011 points (157 workgroups of four waves on
-// 256 units): 1712 -> 950 us (15.9 -> 28.6 TFLOP/s); traction, 3,000 sources and 2,003
-// targets (16 workgroups): 169 -> 30 us. A part keeps at least
-// kMinPartSources sources: below that a workgroup's fixed costs (targets, first tile,
-// slice sums) outweigh its pairs. In mixed precision parts are whole FP32 tiles
-// (kLeafBlock sources, a multiple of every instance's), so that the tiles' partial sums
-// stay what they are without parts.
-constexpr int kTargetItems = 4096, kMinPartSources = 64;
+// cut into equal parts where that pays, one workgroup per (chunk, part). In mixed precision
+// parts are whole FP32 tiles (kLeafBlock sources, a multiple of every instance's), so that
+// the tiles' partial sums stay what they are without parts. Whole chunks have no items.
+//
+// How many parts: the launch's time in units of one source on a full chunk is about
+//   rounds * (a part's sources + F) + (with parts) 100 + 3 per part,
+// rounds = workgroups / kUnits, rounded up; F, a workgroup's fixed costs (targets, first
+// tile, slice sums), 64 for the 512-thread instances and 8 for the 256-thread ones; the rest
+// the launch that adds the parts. Chunks of fewer targets count their sources in proportion.
+// Fitted to 140 sizes from 100 x 128 to 50,000 x 70,000 points and five kernels, each with 1
+// to 128 parts; whole chunks -> the model's parts, per apply: traction, 3,000 sources on 2,003
+// targets 159 -> 27 us; hypersingular, 20,011 points 1660 -> 869 us (16.4 -> 31.3 TFLOP/s);
+// double layer, 1,000 sources on 40,000 targets 72 -> 56 us; and where they do not pay,
+// 300 sources on 60,000 targets 37 us whole, 56 in the five parts that fill more workgroups.
+constexpr int kUnits = 256, kMaxParts = 1024;
+
+static int count_parts(int kid, bool mixed, int nc, int n_tgt, int n_src, int unit, size_t max_parts) {
+    if (kid == K_LH) return 1;  // no work per pair
+    const double F = leaf_stage_tile(kid, mixed) > 256 ? 64 : 8;
+    const double per_source = std::min(n_tgt, kTargetChunk) / (double)kTargetChunk;
+    int best = 1;
+    double best_cost = 0;
+    for (int np = 1; np <= std::min<size_t>(kMaxParts, std::max<size_t>(1, max_parts)); np++) {
+        const int per = div_up(div_up(n_src, np), unit) * unit;
+        if (np > 1 && per * (double)(np - 1) >= n_src) continue;  // fewer parts hold them all
+        const double rounds = std::ceil((double)nc * np / kUnits);
+        const double cost = rounds * (std::min(per, n_src) * per_source + F) + (np > 1 ? 100 + 3 * np : 0);
+        if (np == 1 || cost < best_cost) {
+            best = np;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
 
 struct Split {
     std::vector<WaveItem> h_items;  // kept: their upload may still be in flight
@@ -131,23 +155,20 @@ struct Split {
     size_t part_size = 0;
 };
 
-static void split_sources(const HostTree& tgt, int n_src, int precision, Split& out, hipStream_t s) {
+static void split_sources(const HostTree& tgt, int n_src, int kid, int precision, Split& out, hipStream_t s) {
     std::vector<WaveItem>& items = out.h_items;
     std::vector<WaveLeafParts>& parts = out.h_parts;
-    const int nc = (int)tgt.leaves.size(), unit = precision == TBEM_MIXED ? kLeafBlock : 1;
-    size_t np = std::min<size_t>(div_up(kTargetItems, nc), div_up(std::max(n_src, 1), kMinPartSources));
-    np = std::min(np, kPartDoubles / ((size_t)kPartRows * std::max(tgt.n_pts, 1)));
-    int per = np > 1 ? div_up((size_t)n_src, np) : std::max(n_src, 1);
-    per = div_up(per, unit) * unit;
+    const bool mixed = precision == TBEM_MIXED;
+    const int nc = (int)tgt.leaves.size(), unit = mixed ? kLeafBlock : 1;
+    const int np = count_parts(kid, mixed, nc, tgt.n_pts, std::max(n_src, 1), unit,
+                               kPartDoubles / ((size_t)kPartRows * std::max(tgt.n_pts, 1)));
+    const int per = div_up(div_up((size_t)std::max(n_src, 1), np), unit) * unit;
     const int n = div_up(std::max(n_src, 1), per);
+    if (n == 1) return;
     size_t part = 0;
     for (int k = 0; k < nc; k++) {
         const size_t m = tgt.count[k];
         if (m == 0) continue;
-        if (n == 1) {
-            items.push_back(WaveItem{k, 0, n_src > 0 ? 1 : 0, 0, n_src, 0, 0, 0, -1});
-            continue;
-        }
         parts.push_back(WaveLeafParts{k, (int)part, n});
         for (int p = 0; p < n; p++, part += kPartRows * m)
             items.push_back(WaveItem{k, 0, 1, p * per, std::min(n_src, (p + 1) * per), 0, 0, 0, (int)part});
@@ -218,6 +239,7 @@ static void nb_adjoint(NbodyPlan& P, const double* g, double* y, hipStream_t s) 
 }
 
 static void set_items(LeafStage& f, const Split& sp, double* parts) {
+    if (sp.n_parts == 0) return;  // whole chunks: one workgroup each, without the items' indirection
     f.split = 1;
     f.block_items = sp.items.p; f.n_block_items = sp.n_items;
     f.parts = sp.parts.p; f.n_parts = sp.n_parts;
@@ -302,8 +324,8 @@ int tbem_nbody_create(const tbem_nbody_desc* d, tbem_nbody_t* out) {
         P.adj.upload(all_pairs(P.src_t, P.n_obs), s);
         P.obs_leaves.upload(P.obs_t.leaves, s);
         P.src_leaves.upload(P.src_t.leaves, s);
-        split_sources(P.obs_t, P.n_src, P.precision, P.fwd_split, s);
-        split_sources(P.src_t, P.n_obs, P.precision, P.adj_split, s);
+        split_sources(P.obs_t, P.n_src, P.kid, P.precision, P.fwd_split, s);
+        split_sources(P.src_t, P.n_obs, P.kid, P.precision, P.adj_split, s);
         P.dens.alloc((size_t)P.R * P.n_src);
         P.parts.alloc(std::max(P.fwd_split.part_size, P.adj_split.part_size));
         TBEM_HIP(hipEventRecord(P.done, s));
