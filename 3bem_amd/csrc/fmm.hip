@@ -191,7 +191,11 @@ class YLease {
     std::unique_lock<std::mutex> lk_;
 };
 
-constexpr double kOverlapPairs = 1.2e9;  // Work::overlap
+// Work::overlap's default below 48 rows: the far field is a chain of launches long enough to
+// fill the time of the point pairs (four levels or more; with fewer, operators of at least
+// kOverlapRows and kOverlapMin pairs), and the pairs are few enough for the chain to matter.
+constexpr double kOverlapPairs = 1.2e9, kOverlapMin = 5e7;
+constexpr int kOverlapLevels = 4, kOverlapRows = 20;
 
 struct Work {
     hipStream_t stream = nullptr;
@@ -224,7 +228,11 @@ struct Work {
     // field's chain of short launches takes a fair part of the pass (order 6, off -> on:
     // 20k points 252 -> 237 us, 100k 652 -> 530, 250k (4e8 pairs) 1049 -> 863, 500k (1.1e9)
     // 1672 -> 1620; 1M (1.8e9) 2735 -> 2775: the second surface launch then costs what
-    // the overlap gains).
+    // the overlap gains). With three levels or fewer the second stream's launches and waits
+    // cost 15 to 45 us where there is little to overlap (order 6, off -> on: 10 points 21 ->
+    // 68 us, 100 30 -> 69, 2,000 63 -> 89, Kelvin U 10,000 (9e7 pairs) 181 -> 191), except
+    // beside larger operators (order 35, 10,000 points 162 -> 133); with four and more they
+    // pay at any size (5,000 points, hypersingular 138 -> 129; 2,000 137 -> 133).
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
     bool overlap = true;
@@ -247,7 +255,8 @@ struct Work {
         TBEM_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         TBEM_HIP(hipEventRecord(done, stream));
         TBEM_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-        overlap = P.blk >= 48 || P.p2p_pairs <= kOverlapPairs;
+        const bool chain = P.ot.n_levels >= kOverlapLevels || (P.blk >= kOverlapRows && P.p2p_pairs >= kOverlapMin);
+        overlap = P.blk >= 48 || (chain && P.p2p_pairs <= kOverlapPairs);
         TBEM_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
         TBEM_HIP(hipEventCreateWithFlags(&join, hipEventDisableTiming));
         dens.alloc(P.R * P.n_src);

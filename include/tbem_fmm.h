@@ -290,8 +290,9 @@ int tbem_fmm_m2l_ms(tbem_fmm_t h, double* ms);
  * stream of the handle beside the far field, and the surface sources (M2P, L2P) are
  * added after both; on == 0: one fused leaf launch after the far field, as the
  * reference orders the stages (cpp/fmm.cpp:550-558). Same results to rounding. The
- * default is on where the operator size R * n_e is at least 48 (a large far field) or
- * the point pairs are at most 1.2e9, and off otherwise. No reference counterpart: it
+ * default is on where the operator size R * n_e is at least 48 (a large far field), or
+ * the point pairs are at most 1.2e9 and the observation tree has four levels or more (or
+ * R * n_e >= 20 and the pairs are at least 5e7); off otherwise. No reference counterpart: it
  * also lets a profiler time each kernel on an idle device. */
 int tbem_fmm_set_overlap(tbem_fmm_t h, int on);
 
