@@ -2180,7 +2180,7 @@ int tbem_fmm_info(tbem_fmm_t h, tbem_fmm_info_t* o) {
         for (const DevBuf<float>* b : {&W.chk_up, &W.m2l_w}) wb += (double)b->n * sizeof(float);
         o->work_bytes = wb;
         o->leaf_wave_items = P.leaf_split.n_work;
-        o->leaf_chunked = P.leaf_split.n_parts;
+        o->leaf_chunked = P.leaf_split.n_wave_parts;
         o->leaf_block = P.leaf_split.n_block_leaves;
         o->leaf_symmetric = P.sym.n_leaves;
         o->symmetric_pairs = P.sym.pairs;

@@ -166,8 +166,8 @@ typedef struct {
                                 the adjoint and gradient add theirs on first use) */
     /* How the forward point-target stage (P2P + M2P + L2P) runs its observation leaves:
        leaf_wave_items one-wave work items (whole small leaves and chunks), of which the
-       chunks of leaf_chunked leaves too large for one wave; leaf_block leaves on the
-       one-workgroup kernel (more than 64 points with more pairs than one wave takes).
+       chunks of leaf_chunked leaves; leaf_block leaves on the one-workgroup kernel (more
+       than 64 points with more pairs than one wave takes), whole or in chunks of their own.
        leaf_symmetric leaves evaluate symmetric_pairs point pairs of their neighbours'
        once for both directions (TBEM_POINT_PAIRS_AUTO); the counts above then describe
        the rest of the pairs. */
