@@ -212,8 +212,10 @@ struct Work {
     // Stage boundaries 0..7; 8, 9 around the M2L translation kernel; 10, 11 around the
     // point-pair (P2P) launch on the side stream. Where the surface stages apply the C2E (small
     // operators, where a pass may be as short as its launches) 0..9 are stamps in ts that the
-    // stages' own kernels write, else events. A sphere of 15,360 points, order 5, host-bound:
-    // 142 us a pass with the ten events, 122 with the stamps; 61k points, order 35, 848 -> 822.
+    // stages' own kernels write, else events. Stamp 10 is the end of the far field, by each of
+    // its last stages in turn: beside the point pairs' stream the leaf stage (5) may start much
+    // later. A sphere of 15,360 points, order 5, host-bound: 142 us a pass with the ten events,
+    // 122 with the stamps; 61k points, order 35, 848 -> 822.
     hipEvent_t ev[12];
     DevBuf<unsigned long long> ts;
     double ts_per_ms = 0;
@@ -1485,6 +1487,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         m.out = W.fld.p;
         m.no_cutoff = P.m2l_no_cutoff;
         fuse_down(m);
+        m.stamp_last = st(10);
         launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         mark(9);
         if (!P.fuse_c2e) down_c2e(P.t_m2l);
@@ -1496,6 +1499,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     pl.out = W.fld.p;
     fuse_down(pl);
     if (!P.m2l_mfma.enabled) pl.stamp = st(9);
+    pl.stamp_last = st(10);
     launch_surf_stage(P.kid, false, false, false, pl, P.kc, s);
     if (!P.fuse_c2e) down_c2e(P.t_p2l);
     mark(4);
@@ -1513,6 +1517,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             l.out = W.fld.p;
             fuse_down(l);
             if (L == 1) l.stamp = st(4);
+            l.stamp_last = st(10);
             launch_surf_stage(P.kid, true, false, false, l, P.kc, s);
         }
         if (!P.fuse_c2e) down_c2e(P.t_olev[L]);
@@ -1903,12 +1908,14 @@ static int guard(F&& f) {
 }
 
 // The last forward's stamps in milliseconds from the first. A stage without a kernel left
-// none: it takes the next boundary's (the M2L's end, 9, comes before 4).
+// none: it takes the next boundary's (the M2L's end, 9, comes before 4, the far field's, 10,
+// before 5, and the local expansions' clearing, 8, is the last of it where nothing follows).
 static std::array<double, kStamps> stamps_ms(Work& W) {
     TBEM_HIP(hipEventSynchronize(W.done));
-    const std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
+    std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
+    if (!raw[10]) raw[10] = raw[8];
     std::array<double, kStamps> t{};
-    const int order[kStamps] = {0, 1, 2, 3, 8, 9, 4, 5, 6, 7};
+    const int order[kStamps] = {0, 1, 2, 3, 8, 9, 4, 10, 5, 6, 7};
     // (a gradient's own far field ends without a leaf stage: the last stamp stands for the rest)
     double next = (double)(long long)(*std::max_element(raw.begin(), raw.end()) - raw[0]) / W.ts_per_ms;
     for (int i = kStamps - 1; i >= 0; i--) {
@@ -2268,6 +2275,7 @@ int tbem_fmm_stage_times(tbem_fmm_t h, double* ms) {
         if (W.stamped) {
             const std::array<double, kStamps> t = stamps_ms(W);
             for (int k = 0; k < 7; k++) ms[k] = t[k + 1] - t[k];
+            ms[4] = t[10] - t[4];  // to the end of the far field, not to the leaf stage's start
         } else {
             TBEM_HIP(hipEventSynchronize(W.ev[7]));
             for (int k = 0; k < 7; k++) {

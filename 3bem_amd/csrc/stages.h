@@ -114,7 +114,7 @@ struct SurfStage {
     const double* c2e;
     double* c2e_out;
     int c2e_add;
-    unsigned long long* stamp;  // see stamp_start
+    unsigned long long *stamp, *stamp_last;  // see stamp_start, stamp_end (with c2e)
     int no_cutoff;          // surface sources: every pair is known to lie beyond the r2 < 1e-12
                             // cutoff, so the kernels leave the test out (same result)
 };
@@ -232,7 +232,7 @@ void launch_range_close(int n_items, const int* leaves, const TreeView& tt, cons
                         hipStream_t s);
 
 // ts (optional): kStamps stamps, cleared, and the first set as the kernel starts
-constexpr int kStamps = 10;
+constexpr int kStamps = 11;
 void launch_gather_dens(const double* x, const int* perm, const double* w, int n, int R,
                         double* dens, hipStream_t s, unsigned long long* ts = nullptr);
 // t0, t1 (optional): stamps of the kernel's start and end

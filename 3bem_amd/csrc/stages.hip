@@ -508,6 +508,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
         double* e = a.c2e_out + (size_t)cell * a.blk + tid;
         *e = a.c2e_add ? *e + s : s;
     }
+    stamp_end(a.stamp_last);
 }
 
 // The same stage for kSurfBlock / 2 < n_e <= kSurfOneMax with one target per lane and a

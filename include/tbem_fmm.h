@@ -278,12 +278,20 @@ int tbem_fmm_octree(tbem_fmm_t h, int which, double* cells, long* indices,
                     size_t* n_cells, size_t* n_indices);
 
 /* Per-stage device times of the last apply, milliseconds, in the order
- * gather, p2m, m2m, m2l, l2l, p2p(+m2p+l2p), scatter (7 doubles). */
+ * gather, p2m, m2m, m2l, l2l, p2p(+m2p+l2p), scatter (7 doubles). From 48 rows
+ * (R*n_e) on the stages lie between recorded events; below, between device clock
+ * readings of their own kernels: a stage lasts from the start of its first workgroup
+ * to that of the next stage's (l2l and scatter: to the end of their last workgroup by
+ * index), and one without a kernel takes no time. With the point pairs on the second
+ * stream (tbem_fmm_set_overlap) the sixth value is their time and that of the surface
+ * sources together. */
 int tbem_fmm_stage_times(tbem_fmm_t h, double* ms7);
 
 /* Device time of the M2L translation kernel alone in the last apply (ms): the
- * grouped MFMA GEMM in mixed precision, the FP64 M2L stage otherwise. No
- * reference counterpart: a profiling aid for roofline reports. */
+ * grouped MFMA GEMM (FP32 in mixed precision from 48 rows on, else FP64) where the plan
+ * has translation classes, the M2L stage on the surfaces otherwise (below 48 rows with
+ * its check-to-equivalent product). No reference counterpart: a profiling aid for
+ * roofline reports. */
 int tbem_fmm_m2l_ms(tbem_fmm_t h, double* ms);
 
 /* on != 0: the point-to-point pairs (P2P, and the transpose's P2P^T) run on a second
