@@ -819,6 +819,11 @@ static std::vector<I> xcd_layout(const std::vector<std::pair<long, I>>& items, i
 constexpr int kWaveChunkLeaf = 64;
 constexpr long kWaveFill = 16384, kWaveCapMin = 4096;
 constexpr long kBlockFill = 8192, kBlockCapMin = 16384;
+// The chunk sums of the workgroup leaves take at most 2 GiB, shared out by their pairs: 24,576
+// doubles per target at kBlockFill items, so that only leaves of some 10,000 points and more
+// get longer chunks for it (one leaf of 400,000 points took 7.5 GB, and of 1.2 million, past
+// the items' 32-bit offsets, one workgroup for all of it).
+constexpr double kBlockPartDoubles = double(size_t(1) << 28);
 
 static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
                          const HostList& surf, int n_e, int block_tile, LeafSplit& out, hipStream_t s) {
@@ -855,7 +860,11 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
         // points, whole tiles from the run's start
         const long tile = wave ? kWaveTile : block_tile, cap = wave ? wave_cap : block_cap;
         const long per = wave && nc > 1 ? (src + nc - 1) / nc : std::max(1L, src);
-        const long sub = m * src > cap ? std::max(1L, (cap / m + tile - 1) / tile) * tile : per;
+        long sub = m * src > cap ? std::max(1L, (cap / m + tile - 1) / tile) * tile : per;
+        if (!wave) {
+            const long most = std::max(1L, (long)(kBlockPartDoubles * (m * src) / block_total / (kPartRows * m)));
+            sub = std::max(sub, ((np + most - 1) / most + tile - 1) / tile * tile);
+        }
         long n_chunks = (np + per - 1) / per * ((per + sub - 1) / sub) + (c1 - c0) + 1;  // at most
         if ((nc <= 1 || !wave) && np <= sub) n_chunks = 1;
         auto& items = wave ? w : bi;
