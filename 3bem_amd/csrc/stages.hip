@@ -1649,7 +1649,7 @@ __global__ __launch_bounds__(kWaveLeafMax) void k_leaf_grad_parts(LeafStage a, d
 // Measured against FP64 FMAs from 4 x 4 register tiles, per launch: blk 453 (traction,
 // order 150, at most 1,024 cells) 58 -> 22 us; blk 150 (mesh of 9,102 points) 22 -> 9.5;
 // 2M points, order 100 (blk 297): 16 launches 2311 -> 1500 us beside the point pairs.
-constexpr int kGemmWideMin = 512;
+constexpr int kGemmWideMin = 512, kGemmTiles = 65536;
 typedef double gemm_f64x4 __attribute__((ext_vector_type(4)));
 
 template <int WR, int WC, int RT, int CT, int KC>
@@ -1803,13 +1803,19 @@ void launch_level_gemm(const CellTiles& T, int blk, const double* M, bool trans,
                        const double* addin, double* out, float* out32, bool add, hipStream_t s) {
     if (T.n == 0) return;
     const int rb = div_up(blk, 64);
-    if (rb * T.n >= kGemmWideMin)
-        hipLaunchKernelGGL((k_level_gemm<2, 2, 2, 2, 32>), dim3(rb, T.n), dim3(256), 0, s, blk, T.cells.p, T.tiles.p,
-                           M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
-    else
-        hipLaunchKernelGGL((k_level_gemm<4, 1, 1, 1, 64>), dim3(rb, T.n, 4), dim3(256), 0, s, blk, T.cells.p,
-                           T.tiles.p, M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
-    TBEM_LAUNCH_CHECK();
+    const bool wide = (long)rb * T.n >= kGemmWideMin;
+    // (a launch holds 65,536 workgroups in y: more tiles than that, of 4.2 million cells, in turn)
+    for (int t0 = 0; t0 < T.n; t0 += kGemmTiles) {
+        const int nt = std::min(kGemmTiles, T.n - t0);
+        const int* tiles = T.tiles.p + 3 * (size_t)t0;
+        if (wide)
+            hipLaunchKernelGGL((k_level_gemm<2, 2, 2, 2, 32>), dim3(rb, nt), dim3(256), 0, s, blk, T.cells.p, tiles, M,
+                               trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+        else
+            hipLaunchKernelGGL((k_level_gemm<4, 1, 1, 1, 64>), dim3(rb, nt, 4), dim3(256), 0, s, blk, T.cells.p, tiles,
+                               M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+        TBEM_LAUNCH_CHECK();
+    }
 }
 
 // One workgroup per item: the tight box of the item's target points (block min/max),
