@@ -825,8 +825,32 @@ constexpr long kBlockFill = 8192, kBlockCapMin = 16384;
 // the items' 32-bit offsets, one workgroup for all of it).
 constexpr double kBlockPartDoubles = double(size_t(1) << 28);
 
-static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
-                         const HostList& surf, int n_e, int block_tile, LeafSplit& out, hipStream_t s) {
+// The layout on the host, and its upload (the layouts of one tree are made side by side).
+struct LeafLayout {
+    std::vector<WaveItem> items, block_items;
+    std::vector<WaveLeafParts> parts;
+    std::vector<int> block;
+    int n_wave_parts = 0, n_work = 0, n_block_leaves = 0;
+    size_t part_size = 0;
+    void upload(LeafSplit& out, hipStream_t s) const {
+        out.n_work = n_work;
+        out.n_block_leaves = n_block_leaves;
+        out.n_items = (int)items.size();
+        out.n_block_items = (int)block_items.size();
+        out.n_block = (int)block.size();
+        out.n_wave_parts = n_wave_parts;
+        out.n_parts = (int)parts.size();
+        out.part_size = part_size;
+        out.items.upload(items, s);
+        out.block_items.upload(block_items, s);
+        out.parts.upload(parts, s);
+        out.block.upload(block, s);
+    }
+};
+
+static LeafLayout split_leaves(const HostTree& tt, const std::vector<int>& leaves, const HostList& pts,
+                               const HostList& surf, int n_e, int block_tile) {
+    LeafLayout out;
     std::vector<std::pair<long, WaveItem>> w, bi, ch;
     std::vector<std::pair<long, int>> b;
     w.reserve(leaves.size());
@@ -902,21 +926,16 @@ static void split_leaves(const HostTree& tt, const std::vector<int>& leaves, con
         part += (long)ch.size() * kPartRows * m;
     }
     const WaveItem empty{-1, 0, 0, 0, 0, 0, 0, 0, -1};
-    const std::vector<WaveItem> wi = xcd_layout(w, kWaveBlock / 64, empty), bl = xcd_layout(bi, 1, empty);
-    const std::vector<int> whole = xcd_layout(b, 1, -1);
+    out.items = xcd_layout(w, kWaveBlock / 64, empty);
+    out.block_items = xcd_layout(bi, 1, empty);
+    out.block = xcd_layout(b, 1, -1);
     out.n_work = (int)w.size();
     out.n_block_leaves = (int)b.size();
-    out.n_items = (int)wi.size();
-    out.n_block_items = (int)bl.size();
-    out.n_block = (int)whole.size();
     out.n_wave_parts = (int)wparts.size();
     wparts.insert(wparts.end(), bparts.begin(), bparts.end());
-    out.n_parts = (int)wparts.size();
+    out.parts = std::move(wparts);
     out.part_size = (size_t)part;
-    out.items.upload(wi, s);
-    out.block_items.upload(bl, s);
-    out.parts.upload(wparts, s);
-    out.block.upload(whole, s);
+    return out;
 }
 
 // FmmPlan::sym from the P2P pairs of the shared tree T (forward lists by leaf
@@ -1085,7 +1104,7 @@ static void build_sym(FmmPlan& P, const HostTree& T, const std::vector<std::arra
     Y.n_g = (int)g_pos.size();
     Y.n_rev = n_rev;
     clk.mark("sym: upload");
-    split_leaves(T, leaves, ord, lm, P.n_e, leaf_stage_tile(P.kid, P.precision == TBEM_MIXED), Y.split, s);
+    split_leaves(T, leaves, ord, lm, P.n_e, leaf_stage_tile(P.kid, P.precision == TBEM_MIXED)).upload(Y.split, s);
     clk.mark("sym: split");
     close_flags(Y.ord, P.obs_leaves.p, P.dot, P.op, P.sp, s);
     Y.on = true;
@@ -1296,8 +1315,11 @@ static std::shared_ptr<FmmPlan> build_plan(const tbem_fmm_desc* d, hipStream_t s
         P->leaf_p2p.upload(lp, s);
         P->leaf_m2p.upload(lm, s);
         const int tile = leaf_stage_tile(P->kid, P->precision == TBEM_MIXED);
-        split_leaves(OT, OT.leaves, lp, lm, P->n_e, tile, P->leaf_split, s);
-        split_leaves(OT, OT.leaves, HostList(), lm, P->n_e, tile, P->surf_split, s);
+        const HostList none, *pts[2] = {&lp, &none};
+        LeafLayout lay[2];
+        parallel_for(2, [&](size_t i) { lay[i] = split_leaves(OT, OT.leaves, *pts[i], lm, P->n_e, tile); });
+        lay[0].upload(P->leaf_split, s);
+        lay[1].upload(P->surf_split, s);
         clk.mark("leaf lists");
         if (P->same_tree && (P->kid == TBEM_K_ELASTIC_DISPLACEMENT || P->kid == TBEM_K_LAPLACE_SINGLE) &&
             d->point_pairs == TBEM_POINT_PAIRS_AUTO)
@@ -1338,10 +1360,9 @@ const FmmPlan::AdjLists& FmmPlan::adjoint_lists(hipStream_t s) const {
         A->leaf_p2p.upload(lp, s);
         A->leaf_p2l.upload(ll, s);
         const int tile = leaf_stage_tile(kid, precision == TBEM_MIXED);
-        split_leaves(ST, ST.leaves, lp, ll, n_e, tile, A->leaf_split, s);
-        split_leaves(ST, ST.leaves, HostList(), ll, n_e, tile, A->surf_split, s);
+        HostList ord;
         if (sym.on) {  // one shared tree: source leaf positions are the forward's
-            HostList ord = list_from_pairs(ST.leaves, ST.n_cells, tl.p2p, 1, nullptr);
+            ord = list_from_pairs(ST.leaves, ST.n_cells, tl.p2p, 1, nullptr);
             const size_t nl = ord.ptr.size() - 1;
             std::vector<char> keep(ord.cell.size());
             std::vector<int> ptr(nl + 1, 0), cell;
@@ -1369,9 +1390,14 @@ const FmmPlan::AdjLists& FmmPlan::adjoint_lists(hipStream_t s) const {
             ord.cell = std::move(cell);
             cells_to_ranges(ord, ST);
             A->sym_ord.upload(ord, s);
-            split_leaves(ST, ST.leaves, ord, ll, n_e, tile, A->sym_split, s);
             close_flags(A->sym_ord, src_leaves.p, dst, sp, op, s);
         }
+        const HostList none, *pts[3] = {&lp, &none, &ord};
+        LeafLayout lay[3];
+        parallel_for(sym.on ? 3 : 2, [&](size_t i) { lay[i] = split_leaves(ST, ST.leaves, *pts[i], ll, n_e, tile); });
+        lay[0].upload(A->leaf_split, s);
+        lay[1].upload(A->surf_split, s);
+        if (sym.on) lay[2].upload(A->sym_split, s);
     }
     close_flags(A->leaf_p2p, src_leaves.p, dst, sp, op, s);
     A->t_slev.resize(ST.n_levels);
