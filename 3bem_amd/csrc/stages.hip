@@ -43,27 +43,23 @@
 
 namespace tbem {
 
-// SoA source tile: FP64 coordinates, normals and densities in VT; sv: normal . density
-// (FP64 tiles of three components, kop_pt).
-template <class VT, int R, bool NRM>
-constexpr bool tile_has_sv() {
-    return NRM && R == 3 && std::is_same<VT, double>::value;
-}
-template <class VT, int R, bool NRM, int NB>
+// SoA source tile: FP64 coordinates, normals and densities in VT; with SV also
+// sv = normal . density (kop_pt's points).
+template <class VT, int R, bool NRM, int NB, bool SV = false>
 struct Tile {
     double x[NB], y[NB], z[NB];
     VT nx[NRM ? NB : 1], ny[NRM ? NB : 1], nz[NRM ? NB : 1];
     VT d[R][NB];
-    VT sv[tile_has_sv<VT, R, NRM>() ? NB : 1];
+    VT sv[SV ? NB : 1];
 };
 
 // LDS of a stage kernel: the point tile (values in PT), the surface tile (FP64),
 // and the cross-slice reduction (RED doubles per thread) share bytes, since they
 // are live one at a time; the range cache serves the packed point stream.
-template <class PT, int R, bool NRM, int NB, int RED>
+template <class PT, int R, bool NRM, int NB, int RED, bool SV = false>
 struct StageSmem {
     union {
-        Tile<PT, R, NRM, NB> pt;
+        Tile<PT, R, NRM, NB, SV> pt;
         Tile<double, R, NRM, NB> st;
         double red[RED * NB];
     };
@@ -181,14 +177,14 @@ __device__ inline void load_surf(SrcReg<R, NRM>& r, int c, int j, const TreeView
     for (int q = 0; q < R; q++) r.d[q] = coeff[(size_t)c * blk + q * n_e + j];
 }
 
-template <class VT, int R, bool NRM, int NB>
-__device__ inline void store_tile(Tile<VT, R, NRM, NB>& tl, int slot, const SrcReg<R, NRM>& r) {
+template <class VT, int R, bool NRM, int NB, bool SV>
+__device__ inline void store_tile(Tile<VT, R, NRM, NB, SV>& tl, int slot, const SrcReg<R, NRM>& r) {
     tl.x[slot] = r.x;
     tl.y[slot] = r.y;
     tl.z[slot] = r.z;
     if (NRM) { tl.nx[slot] = VT(r.nx); tl.ny[slot] = VT(r.ny); tl.nz[slot] = VT(r.nz); }
     for (int q = 0; q < R; q++) tl.d[q][slot] = VT(r.d[q]);
-    if constexpr (tile_has_sv<VT, R, NRM>()) tl.sv[slot] = r.nx * r.d[0] + r.ny * r.d[1] + r.nz * r.d[2];
+    if constexpr (SV) tl.sv[slot] = r.nx * r.d[0] + r.ny * r.d[1] + r.nz * r.d[2];
 }
 
 // Streams the points of ranges e0..e1 (sorted points [rbeg[e], rbeg[e]+rcnt[e]))
@@ -249,8 +245,8 @@ __device__ inline void stream_ranges(Tile<VT, R, NRM, NB>& tl, int e0, int e1,
 // of the cached range starts (point indices are below 2^30).
 constexpr int kCloseBit = 1 << 30;
 
-template <class VT, int R, bool NRM, int NB, class F>
-__device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB>& tl, int* s_pre, int* s_beg, int e0, int e1,
+template <class VT, int R, bool NRM, int NB, bool SV, class F>
+__device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB, SV>& tl, int* s_pre, int* s_beg, int e0, int e1,
                                             int v0, int v1, const int* __restrict__ rbeg,
                                             const int* __restrict__ rpre, const PtsView& sp,
                                             const double* __restrict__ dens, int n_src, F&& compute,
@@ -358,8 +354,8 @@ __device__ inline void stream_surfaces(Tile<double, R, NRM, NB>& tl, int e0, int
 // One source j of the tile on one target (FP64 coordinates tx, ty, tz): the
 // displacement is formed in FP64, then the kernel runs in T.
 template <int KID, bool ADJ, bool FAST = false, bool CUT = true, bool TWO = false, class T, class VT, int R, bool NRM,
-          int NB>
-__device__ __forceinline__ void pair(const Tile<VT, R, NRM, NB>& tl, int j, double tx, double ty, double tz,
+          int NB, bool SV>
+__device__ __forceinline__ void pair(const Tile<VT, R, NRM, NB, SV>& tl, int j, double tx, double ty, double tz,
                                      const T* tn, T* acc, const KC<T>& kc) {
     const T sn[3] = {NRM ? T(tl.nx[j]) : T(0), NRM ? T(tl.ny[j]) : T(0), NRM ? T(tl.nz[j]) : T(0)};
     T v[R];
@@ -385,8 +381,8 @@ template <int KID, class T, bool ADJ>
 constexpr int leaf_slots() {
     return uses_pt<KID, T, ADJ>() ? pt_slots<KID, ADJ>() : kernel_dim(KID);
 }
-template <int KID, bool ADJ, bool FAST, bool CUT, class T, class VT, int R, bool NRM, int NB>
-__device__ __forceinline__ void point_pair(const Tile<VT, R, NRM, NB>& tl, int j, double tx, double ty, double tz,
+template <int KID, bool ADJ, bool FAST, bool CUT, class T, class VT, int R, bool NRM, int NB, bool SV>
+__device__ __forceinline__ void point_pair(const Tile<VT, R, NRM, NB, SV>& tl, int j, double tx, double ty, double tz,
                                            const T* tn, T* acc, const KC<T>& kc) {
     if constexpr (uses_pt<KID, T, ADJ>()) {
         const double sn[3] = {tl.nx[j], tl.ny[j], tl.nz[j]}, v[3] = {tl.d[0][j], tl.d[1][j], tl.d[2][j]};
@@ -692,7 +688,7 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
     constexpr int R = kernel_dim(KID);
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
-    __shared__ StageSmem<T, R, NRM, NB, 2 * R> sm;
+    __shared__ StageSmem<T, R, NRM, NB, 2 * R, uses_pt<KID, T, ADJ>()> sm;
     stamp_start(a.stamp);
     const WaveItem* it = a.split ? a.block_items + blockIdx.x : nullptr;
     const int pos = it ? uni(it->pos) : (int)blockIdx.x;
@@ -819,10 +815,10 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
 // from setting the launch's length: on the 1M-point leaf-64 workload a 3-point leaf
 // has 674k point sources, and 20 leaves have 1-2.4M pairs each.
 
-template <class PT, int R, bool NRM>
+template <class PT, int R, bool NRM, bool SV>
 struct WaveSmem {
     union {
-        Tile<PT, R, NRM, 64> pt;
+        Tile<PT, R, NRM, 64, SV> pt;
         Tile<double, R, NRM, 64> st;
         double red[2 * R * 64];
     };
@@ -842,7 +838,8 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     constexpr int R = kernel_dim(KID);
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     constexpr bool SPLIT = !std::is_same<T, double>::value;
-    __shared__ WaveSmem<T, R, NRM> smw[kWaveBlock / 64];
+    using Smem = WaveSmem<T, R, NRM, uses_pt<KID, T, ADJ>()>;
+    __shared__ Smem smw[kWaveBlock / 64];
     stamp_start(a.stamp);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int idx = blockIdx.x * (kWaveBlock / 64) + w;
@@ -850,7 +847,7 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     const WaveItem* it = a.wave_items + idx;
     const int pos = uni(it->pos);
     if (pos < 0) return;  // padding of the layout
-    WaveSmem<T, R, NRM>& sm = smw[w];
+    Smem& sm = smw[w];
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);  // m <= kWaveLeafMax
     const int nslot = (m + 1) >> 1, S = 64 / nslot;
