@@ -570,11 +570,11 @@ __global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double
 }
 
 // The same sums again where few items, or a few long ones, leave the chip idle behind one
-// lane's chain of sources: the elastic kernels' surface sources. An item's targets go to
-// surf_parts(n_e) workgroups of at most 64 targets, and the four waves of each take every
-// fourth source of a chunk; what a source adds to a target goes to LDS, and one thread per
-// target and component adds the chunk in source order (slice by slice, as k_surf_one's lanes
-// do), so that the sums keep their bits. The traction and hypersingular kernels add a value
+// lane's chain of sources: the elastic kernels' surface sources, where k_surf_one has one
+// slice (n_e > kSurfBlock). An item's targets go to surf_parts(n_e) workgroups of at most 64
+// targets, and the four waves of each take every fourth source of a chunk; what a source adds
+// to a target goes to LDS, and one thread per target and component adds the chunk in source
+// order, so that the sums keep their bits. The traction and hypersingular kernels add a value
 // by a plain add; Kelvin U adds ri w in one FMA, so ri goes along. Two chunk buffers: one
 // barrier per chunk. Bound: vector issue, with the LDS round trip of a source beside its 50
 // instructions; chunks of eight sources, so that registers (128) and LDS (35 KB) leave four
@@ -588,7 +588,7 @@ constexpr bool has_split(int kid) { return kid == K_EU || kid == K_ET || kid == 
 static int surf_parts(int n_e) { return (n_e + 63) / 64; }
 
 template <int KID, bool ADJ, bool CUT>
-__global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> kc, double scale, int S, int add, int parts) {
+__global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> kc, double scale, int add, int parts) {
     constexpr int R = kernel_dim(KID), NV = split_values<KID>(), C = 8;
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     static_assert(R == 3, "one wave per component adds");
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> k
             o[2][lane] = x[2];
         }
     };
-    double acc[3] = {0.0, 0.0, 0.0};  // component w of the lane's target, per slice (S <= 3)
+    double acc = 0.0;  // component w of the lane's target
     int buf = 0;
     auto plus = [&](double s, int jj) {
         if constexpr (KID == K_EU) return fma(inc[buf][jj][NV - 1][lane], inc[buf][jj][w][lane], s);
@@ -646,14 +646,11 @@ __global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> k
                 if (w + 4 * i < n) values(c0 + w + 4 * i, inc[buf][w + 4 * i]);
             __syncthreads();
             if (w < R) {
-                if (S == 1 && n == C) {
+                if (n == C) {
 #pragma unroll
-                    for (int jj = 0; jj < C; jj++) acc[0] = plus(acc[0], jj);
+                    for (int jj = 0; jj < C; jj++) acc = plus(acc, jj);
                 } else {
-#pragma unroll
-                    for (int k = 0; k < 3; k++)  // slice k: the tile's sources k, k + S, ..
-                        if (k < S)
-                            for (int jj = (k + S - c0 % S) % S; jj < n; jj += S) acc[k] = plus(acc[k], jj);
+                    for (int jj = 0; jj < n; jj++) acc = plus(acc, jj);
                 }
             }
             buf ^= 1;
@@ -662,9 +659,7 @@ __global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> k
     stream_surfaces(st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
     if (w < R && mine) {
         double s = 0;
-        s += acc[0];
-        if (S > 1) s += acc[1];
-        if (S > 2) s += acc[2];
+        s += acc;
         s *= scale;
         double* o = a.out + (size_t)cell * a.blk + w * n_e + tg;
         *o = add ? *o + s : s;
@@ -1908,10 +1903,16 @@ KC<float> kc_of<float>(const KConst& c) { return make_kc32(c); }
 
 // k_surf_one takes as long as its longest item's waves, or as all its waves take on the chip's
 // SIMDs: k_surf_split, a quarter more work but 1/4 of the chain and finer pieces, where the
-// first is kSurfSplit times the second. Traction, order 150: 454 items of up to 74 cells, 13,546
-// cells, M2L 1466 -> 1026 us, transposed 1306 -> 965; L2L^T and M2M (eight cells an item, up to
-// 256 items) 404 -> 270 us for five levels; the whole pass, both directions and gradient, 5356
-// -> 4330 us. Items of equal length that fill the chip stay (M2M of a deep tree's lowest level).
+// first is kSurfSplit times the second, and k_surf_one's lanes have one slice. Traction, order
+// 150: 454 items of up to 74 cells, 13,546 cells, M2L 1466 -> 1026 us, transposed 1306 -> 965;
+// L2L^T and M2M (eight cells an item, up to 256 items) 404 -> 270 us for five levels; the whole
+// pass, both directions and gradient, 5356 -> 4330 us. Passes, 9,000 sources and 9,001 targets,
+// k_surf_one -> k_surf_split: 130 surface points hypersingular 2492 -> 1333 us, traction 1688
+// -> 1195, Kelvin U 1216 -> 1173; 240 points 5475 -> 2739, 3587 -> 2365, 2455 -> 2343. With two
+// or three slices the chain is as short without: 76 points (order 75) 717 -> 1070, 567 -> 988,
+// 460 -> 960. Items of equal length that fill the chip stay (M2M of a deep tree's lowest level;
+// two cubes of 20,000 and 10,000 points, Kelvin U, 150 points 6567 -> 8491); kSurfSplit between
+// 0.7 and 3 moves the passes by up to 3%.
 constexpr double kSurfSimds = 1024, kSurfSplit = 1.3;
 
 template <int KID, class T>
@@ -1926,17 +1927,18 @@ static void surf_launch(bool src_surf, bool add, bool adj, const SurfStage& a, c
         const dim3 w(div_up((size_t)a.n_e * S, 64) * 64);
         const int ad = add ? 1 : 0;
         if constexpr (has_split(KID)) {
-            if (src_surf && (double)a.longest * kSurfSimds > kSurfSplit * (double)a.n_cells * (w.x / 64)) {
+            if (src_surf && S == 1 &&
+                (double)a.longest * kSurfSimds > kSurfSplit * (double)a.n_cells * (w.x / 64)) {
                 const int parts = surf_parts(a.n_e);
                 const dim3 gp((unsigned)a.n_items * parts), bp(256);
-                if (a.no_cutoff && !adj) hipLaunchKernelGGL((k_surf_split<KID, false, false>), gp, bp, 0, s, a, kc, scale, S, ad,
-                                   parts);
-                else if (a.no_cutoff) hipLaunchKernelGGL((k_surf_split<KID, true, false>), gp, bp, 0, s, a, kc, scale, S, ad,
-                                   parts);
-                else if (!adj) hipLaunchKernelGGL((k_surf_split<KID, false, true>), gp, bp, 0, s, a, kc, scale, S, ad,
-                                   parts);
-                else hipLaunchKernelGGL((k_surf_split<KID, true, true>), gp, bp, 0, s, a, kc, scale, S, ad,
-                                   parts);
+                if (a.no_cutoff && !adj)
+                    hipLaunchKernelGGL((k_surf_split<KID, false, false>), gp, bp, 0, s, a, kc, scale, ad, parts);
+                else if (a.no_cutoff)
+                    hipLaunchKernelGGL((k_surf_split<KID, true, false>), gp, bp, 0, s, a, kc, scale, ad, parts);
+                else if (!adj)
+                    hipLaunchKernelGGL((k_surf_split<KID, false, true>), gp, bp, 0, s, a, kc, scale, ad, parts);
+                else
+                    hipLaunchKernelGGL((k_surf_split<KID, true, true>), gp, bp, 0, s, a, kc, scale, ad, parts);
                 TBEM_LAUNCH_CHECK();
                 return;
             }

@@ -1,7 +1,8 @@
 """The surface stages above 64 surface points at the edges of their shapes: slices per target
-(three up to 84 points, two to 128, one above), parts of 64 targets (two to four, even and
-uneven), and the general kernel again past 256 points. Laplace takes one workgroup per item
-(k_surf_one), the elastic kernels of these small problems several (k_surf_split). Against the
+(three up to 84 points, two to 128, one above), parts of 64 targets (three and four, even and
+uneven), and the general kernel again past 256 points. Laplace, and the elastic kernels up to
+128 points, take one workgroup per item (k_surf_one), the elastic kernels of these small
+problems above that several (k_surf_split). Against the
 oracle FMM on its own check-to-equivalent matrices, so that neither the method's error nor
 another pseudo-inverse enters; the transpose by its identity.
 
