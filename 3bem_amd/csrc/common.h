@@ -98,10 +98,12 @@ inline int div_up(size_t a, size_t b) { return (int)((a + b - 1) / b); }
 // that were active in a loop's last partial iteration.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Device-side times of a pass's stages: a kernel that begins a stage writes the clock as its
-// first workgroup starts, one that ends the pass as its last workgroup (by index) is through.
-// A null pointer writes nothing. (A recorded event is a packet and a host call of its own
-// between two launches.)
+// Device-side times of a pass's stages: a kernel writes the clock as its first workgroup
+// starts, or as its last workgroup (by index) is through; of several kernels of a stage the
+// last one's stays. A null pointer writes nothing. (A recorded event is a packet and a host
+// call of its own between two launches. A clock read at the start of a kernel keeps its later
+// uniform loads off the scalar unit: eight VGPRs and more in the surface stage, which only
+// takes the time at its end.)
 __device__ __forceinline__ void stamp_start(unsigned long long* t) {
     if (t && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *t = wall_clock64();
 }

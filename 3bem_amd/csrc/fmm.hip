@@ -211,10 +211,10 @@ struct Work {
     DevBuf<double> wrev;    // reverse sums of the symmetric pairs (R rows of FmmPlan::sym.n_rev)
     // Stage boundaries 0..7; 8, 9 around the M2L translation kernel; 10, 11 around the
     // point-pair (P2P) launch on the side stream. Where the surface stages apply the C2E (small
-    // operators, where a pass may be as short as its launches) 0..9 are stamps in ts that the
-    // stages' own kernels write, else events. Stamp 10 is the end of the far field, by each of
-    // its last stages in turn: beside the point pairs' stream the leaf stage (5) may start much
-    // later. A sphere of 15,360 points, order 5, host-bound: 142 us a pass with the ten events,
+    // operators, where a pass may be as short as its launches) they are stamps in ts that the
+    // stages' own kernels write, else events. Stamps 1 to 4 and 8 to 10 are the ends of the
+    // gather, P2M, M2M, M2L and P2L, the clearing before the M2L, its kernel and L2L, 5 the leaf
+    // stage's start, which beside the point pairs' stream may come much later than 10. A sphere of 15,360 points, order 5, host-bound: 142 us a pass with the ten events,
     // 122 with the stamps; 61k points, order 35, 848 -> 822.
     hipEvent_t ev[12];
     DevBuf<unsigned long long> ts;
@@ -1437,7 +1437,7 @@ template <class F = std::nullptr_t>
 static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, bool mfma, F&& after_gather = nullptr) {
     const int R = P.R;
     const int Ns = (int)P.n_src;
-    // boundary k: a stamp of the kernel that begins the stage, or an event
+    // boundary k: a stamp of the stages' kernels, or an event
     auto st = [&](int k) { return P.fuse_c2e ? W.ts.p + k : nullptr; };
     auto mark = [&](int k) {
         if (!P.fuse_c2e) TBEM_HIP(hipEventRecord(W.ev[k], s));
@@ -1455,7 +1455,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     };
     // down-check potentials -> added to the down-equivalent densities
     auto down_c2e = [&](const CellTiles& T) {
-        launch_level_gemm(T, P.blk, P.dc2e.p, false, W.fld.p, nullptr, W.locals.p, nullptr, true, s);
+        launch_level_gemm(T, P.blk, P.dc2e.p, false, W.fld.p, nullptr, W.locals.p, nullptr, true, s, st(4));
     };
 
     auto fuse_up = [&](SurfStage& a) {
@@ -1472,7 +1472,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     a.st = view(P.dst); a.sp = view(P.sp); a.dens = W.dens.p; a.n_src_pts = Ns;
     a.out = W.fld.p;
     fuse_up(a);
-    a.stamp = st(1);
+    a.stamp = st(2);
     launch_surf_stage(P.kid, false, false, false, a, P.kc, s);
     up_c2e(P.t_p2m);
     mark(2);
@@ -1489,7 +1489,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             m.st = view(P.dst); m.s_surf = P.d_inner.p; m.s_coeff = W.mult.p;
             m.out = W.fld.p;
             fuse_up(m);
-            if (L == P.st.n_levels - 2) m.stamp = st(2);
+            m.stamp = st(3);
             launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         }
         up_c2e(P.t_m2m[L]);
@@ -1501,7 +1501,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     mark(3);
 
     // M2L (cpp/fmm.cpp:362-382) and P2L (cpp/fmm.cpp:296-330) into locals
-    launch_fill(W.locals.p, W.locals.n, 0.0, s, st(3), st(8));
+    launch_fill(W.locals.p, W.locals.n, 0.0, s, nullptr, st(8));
     mark(8);
     if (mfma) {
         // Vd M_c Bu check = DC2E K_c UC2E check = the FP64 stage's DC2E K_c mult
@@ -1522,7 +1522,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
         m.out = W.fld.p;
         m.no_cutoff = P.m2l_no_cutoff;
         fuse_down(m);
-        m.stamp_last = st(10);
+        m.stamp = st(9);
         launch_surf_stage(P.kid, true, false, false, m, P.kc, s);
         mark(9);
         if (!P.fuse_c2e) down_c2e(P.t_m2l);
@@ -1533,8 +1533,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
     pl.st = view(P.dst); pl.sp = view(P.sp); pl.dens = W.dens.p; pl.n_src_pts = Ns;
     pl.out = W.fld.p;
     fuse_down(pl);
-    if (!P.m2l_mfma.enabled) pl.stamp = st(9);
-    pl.stamp_last = st(10);
+    pl.stamp = st(4);
     launch_surf_stage(P.kid, false, false, false, pl, P.kc, s);
     if (!P.fuse_c2e) down_c2e(P.t_p2l);
     mark(4);
@@ -1551,8 +1550,7 @@ static void farfield(const FmmPlan& P, Work& W, const double* x, hipStream_t s, 
             l.st = view(P.dot); l.s_surf = P.d_outer.p; l.s_coeff = W.locals.p;
             l.out = W.fld.p;
             fuse_down(l);
-            if (L == 1) l.stamp = st(4);
-            l.stamp_last = st(10);
+            l.stamp = st(10);
             launch_surf_stage(P.kid, true, false, false, l, P.kc, s);
         }
         if (!P.fuse_c2e) down_c2e(P.t_olev[L]);
@@ -1943,20 +1941,16 @@ static int guard(F&& f) {
 }
 
 // The last forward's stamps in milliseconds from the first. A stage without a kernel left
-// none: it takes the next boundary's (the M2L's end, 9, comes before 4, the far field's, 10,
-// before 5, and the local expansions' clearing, 8, is the last of it where nothing follows).
+// none: it ends where the one before it did. (A gradient's own far field ends without a leaf
+// stage.)
 static std::array<double, kStamps> stamps_ms(Work& W) {
     TBEM_HIP(hipEventSynchronize(W.done));
-    std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
-    if (!raw[10]) raw[10] = raw[8];
+    const std::vector<unsigned long long> raw = W.ts.to_host(W.stream);
     std::array<double, kStamps> t{};
-    const int order[kStamps] = {0, 1, 2, 3, 8, 9, 4, 10, 5, 6, 7};
-    // (a gradient's own far field ends without a leaf stage: the last stamp stands for the rest)
-    double next = (double)(long long)(*std::max_element(raw.begin(), raw.end()) - raw[0]) / W.ts_per_ms;
-    for (int i = kStamps - 1; i >= 0; i--) {
-        const int k = order[i];
-        if (raw[k]) next = (double)(long long)(raw[k] - raw[0]) / W.ts_per_ms;
-        t[k] = next;
+    double last = 0;
+    for (int k: {0, 1, 2, 3, 8, 9, 4, 10, 5, 6, 7}) {
+        if (raw[k]) last = (double)(long long)(raw[k] - raw[0]) / W.ts_per_ms;
+        t[k] = last;
     }
     return t;
 }
@@ -2310,7 +2304,7 @@ int tbem_fmm_stage_times(tbem_fmm_t h, double* ms) {
         if (W.stamped) {
             const std::array<double, kStamps> t = stamps_ms(W);
             for (int k = 0; k < 7; k++) ms[k] = t[k + 1] - t[k];
-            ms[4] = t[10] - t[4];  // to the end of the far field, not to the leaf stage's start
+            ms[4] = t[10] - t[4];  // to its own end, not to the leaf stage's start
         } else {
             TBEM_HIP(hipEventSynchronize(W.ev[7]));
             for (int k = 0; k < 7; k++) {

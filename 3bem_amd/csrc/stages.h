@@ -114,7 +114,7 @@ struct SurfStage {
     const double* c2e;
     double* c2e_out;
     int c2e_add;
-    unsigned long long *stamp, *stamp_last;  // see stamp_start, stamp_end (with c2e)
+    unsigned long long* stamp;  // see stamp_end (with c2e)
     int no_cutoff;          // surface sources: every pair is known to lie beyond the r2 < 1e-12
                             // cutoff, so the kernels leave the test out (same result)
 };
@@ -129,7 +129,8 @@ CellTiles make_level_tiles(const HostTree& t, int level, hipStream_t s);
 // level blk*blk row-major. FP64; out32 receives the result rounded to FP32 instead
 // of out when given. A tiled GEMM: each level matrix is read once per 64 cells.
 void launch_level_gemm(const CellTiles& T, int blk, const double* M, bool trans, const double* in,
-                       const double* addin, double* out, float* out32, bool add, hipStream_t s);
+                       const double* addin, double* out, float* out32, bool add, hipStream_t s,
+                       unsigned long long* stamp = nullptr);  // see stamp_end
 
 // Point-target stage (FP64, or T = float for the point sources (a) with every
 // displacement formed in FP64; the surface sources (b), (c) are always FP64).
@@ -231,7 +232,7 @@ void launch_range_close(int n_items, const int* leaves, const TreeView& tt, cons
                         const int* rbeg, const int* rcnt, const PtsView& sp, double margin, int* close,
                         hipStream_t s);
 
-// ts (optional): kStamps stamps, cleared, and the first set as the kernel starts
+// ts (optional): kStamps stamps, cleared but the first two, set as the kernel starts and ends
 constexpr int kStamps = 11;
 void launch_gather_dens(const double* x, const int* perm, const double* w, int n, int R,
                         double* dens, hipStream_t s, unsigned long long* ts = nullptr);

@@ -430,7 +430,6 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
     constexpr bool NRM = kernel_uses_nsrc(KID) || kernel_uses_nobs(KID);
     __shared__ StageSmem<double, R, NRM, NB, (DUAL ? 2 : 1) * R> sm;
     extern __shared__ double field[];  // R * n_e
-    stamp_start(a.stamp);
     const int item = a.order ? uni(a.order[blockIdx.x]) : (int)blockIdx.x;
     const int cell = uni(a.items[item]);
     const int lvl = uni(a.tt.level[cell]);
@@ -491,7 +490,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
         __syncthreads();
     }
     double* o = a.out + (size_t)cell * a.blk;
-    if (!a.c2e) {
+    if (DUAL || !a.c2e) {  // (two targets per lane: above 64 points, where no C2E follows)
         for (int row = tid; row < a.blk; row += NB) o[row] = add ? o[row] + field[row] : field[row];
         return;
     }
@@ -504,7 +503,7 @@ __global__ __launch_bounds__(kSurfBlock) void k_surf_stage(SurfStage a, KC<doubl
         double* e = a.c2e_out + (size_t)cell * a.blk + tid;
         *e = a.c2e_add ? *e + s : s;
     }
-    stamp_end(a.stamp_last);
+    stamp_end(a.stamp);
 }
 
 // The same stage for kSurfBlock / 2 < n_e <= kSurfOneMax with one target per lane and a
@@ -1650,7 +1649,8 @@ __global__ __launch_bounds__(WR* WC * 64) void k_level_gemm(int n, const int* __
                                                           const double* __restrict__ M, int trans,
                                                           const double* __restrict__ in,
                                                           const double* __restrict__ addin, double* __restrict__ out,
-                                                          float* __restrict__ out32, int add) {
+                                                          float* __restrict__ out32, int add,
+                                                          unsigned long long* stamp) {
     constexpr int NT = WR * WC * 64, RB = 16 * WR * RT, CB = 16 * WC * CT;
     constexpr int PR = RB * KC / NT, PC = CB * KC / NT;  // elements of each operand per thread and chunk
     const int t = blockIdx.y, z = blockIdx.z * CB;
@@ -1734,17 +1734,22 @@ __global__ __launch_bounds__(WR* WC * 64) void k_level_gemm(int n, const int* __
                 else out[o] = add ? out[o] + v : v;
             }
         }
+    stamp_end(stamp);
 }
 
 __global__ void k_gather_dens(const double* __restrict__ x, const int* __restrict__ perm,
                               const double* __restrict__ w, int n, int R, double* __restrict__ dens,
                               unsigned long long* ts) {
-    if (ts && blockIdx.x == 0 && threadIdx.x < kStamps) ts[threadIdx.x] = threadIdx.x == 0 ? wall_clock64() : 0ull;
+    if (ts) {
+        stamp_start(ts);
+        if (blockIdx.x == gridDim.x - 1 && threadIdx.x > 1 && threadIdx.x < kStamps) ts[threadIdx.x] = 0ull;
+    }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int g = perm[i];
     const double wi = w ? w[i] : 1.0;
     for (int q = 0; q < R; q++) dens[(size_t)q * n + i] = x[(size_t)q * n + g] * wi;
+    if (ts) stamp_end(ts + 1);
 }
 
 __global__ void k_scatter_out(const double* __restrict__ out_sorted, const int* __restrict__ perm, int n,
@@ -1792,7 +1797,8 @@ CellTiles make_level_tiles(const HostTree& t, int level, hipStream_t s) {
 }
 
 void launch_level_gemm(const CellTiles& T, int blk, const double* M, bool trans, const double* in,
-                       const double* addin, double* out, float* out32, bool add, hipStream_t s) {
+                       const double* addin, double* out, float* out32, bool add, hipStream_t s,
+                       unsigned long long* stamp) {
     if (T.n == 0) return;
     const int rb = div_up(blk, 64);
     const bool wide = (long)rb * T.n >= kGemmWideMin;
@@ -1802,10 +1808,10 @@ void launch_level_gemm(const CellTiles& T, int blk, const double* M, bool trans,
         const int* tiles = T.tiles.p + 3 * (size_t)t0;
         if (wide)
             hipLaunchKernelGGL((k_level_gemm<2, 2, 2, 2, 32>), dim3(rb, nt), dim3(256), 0, s, blk, T.cells.p, tiles, M,
-                               trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+                               trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0, stamp);
         else
             hipLaunchKernelGGL((k_level_gemm<4, 1, 1, 1, 64>), dim3(rb, nt, 4), dim3(256), 0, s, blk, T.cells.p, tiles,
-                               M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0);
+                               M, trans ? 1 : 0, in, addin, out, out32, add ? 1 : 0, stamp);
         TBEM_LAUNCH_CHECK();
     }
 }

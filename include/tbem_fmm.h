@@ -280,9 +280,9 @@ int tbem_fmm_octree(tbem_fmm_t h, int which, double* cells, long* indices,
 /* Per-stage device times of the last apply, milliseconds, in the order
  * gather, p2m, m2m, m2l, l2l, p2p(+m2p+l2p), scatter (7 doubles). From 48 rows
  * (R*n_e) on the stages lie between recorded events; below, between device clock
- * readings of their own kernels: a stage lasts from the start of its first workgroup
- * to that of the next stage's (l2l and scatter: to the end of their last workgroup by
- * index), and one without a kernel takes no time. With the point pairs on the second
+ * readings of their own kernels: a stage lasts from the end of the one before to the end
+ * of its own last workgroup (by index), the leaf stage from its first workgroup's start to
+ * scatter's, and a stage without a kernel takes no time. With the point pairs on the second
  * stream (tbem_fmm_set_overlap) the sixth value is their time and that of the surface
  * sources together. */
 int tbem_fmm_stage_times(tbem_fmm_t h, double* ms7);
