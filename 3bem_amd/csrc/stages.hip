@@ -50,7 +50,10 @@ struct Tile {
     double x[NB], y[NB], z[NB];
     VT nx[NRM ? NB : 1], ny[NRM ? NB : 1], nz[NRM ? NB : 1];
     VT d[R][NB];
-    VT sv[SV ? NB : 1];
+};
+template <class VT, int R, bool NRM, int NB>
+struct Tile<VT, R, NRM, NB, true> : Tile<VT, R, NRM, NB, false> {
+    VT sv[NB];
 };
 
 // LDS of a stage kernel: the point tile (values in PT), the surface tile (FP64),
@@ -227,7 +230,7 @@ __device__ inline void stream_ranges(Tile<VT, R, NRM, NB>& tl, int e0, int e1,
     }
 }
 
-// Streams the points [v0, v1) of the list's virtual concatenation of ranges (range e
+// Streams the points [v0, v1), v0 < v1, of the list's virtual concatenation of ranges (range e
 // starts at offset rpre[e] of it; ranges e0..e1 hold them, v0 lying in e0) through the
 // tile in full NB-point tiles, so a tile may span range boundaries and only the last
 // one is partial. Up to NB
@@ -253,7 +256,6 @@ __device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB, SV>& tl, int* s
                                             const int* __restrict__ rclose = nullptr, int* tile_close = nullptr,
                                             int* s_wflag = nullptr) {
     const int tid = threadIdx.x;
-    if (v0 >= v1) return;
     const int total = v1;
     SrcReg<R, NRM> r;
     int mclose = 0;  // the lane's next point comes from a close range
@@ -318,8 +320,9 @@ __device__ inline void stream_ranges_packed(Tile<VT, R, NRM, NB, SV>& tl, int* s
     }
 }
 
-// Streams the equivalent/check surfaces of cells cell[e0..e1) (n_e points each).
-template <int R, bool NRM, int NB, class F>
+// Streams the equivalent/check surfaces of cells cell[e0..e1) (n_e points each). WIDE: the
+// workgroup may have more threads than the tile points.
+template <bool WIDE = false, int R, bool NRM, int NB, class F>
 __device__ inline void stream_surfaces(Tile<double, R, NRM, NB>& tl, int e0, int e1,
                                        const int* __restrict__ cell, const TreeView& st,
                                        const double* __restrict__ surf, const double* __restrict__ unit,
@@ -331,7 +334,7 @@ __device__ inline void stream_surfaces(Tile<double, R, NRM, NB>& tl, int e0, int
     int base = 0;
     auto fetch = [&](int b) {
         const int v = b + tid;
-        if (tid < NB && v < total) {
+        if ((!WIDE || tid < NB) && v < total) {
             const int k = v / n_e;
             load_surf(r, cell[e0 + k], v - k * n_e, st, surf, unit, coeff, n_e, blk);
         }
@@ -551,7 +554,7 @@ __global__ __launch_bounds__(kSurfOneMax) void k_surf_one(SurfStage a, KC<double
         for (; j < cnt; j += S) pair<KID, ADJ, false, CUT, true>(sm.st, j, p[0], p[1], p[2], tn, acc, kc);
     };
     if (SRC_SURF)
-        stream_surfaces(sm.st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
+        stream_surfaces<true>(sm.st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
     else
         stream_ranges(sm.st, e0, e1, a.rbeg, a.rcnt, a.sp, a.dens, a.n_src_pts, compute);
     __syncthreads();
@@ -655,7 +658,7 @@ __global__ __launch_bounds__(256, 4) void k_surf_split(SurfStage a, KC<double> k
             buf ^= 1;
         }
     };
-    stream_surfaces(st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
+    stream_surfaces<true>(st, e0, e1, a.cell, a.st, a.s_surf, a.unit, a.s_coeff, n_e, a.blk, compute);
     if (w < R && mine) {
         double s = 0;
         s += acc;
@@ -760,9 +763,10 @@ __global__ __launch_bounds__((leaf_block<KID, T>()), (leaf_waves<KID, T>())) voi
                 }
             }
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, v0, v1, a.rp_beg, a.rp_pre, a.ps, a.pdens,
-                             a.n_ps, points, CLOSE ? a.rp_close : nullptr, CLOSE ? &tclose : nullptr,
-                             sm.wflag);                                                              // (a)
+        if (v0 < v1)
+            stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, v0, v1, a.rp_beg, a.rp_pre, a.ps, a.pdens,
+                                 a.n_ps, points, CLOSE ? a.rp_close : nullptr, CLOSE ? &tclose : nullptr,
+                                 sm.wflag);                                                          // (a)
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk,
                         surfaces);                                                                // (b)
         if (self)
@@ -1265,7 +1269,6 @@ __global__ __launch_bounds__(kGradBlock) void k_leaf_grad(LeafStage a, KC<D3> kc
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
     const int pe0 = a.rp_ptr ? uni(a.rp_ptr[pos]) : 0, pe1 = a.rp_ptr ? uni(a.rp_ptr[pos + 1]) : 0;
     const int se0 = a.sl_ptr ? uni(a.sl_ptr[pos]) : 0, se1 = a.sl_ptr ? uni(a.sl_ptr[pos + 1]) : 0;
-    const int np = pe0 < pe1 ? uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]) : 0;
     const int tid = threadIdx.x;
     for (int t0 = 0; t0 < m; t0 += NB) {
         const int nt = min(NB, m - t0);
@@ -1296,8 +1299,9 @@ __global__ __launch_bounds__(kGradBlock) void k_leaf_grad(LeafStage a, KC<D3> kc
             if (!active) return;
             for (int j = slice; j < cnt; j += S) pair_d(sm.st, j);
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, np, a.rp_beg, a.rp_pre, a.ps, a.pdens,
-                             a.n_ps, points);
+        if (pe0 < pe1)
+            stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]),
+                                 a.rp_beg, a.rp_pre, a.ps, a.pdens, a.n_ps, points);
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk, surfaces);
         if (a.self_coeff)
             stream_surfaces(sm.st, 0, 1, &leaf, a.tt, a.self_surf, a.unit, a.self_coeff, a.n_e, a.blk, surfaces);
@@ -1356,7 +1360,6 @@ __global__ __launch_bounds__(kGradBlock, (grad_waves<KID, T>())) void k_leaf_gra
     const int leaf = uni(a.leaves[pos]);
     const int b = uni(a.tt.begin[leaf]), m = uni(a.tt.count[leaf]);
     const int pe0 = a.rp_ptr ? uni(a.rp_ptr[pos]) : 0, pe1 = a.rp_ptr ? uni(a.rp_ptr[pos + 1]) : 0;
-    const int np = pe0 < pe1 ? uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]) : 0;
     const int se0 = a.sl_ptr ? uni(a.sl_ptr[pos]) : 0, se1 = a.sl_ptr ? uni(a.sl_ptr[pos + 1]) : 0;
     const int tid = threadIdx.x;
     for (int t0 = 0; t0 < m; t0 += 2 * NB) {
@@ -1423,8 +1426,12 @@ __global__ __launch_bounds__(kGradBlock, (grad_waves<KID, T>())) void k_leaf_gra
                 grad_pair<KID, double>(dxb, dyb, dzb, dxb * dxb + dyb * dyb + dzb * dzb, sn, v, gB, GB, kc64);
             }
         };
-        stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, np, a.rp_beg, a.rp_pre, a.ps, a.pdens,
-                             a.n_ps, points, a.rp_close, a.rp_close ? &tclose : nullptr, sm.wflag);
+        // (the count at the call, and no test of it inside: held over the tiles, or tested again, it
+        // pressed the compiler into taking the two targets' roots one after the other, up to 13%)
+        if (pe0 < pe1)
+            stream_ranges_packed(sm.pt, sm.rpre, sm.rbeg, pe0, pe1, 0, uni(a.rp_pre[pe1 - 1] + a.rp_cnt[pe1 - 1]),
+                                 a.rp_beg, a.rp_pre, a.ps, a.pdens, a.n_ps, points, a.rp_close,
+                                 a.rp_close ? &tclose : nullptr, sm.wflag);
         stream_surfaces(sm.st, se0, se1, a.sl_cell, a.slt, a.sl_surf, a.unit, a.sl_coeff, a.n_e, a.blk, surfaces);
         if (a.self_coeff)
             stream_surfaces(sm.st, 0, 1, &leaf, a.tt, a.self_surf, a.unit, a.self_coeff, a.n_e, a.blk, surfaces);
