@@ -115,32 +115,38 @@ static HostList all_pairs(const HostTree& tgt, int n_src) {
 // parts are whole FP32 tiles (kLeafBlock sources, a multiple of every instance's), so that
 // the tiles' partial sums stay what they are without parts. Whole chunks have no items.
 //
-// How many parts: the launch's time in units of one source on a full chunk is about
-//   rounds * (a part's sources + F) + (with parts) 100 + 3 per part,
-// rounds = workgroups / kUnits, rounded up; F, a workgroup's fixed costs (targets, first
-// tile, slice sums), 64 for the 512-thread instances and 8 for the 256-thread ones; the rest
-// the launch that adds the parts. Chunks of fewer targets count their sources in proportion.
-// Fitted to 140 sizes from 100 x 128 to 50,000 x 70,000 points and five kernels, each with 1
-// to 128 parts; whole chunks -> the model's parts, per apply: traction, 3,000 sources on 2,003
-// targets 159 -> 27 us; hypersingular, 20,011 points 1660 -> 869 us (16.4 -> 31.3 TFLOP/s);
-// double layer, 1,000 sources on 40,000 targets 72 -> 56 us; and where they do not pay,
-// 300 sources on 60,000 targets 37 us whole, 56 in the five parts that fill more workgroups.
+// How many parts: the one with the least modelled time of the launch in microseconds,
+//   (1 + a (rounds - 1)) (a part's sources * c + F) + (with parts) 2.4 + 0.04 per part,
+// rounds = workgroups / kUnits, rounded up; c the kernel's time per source and round, F a
+// workgroup's fixed costs (targets, first tile, slice sums) and a what a further round takes
+// of the first, by the instance's width; the last the launch that adds the parts. Chunks of
+// fewer targets count their sources in proportion. Fitted to 140 sizes from 100 x 128 to
+// 50,000 x 70,000 points and five kernels, each with 1 to 128 parts (12.5 us more for the rest
+// of an apply): the parts it takes cost 1.1% more than the best ones on average and 8% at most.
+// Whole chunks -> its parts, per apply: traction, 3,000 sources on 2,003 targets 159 -> 27 us;
+// hypersingular, 20,011 points 1660 -> 869 us (16.4 -> 31.3 TFLOP/s); double layer, 1,000
+// sources on 40,000 targets 72 -> 56 us; and where they do not pay, 300 sources on 60,000
+// targets 37 us whole, 56 in the five parts that fill more workgroups.
 constexpr int kUnits = 256, kMaxParts = 1024;
 
 static int count_parts(int kid, bool mixed, int nc, int n_tgt, int n_src, int unit, size_t max_parts) {
     if (kid == K_LH) return 1;  // no work per pair
-    const double F = leaf_stage_tile(kid, mixed) > 256 ? 64 : 8;
-    const double per_source = std::min(n_tgt, kTargetChunk) / (double)kTargetChunk;
+    // microseconds per source, by kernel id (the identities: from whole chunks alone)
+    static const double kSource[9] = {0.0274, 0.0294, 0, 0.0354, 0.0491, 0.0491, 0.0871, 0.013, 0.017};
+    const bool wide = leaf_stage_tile(kid, mixed) > 256;
+    const double F = wide ? 1.68 : 0.65, a = wide ? 0.91 : 0.75;
+    const double c = kSource[kid] * std::min(n_tgt, kTargetChunk) / kTargetChunk;
     int best = 1;
-    double best_cost = 0;
+    double best_time = 0;
     for (int np = 1; np <= std::min<size_t>(kMaxParts, std::max<size_t>(1, max_parts)); np++) {
         const int per = div_up(div_up(n_src, np), unit) * unit;
         if (np > 1 && per * (double)(np - 1) >= n_src) continue;  // fewer parts hold them all
         const double rounds = std::ceil((double)nc * np / kUnits);
-        const double cost = rounds * (std::min(per, n_src) * per_source + F) + (np > 1 ? 100 + 3 * np : 0);
-        if (np == 1 || cost < best_cost) {
+        const double time =
+            (1 + a * (rounds - 1)) * (std::min(per, n_src) * c + F) + (np > 1 ? 2.4 + 0.04 * np : 0);
+        if (np == 1 || time < best_time) {
             best = np;
-            best_cost = cost;
+            best_time = time;
         }
     }
     return best;

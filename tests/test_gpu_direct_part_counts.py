@@ -10,8 +10,8 @@ from conftest import rel_err
 pytestmark = pytest.mark.gpu
 
 
-# targets x sources: whole (10 x 1000, 130 x 40, 20000 x 300), 2 to 4 parts (16384 x 300,
-# 40000 x 1000), about 20 (1 x 60000, 128 x 2000), 85 (384 x 20000)
+# targets x sources: mostly whole (10 x 1000, 130 x 40, 20000 x 300), a few parts (16384 x 300,
+# 40000 x 1000), tens of them (1 x 60000, 128 x 2000, 384 x 20000)
 @pytest.mark.parametrize("n_obs,n_src", [(10, 1000), (130, 40), (20000, 300), (16384, 300), (40000, 1000), (1, 60000),
                                          (128, 2000), (384, 20000)])
 @pytest.mark.parametrize("kid", [1, 3, 6])
