@@ -979,6 +979,19 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_wave(LeafStage a, KC<T> kc,
     }
 }
 
+// The sum of a target's n chunk sums, step apart, in chunk order, eight loads in flight.
+__device__ __forceinline__ double add_parts(const double* __restrict__ p, int n, size_t step) {
+    double s = 0;
+    int c = 0;
+    for (; c + 8 <= n; c += 8) {
+        double v[8];
+        for (int u = 0; u < 8; u++) v[u] = p[(c + u) * step];
+        for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; c < n; c++) s += p[c * step];
+    return s;
+}
+
 // The leaves that ran in chunks: one workgroup per leaf and output component (grid y),
 // the chunks' partial sums added in chunk order, eight loads in flight.
 __global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, double scale) {
@@ -989,14 +1002,7 @@ __global__ __launch_bounds__(kPartsBlock) void k_leaf_parts(LeafStage a, double 
     for (int t = threadIdx.x; t < m; t += kPartsBlock) {
         const int i = b + t;
         const double* p = a.part_buf + (size_t)lp.part + (size_t)q * m + t;
-        double s = 0;
-        int c = 0;
-        for (; c + 8 <= lp.n; c += 8) {
-            double v[8];
-            for (int u = 0; u < 8; u++) v[u] = p[(c + u) * step];
-            for (int u = 0; u < 8; u++) s += v[u];
-        }
-        for (; c < lp.n; c++) s += p[c * step];
+        const double s = add_parts(p, lp.n, step);
         const double wgt = a.t_weight ? a.t_weight[i] : 1.0;
         double* o = a.out_sorted + (size_t)q * a.n_tgt + i;
         *o = a.accumulate ? *o + wgt * (s * scale) : wgt * (s * scale);
@@ -1617,19 +1623,18 @@ __global__ __launch_bounds__(kWaveBlock) void k_leaf_grad2_wave(LeafStage a, KC<
     }
 }
 
-// The gradient's chunked leaves: grad_out[3 i + mm] = the chunks' sums, in chunk order.
+// The gradient's chunked leaves, one workgroup per leaf and component (grid y): grad_out[3 i +
+// mm] = the chunks' sums. One load after the other, three components in turn, took most of the
+// gradient where few targets have many sources in the finer chunks (94,481 sources on 767
+// targets, Kelvin U, order 5: 459 us a gradient with the coarse chunks, 720 with the fine).
 __global__ __launch_bounds__(kWaveLeafMax) void k_leaf_grad_parts(LeafStage a, double scale) {
     const WaveLeafParts lp = a.parts[blockIdx.x];
-    const int leaf = a.leaves[lp.pos];
+    const int leaf = a.leaves[lp.pos], mm = blockIdx.y;
     const int b = a.tt.begin[leaf], m = a.tt.count[leaf];
     const int t = threadIdx.x;
     if (t >= m) return;
-    for (int mm = 0; mm < 3; mm++) {
-        const double* p = a.part_buf + (size_t)lp.part + mm * m + t;
-        double s = 0;
-        for (int c = 0; c < lp.n; c++) s += p[(size_t)c * kPartRows * m];
-        a.grad_out[3 * (size_t)(b + t) + mm] = s * scale;
-    }
+    const double s = add_parts(a.part_buf + (size_t)lp.part + mm * m + t, lp.n, (size_t)kPartRows * m);
+    a.grad_out[3 * (size_t)(b + t) + mm] = s * scale;
 }
 
 // ------------------------------------------------------------------------ helpers
@@ -2073,7 +2078,8 @@ static void grad_launch(bool fp32_points, const LeafStage& a, const KConst& c, h
                                        scale);
                 TBEM_LAUNCH_CHECK();
                 if (a.n_wave_parts > 0) {
-                    hipLaunchKernelGGL(k_leaf_grad_parts, dim3(a.n_wave_parts), dim3(kWaveLeafMax), 0, s, a, scale);
+                    hipLaunchKernelGGL(k_leaf_grad_parts, dim3(a.n_wave_parts, 3), dim3(kWaveLeafMax), 0, s, a,
+                                       scale);
                     TBEM_LAUNCH_CHECK();
                 }
             }
