@@ -177,8 +177,9 @@ class FMMOperator:
     serves, where both share the union box), "own" or "common" to force either.
     translations: the translations between surfaces (M2M, L2L, and the FP64 path's
     M2L), "auto" (one FP64 operator per translation class on the FP64 MFMA units
-    where the classes exist, else as "surfaces") or "surfaces" (the kernel between
-    the two surfaces of every pair, as the reference).
+    where the classes exist, and below 48 rows where they pay and fit the free memory,
+    else as "surfaces") or "surfaces" (the kernel between the two surfaces of every
+    pair, as the reference).
     m2l_output_budget: bytes the class M2L's per-pair output may take (None: 6 GiB);
     beyond it the pairs run in slices.
     point_pairs: "auto" (the forward evaluates each pair of points in neighbouring
@@ -379,7 +380,8 @@ class FMMOperator:
 
     def set_overlap(self, on=True):
         """Run the forward's point-to-point pairs on a second stream beside the far
-        field (the default), or as one fused leaf launch after it (each kernel then
+        field (the default where that is a chain of launches worth filling:
+        tbem_fmm_set_overlap), or as one fused leaf launch after it (each kernel then
         has the device to itself, for timing). Same results to rounding."""
         _lib.check(self._lib.tbem_fmm_set_overlap(self._h, 1 if on else 0))
 

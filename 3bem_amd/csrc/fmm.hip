@@ -37,16 +37,16 @@ void set_last_error(const std::string& m) { g_last_error = m; }
 // pairs are processed in slices that fit.
 constexpr size_t kM2lOutputBudget = size_t(6) << 30;
 
-// The point-target stage's leaf positions split between the one-wave kernel (leaves of
-// at most kWaveLeafMax points: one work item each, or chunks of a large one) and the
-// one-workgroup kernel (the rest, whole or in chunks), both ordered by decreasing work
-// (split_leaves).
 // Below this many operator rows the surface stages apply the C2E product themselves
 // (SurfStage.c2e) instead of a level GEMM of its own per stage and level; it needs a row per
 // thread of kSurfBlock. From here on the MFMA products of the classes and levels take over.
 constexpr int kFuseC2eMax = 48;
 static_assert(kFuseC2eMax <= kSurfBlock, "one row per thread");
 
+// The point-target stage's leaf positions split between the one-wave kernel (leaves of
+// at most kWaveLeafMax points: one work item each, or chunks of a large one) and the
+// one-workgroup kernel (the rest, whole or in chunks), both ordered by decreasing work
+// (split_leaves).
 struct LeafSplit {
     DevBuf<WaveItem> items, block_items;
     DevBuf<WaveLeafParts> parts;  // the wave items' cut leaves, then the block items'
@@ -758,29 +758,6 @@ static void close_flags(DevList& l, const int* leaves, const DevTree& tt, const 
                               kCloseMargin, l.rclose.p, s);
 }
 
-// Splits the positions of a point-target list (items = leaves of tree tt; point
-// ranges pts, surface cells surf, and each leaf's own surface): leaves of at most
-// kWaveLeafMax points go to the one-wave kernel when they have at most kWavePairsMax
-// pairs (points x sources), or when they have at most kWaveChunkLeaf points, then cut into
-// chunks of about equal sources (points cut anywhere, surface cells whole, the own surface
-// with the last chunk), whose sums k_leaf_parts adds in chunk order; the rest go to the
-// one-workgroup kernel. Both lists are laid out by xcd_layout: per XCD a run of
-// neighbouring leaves, the most work first.
-// (kWaveChunkLeaf: a wave holds ceil(m/2) targets per source slice, so above 64
-// points one slice is left and down to half of its lanes idle, where the 512-thread
-// kernel keeps 96% busy.)
-// A small problem has fewer such items than the chip has room for, and its longest one
-// sets the launch's length. The items of both kernels are therefore also cut where they
-// exceed the kernel's total pairs divided by kWaveFill (kBlockFill) items, about four rounds
-// of what the chip holds at once, but not below kWaveCapMin (kBlockCapMin) pairs, where an
-// item's fixed costs would take over. These cuts fall on whole LDS tiles (wave: kWaveTile sources;
-// block_tile), so that the FP32 partial sum of every tile is the same as uncut.
-// Measured (whole passes): mesh of 9,102 points, hypersingular, mixed 1316 -> 823 us (its
-// block leaves 489 -> 57 us); sphere of 15,360 points, Laplace 310 -> 213 us (leaf waves
-// 67 -> 22 us, symmetric pairs 95 -> 38); 300,007 points, order 50, mixed, forward and
-// backward 6.10 -> 4.30 ms (one round of the whole problem's pairs); then 3.84 -> 3.62 ms,
-// and the double layer, 61,440 points, order 35, 1049 -> 937 us, with four rounds of each
-// kernel's own pairs.
 // Lays out work items (work, item), given in tree order, for a launch whose workgroup
 // b runs on XCD b % 8 (the hardware deals workgroups to the XCDs in turn), g items per
 // workgroup. The items are cut into 8 runs of about equal work, one per XCD, so that
@@ -816,6 +793,29 @@ static std::vector<I> xcd_layout(const std::vector<std::pair<long, I>>& items, i
     return out;
 }
 
+// Splits the positions of a point-target list (items = leaves of tree tt; point
+// ranges pts, surface cells surf, and each leaf's own surface): leaves of at most
+// kWaveLeafMax points go to the one-wave kernel when they have at most kWavePairsMax
+// pairs (points x sources), or when they have at most kWaveChunkLeaf points, then cut into
+// chunks of about equal sources (points cut anywhere, surface cells whole, the own surface
+// with the last chunk), whose sums k_leaf_parts adds in chunk order; the rest go to the
+// one-workgroup kernel. Both lists are laid out by xcd_layout: per XCD a run of
+// neighbouring leaves, the most work first.
+// (kWaveChunkLeaf: a wave holds ceil(m/2) targets per source slice, so above 64
+// points one slice is left and down to half of its lanes idle, where the 512-thread
+// kernel keeps 96% busy.)
+// A small problem has fewer such items than the chip has room for, and its longest one
+// sets the launch's length. The items of both kernels are therefore also cut where they
+// exceed the kernel's total pairs divided by kWaveFill (kBlockFill) items, about four rounds
+// of what the chip holds at once, but not below kWaveCapMin (kBlockCapMin) pairs, where an
+// item's fixed costs would take over. These cuts fall on whole LDS tiles (wave: kWaveTile sources;
+// block_tile), so that the FP32 partial sum of every tile is the same as uncut.
+// Measured (whole passes): mesh of 9,102 points, hypersingular, mixed 1316 -> 823 us (its
+// block leaves 489 -> 57 us); sphere of 15,360 points, Laplace 310 -> 213 us (leaf waves
+// 67 -> 22 us, symmetric pairs 95 -> 38); 300,007 points, order 50, mixed, forward and
+// backward 6.10 -> 4.30 ms (one round of the whole problem's pairs); then 3.84 -> 3.62 ms,
+// and the double layer, 61,440 points, order 35, 1049 -> 937 us, with four rounds of each
+// kernel's own pairs.
 constexpr int kWaveChunkLeaf = 64;
 constexpr long kWaveFill = 16384, kWaveCapMin = 4096;
 constexpr long kBlockFill = 8192, kBlockCapMin = 16384;
@@ -951,11 +951,12 @@ static void build_sym(FmmPlan& P, const HostTree& T, const std::vector<std::arra
     const int nl = (int)leaves.size();
     std::vector<int> pos_of(T.n_cells, -1);
     for (int k = 0; k < nl; k++) pos_of[leaves[k]] = k;
-    // Below 64 points a leaf's pairs pay for the Laplace single layer (4M points, cube +
-    // clusters, leaf 100: FP64 matvec 71.1 -> 66.7 ms with leaves from 16 points, mixed
-    // 47.4 -> 45.6) but not for Kelvin U (1M points, fault + surface, leaf 64: FP64
-    // 2.90 -> 3.15 ms, mixed 2.30 -> 2.75; from 32 points 3.09 and 2.51), whose one-wave
-    // ordered kernel serves small leaves better.
+    // Below 64 points a leaf's pairs pay for the Laplace single layer (1M points, cube +
+    // clusters, order 35, leaf 100: 14.9 ms from 16 points, 15.9 from 32, 16.4 from 64) but not
+    // for Kelvin U, whose one-wave ordered kernel serves small leaves as well or better (1M
+    // points, fault + surface, order 6, leaf 64, from 16, 32, 48, 64 points and none: FP64 2.64,
+    // 2.74, 2.65, 2.63, 2.61 ms, mixed 2.26, 2.23, 2.09, 2.08, 2.04; 300,007 points, order 50,
+    // leaf 128, from 32, 48, 64, 80: 2.47, 2.48, 2.49, 2.52).
     const int lo = P.kid == TBEM_K_LAPLACE_SINGLE ? kSymLeafMin : 64;
     auto fits = [&](int k) {
         const int m = T.count[leaves[k]];

@@ -626,8 +626,11 @@ bool m2l_fp64_size_ok(int n) { return size_ok(n, true); }
 // 0.043 F) ps, F flops per evaluation (Laplace single layer, order 35: 1450 ps; elastic
 // displacement, order 6: 85; hypersingular, order 10: 460), the class operators, bound by
 // their per-pair output's traffic, about 6.5 ps per output row (order 35, 48 rows: 295 ps;
-// 32 rows: 205). A quarter is left for the second launch and the classes' plan, and fewer
-// than kMinClassPairs pairs gain too little to build them for. From kMinBlk rows on the
+// 32 rows: 205). A quarter is left for the second launch and the classes' plan, which takes
+// 1.4 ms (124,000 pairs) to 4 ms (2.5M) more and is even after 2 to 20 passes; fewer than
+// kMinClassPairs pairs gain too little to build them for. Whole passes at the low end, surfaces
+// -> classes: 59,000 pairs, order 35 620 -> 210 us; 132,000, order 20, double layer 303 -> 215;
+// 124,000, hypersingular, order 10 488 -> 185 (with the leaf stage's cuts). From kMinBlk rows on the
 // classes serve every size. M2L stage, surfaces -> classes: 60k points in a cube, order 20
 // 1032 -> 452 us, order 35 3214 -> 654, order 47 6141 -> 688; 500k in clusters, order 35
 // 5964 -> 1671; hypersingular, 100k points, order 10 506 -> 377 (order 6 182 -> 245, left).
@@ -984,7 +987,8 @@ static void mfma32_slice(const M2lMfma& M, int q, const int* pair_src, const flo
 // spreads each unit's row tiles over up to kUnitsFill / units workgroups, each staging the
 // unit's columns again: the rows' products are what a lone workgroup spends its time on.
 // M2M and L2L per launch, blk 453: 70 -> 23 us; blk 150: 38 -> 15 us (300,007 points), 25 ->
-// 12 us (9,102 points).
+// 12 us (9,102 points). Whole passes with 1 (one workgroup a unit), 256, 1024 and 4096: 300,007
+// points, order 50 2577, 2500, 2501, 2507 us; traction, order 150 1901, 1713, 1748, 1737.
 constexpr int kUnitsFill = 1024;
 
 // Y (slice q) = K_c * x[src(p)] (transpose: K_c^T * x[tgt(p)]), FP64 MFMA; with dst, row

@@ -20,8 +20,9 @@ constexpr int kLeafBlock = 512;  // point-target stage (P2P + M2P + L2P)
 //  * FP64 traction kernels: 512 threads at four waves (125 VGPRs, from 148-152; two
 //    workgroups per CU): adjoint-traction forward 75 -> 65 ms, traction adjoint 84
 //    -> 74 ms;
-//  * the rest (<= 128 VGPRs already): 512 threads, no cap; a cap at four waves made
-//    the FP64 elastic-U leaf 16% slower (101 VGPRs, less latency hiding);
+//  * Kelvin U: 512 threads at four waves too, since the work items took it past 128
+//    VGPRs (142 in FP32, 144 in FP64), 1.25 times slower;
+//  * the rest (<= 128 VGPRs already): 512 threads, no cap;
 //  * Laplace single layer, whose pair is cheap, at 256 threads (4M points, leaf 100,
 //    the larger leaves on this kernel: FP64 leaf stage 38.2 -> 36.9 ms, mixed 27.9
 //    -> 26.5 ms).
@@ -168,7 +169,8 @@ struct LeafStage {
     // The leaf positions a gradient launch serves (null: 0 .. n_leaves-1, one workgroup each).
     const int* order;
     int n_order;
-    // Optional split of the positions (launch_leaf_stage; split = 0: none): wave_items, leaves of at most
+    // Optional split of the positions (launch_leaf_stage; split = 0: none, every leaf whole on
+    // one workgroup, as the direct operator's chunks without parts): wave_items, leaves of at most
     // kWaveLeafMax points, whole or in chunks, one wave each, the most work first;
     // block_items, the rest, whole or in chunks, one workgroup each (block_pos: the same
     // leaves whole, for the gradient). parts: the leaves cut into chunks, the n_wave_parts

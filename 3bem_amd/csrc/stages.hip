@@ -1651,7 +1651,9 @@ __global__ __launch_bounds__(kWaveLeafMax) void k_leaf_grad_parts(LeafStage a, d
 // kGemmWideMin workgroups; else 64 x 16, one tile per wave, four times the workgroups.
 // Measured against FP64 FMAs from 4 x 4 register tiles, per launch: blk 453 (traction,
 // order 150, at most 1,024 cells) 58 -> 22 us; blk 150 (mesh of 9,102 points) 22 -> 9.5;
-// 2M points, order 100 (blk 297): 16 launches 2311 -> 1500 us beside the point pairs.
+// 2M points, order 100 (blk 297): 16 launches 2311 -> 1500 us beside the point pairs. Where the
+// line lies hardly matters: whole passes with it at 64, 128, 512 and 2048 workgroups, 300,007
+// points, order 50 2478, 2456, 2489, 2507 us; 2M 22.5, 22.4, 22.5, 22.6 ms.
 constexpr int kGemmWideMin = 512, kGemmTiles = 65536;
 typedef double gemm_f64x4 __attribute__((ext_vector_type(4)));
 
